@@ -96,7 +96,6 @@ template <> struct Tour<float2> { static constexpr int RL = 256, AR = 4; };
 template <typename T> struct TNode {
     int id[TW];                 // the nominees' global rows, in their pivot order
     int count, pad[63];
-    T v[TW * TW];               // their original panel rows, column-major: v[c * TW + i]
 };
 
 __host__ __device__ inline long tour_leaves(long m, int RL) { return (m + RL - 1) / RL; }
