@@ -339,8 +339,8 @@ int m25x_zgemm_nk_batched(int nitems, const m25x_mv_item *items_host, const m25x
 #define M25X_K_NEAR_SCATTER 2   /* per near entry: read-modify-write of Z, its contributions read */
 #define M25X_K_TSLU 3           /* a 64-column panel's tournament: the panel read once; flops: its GEPPs */
 #define M25X_K_APPLY_MOVES 4    /* the panel's row moves: 2 x element per moved element */
-#define M25X_K_L21 5            /* L21 = A21 U11^-1: 8 m 64^2 / 2 flops */
-#define M25X_K_TRSM 6           /* U12 = L11^-1 A12: 8 n 64^2 / 2 flops */
+#define M25X_K_L21 5            /* a tournament panel's L21 = A21 U11^-1 and U12 = L11^-1 A12: 8 m 64^2 flops */
+#define M25X_K_TRSM 6           /* a partial-pivoting panel's U12 = L11^-1 A12: 8 n 128^2 / 2 flops */
 #define M25X_K_GEMM 7           /* trailing update: 8 M N K flops; bytes: C read and written, A and B read */
 #define M25X_K_TRSV 8           /* a triangular solve: its triangle of the factor and the right-hand sides */
 #define M25X_K_ZGEMM_NK 9       /* Y = Z X: 16 N^2 B of Z read */

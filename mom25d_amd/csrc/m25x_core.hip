@@ -132,7 +132,7 @@ long m25x_timing_records(int *kernel, int *dtype, float *ms, double *bytes, doub
 const char *m25x_kernel_name(int kernel)
 {
     static const char *names[] = {"k_fill_far", "k_near_moments", "k_near_scatter", "k_tslu", "k_apply_moves",
-                                  "k_l21", "k_trsm", "k_gemm", "k_trsv", "k_zgemm_nk", "m25x_cgs2", "k_panel",
+                                  "k_tri", "k_trsm", "k_gemm", "k_trsv", "k_zgemm_nk", "m25x_cgs2", "k_panel",
                                   "k_laswp"};
     if (kernel < 0 || kernel >= (int)(sizeof names / sizeof names[0])) return "";
     return names[kernel];

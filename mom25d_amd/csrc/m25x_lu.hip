@@ -13,8 +13,8 @@
 //           (Re C = [Re A, Im A] [Re B; -Im B], Im C = [Re A, Im A] [Im B; Re B]), v_mfma_f64_16x16x4 for
 //           complex128 and v_mfma_f32_16x16x4 for complex64 (FP32 accumulation)
 // Tournament pivoting (CALU), panels of TW = 64 columns: the panel's pivots by a tree of GEPPs in one launch with no
-// grid barrier (k_tslu), its row moves on every column (k_apply_moves), then L21 = A21 U11^-1 by substitution,
-// U12 = L11^-1 A12 by substitution and A22 -= L21 U12 on the matrix cores (complex64 with FP64 accumulation: one
+// grid barrier (k_tslu), its row moves on every column (k_apply_moves), then L21 = A21 U11^-1 and U12 = L11^-1 A12 by
+// substitution (k_tri) and A22 -= L21 U12 on the matrix cores (complex64 with FP64 accumulation: one
 // rounding per update).
 // The solves (getrs): one launch per triangle, one workgroup per 64-row diagonal block; each accumulates the
 // products of its rows with the earlier blocks as their values appear, then solves its own block and hands its
@@ -236,58 +236,27 @@ __global__ void k_laswp(T *A, long lda, long n, long j0, int jb, const int *ipiv
     }
 }
 
-// U12 = L11^-1 A12: rows [j0, j0 + jb), columns [c0, n); TC columns a workgroup, the block in LDS. JB: the largest
-// panel width; with JB = TW (the tournament's panels) L11 is staged in LDS too (column k of L11 as row k of Lt, so a
-// step's reads are consecutive), else read from memory at each step.
+// U12 = L11^-1 A12 of the partial-pivoting panels: rows [j0, j0 + jb), columns [c0, n); TC columns a workgroup, the block
+// in LDS, L11 read from memory at each step.
 constexpr int TC = 16;
-template <typename T, int JB>
-__device__ __forceinline__ void trsm_body(T *A, long lda, long n, long j0, int jb, long c0, long bx)
+template <typename T>
+__global__ __launch_bounds__(256) void k_trsm(T *A, long lda, long n, long j0, int jb, long c0)
 {
-    constexpr bool STAGE = JB <= TW;
-    __shared__ T X[JB][TC + 1];
-    __shared__ T Lt[STAGE ? TW : 1][TW];
-    const long cb = c0 + bx * TC;
+    __shared__ T X[NB][TC + 1];
+    const long cb = c0 + (long)blockIdx.x * TC;
     const int nc = (int)std::min((long)TC, n - cb);
     const int tid = threadIdx.x;
     const T *L = A + j0 * lda + j0;          // L11[i][k] = L[k * lda + i]
-    if constexpr (STAGE) {                   // jb <= TW: the loads of either block in flight before the stores
-        constexpr int NX = TW * TC / 256, NL = TW * TW / 256;
-        T vx[NX], vl[NL];
-#pragma unroll
-        for (int u = 0; u < NX; ++u) {
-            const int idx = tid + u * 256, c = idx / jb, r = idx % jb;
-            vx[u] = ldz(idx < jb * TC && c < nc, A + (cb + c) * lda + j0 + r);
-        }
-#pragma unroll
-        for (int u = 0; u < NL; ++u) {
-            const int idx = tid + u * 256, k = idx / jb, i = idx % jb;
-            vl[u] = ldz(idx < jb * jb, L + (long)k * lda + i);
-        }
-#pragma unroll
-        for (int u = 0; u < NX; ++u) {
-            const int idx = tid + u * 256, c = idx / jb, r = idx % jb;
-            if (idx < jb * TC && c < nc) X[r][c] = vx[u];
-        }
-#pragma unroll
-        for (int u = 0; u < NL; ++u) {
-            const int idx = tid + u * 256, k = idx / jb, i = idx % jb;
-            if (idx < jb * jb) Lt[k][i] = vl[u];
-        }
-    } else {
-        for (int idx = tid; idx < jb * TC; idx += 256) {
-            const int c = idx / jb, r = idx % jb;
-            if (c < nc) X[r][c] = A[(cb + c) * lda + j0 + r];
-        }
+    for (int idx = tid; idx < jb * TC; idx += 256) {
+        const int c = idx / jb, r = idx % jb;
+        if (c < nc) X[r][c] = A[(cb + c) * lda + j0 + r];
     }
     __syncthreads();
     for (int k = 0; k < jb - 1; ++k) {
         const int nr = jb - k - 1;
         for (int idx = tid; idx < nr * TC; idx += 256) {
             const int c = idx % TC, i = k + 1 + idx / TC;
-            T lik;
-            if constexpr (STAGE) lik = Lt[k][i];
-            else lik = L[(long)k * lda + i];
-            if (c < nc) X[i][c] = tsub(X[i][c], tmul(lik, X[k][c]));
+            if (c < nc) X[i][c] = tsub(X[i][c], tmul(L[(long)k * lda + i], X[k][c]));
         }
         __syncthreads();
     }
@@ -295,12 +264,6 @@ __device__ __forceinline__ void trsm_body(T *A, long lda, long n, long j0, int j
         const int c = idx / jb, r = idx % jb;
         if (c < nc) A[(cb + c) * lda + j0 + r] = X[r][c];
     }
-}
-
-template <typename T, int JB>
-__global__ __launch_bounds__(256) void k_trsm(T *A, long lda, long n, long j0, int jb, long c0)
-{
-    trsm_body<T, JB>(A, lda, n, j0, jb, c0, blockIdx.x);
 }
 
 // ---- C -= A B (SUB) or C = A B on the matrix cores -------------------------------------------------------
@@ -496,83 +459,89 @@ __global__ void k_perm(const int *ipiv, long n, int *perm)
 constexpr int SB = 64;
 constexpr int MAXRHS = 8;
 
-// L21 = A21 U11^-1 by substitution (x U11 = a for each row a of A21): a thread a row of [r0, r0 + m), U11 (the
-// upper part of top) in LDS; the 64 columns in two halves of 32 so a row's half stays in registers for either
-// element type.
-template <typename T>
-__device__ __forceinline__ void l21_body(T *A, long lda, long r0, long m, long j0, int jb, const T *top, long bx)
+// A tournament panel's L21 = A21 U11^-1 (x U11 = a for each row a below the panel) and U12 = L11^-1 A12 (L11 x = a for
+// each column a right of it) by substitution: 64 unknowns a vector, the triangle (from top) in LDS. Sixteen lanes (a DPP
+// row) share a vector, lane l holding its elements l, l + 16, l + 32, l + 48; step k broadcasts the finished element k
+// among them (row_newbcast) and every lane subtracts its multiple from the later elements. What bounds it is how many
+// lanes work and the steps' latency: with a row a thread L21 kept 120 of the chip's 1024 SIMDs busy at N = 7799, and U12
+// passed 63 barriers. TRI_V vectors a lane, 32 a workgroup of 256 threads, cover the chip and give a step independent
+// work. Measured, both blocks of a panel at N = 7799: 78 us (complex64), 99 us (complex128) before; 11.8 and 15.4 us so.
+constexpr int TRI_V = 2, TRI_N = 16 * TRI_V;          // vectors a workgroup
+template <int N> __device__ __forceinline__ float row_bcast(float v)
 {
-    __shared__ T Us[TW][TW + 1];
-    __shared__ T rd[TW];
-    const int tid = threadIdx.x;
-    {
-        T v[TW * TW / 256];                     // every load in flight before the first store
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xF, 0xF, true));
+}
+template <int N> __device__ __forceinline__ double row_bcast(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b, 0x150 + N, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + N, 0xF, 0xF, true);
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// UPPER: rows [r0 + 32 bx, ...) of L21 (m rows from r0 = j0 + TW); else columns of U12 (the same m from r0)
+template <typename T, bool UPPER>
+__device__ __forceinline__ void tri_vectors(T *A, long lda, long j0, long m, const T *top, long bx, T (*M)[TW + 1], T *rd)
+{
+    const int tid = threadIdx.x, l16 = tid & 15;
+    const long r0 = j0 + TW, v0 = bx * TRI_N + (tid >> 6) * (4 * TRI_V) + ((tid >> 4) & 3);
+    const long es = UPPER ? lda : 1, vs = UPPER ? 1 : lda;         // steps between elements and between vectors
+    T *base = A + (UPPER ? j0 * lda + r0 : r0 * lda + j0);
+    T v[TW * TW / 256];                               // every load in flight before the first store
 #pragma unroll
-        for (int u = 0; u < TW * TW / 256; ++u) v[u] = top[tid + u * 256];
+    for (int u = 0; u < TW * TW / 256; ++u) v[u] = top[tid + u * 256];
+    T a[TRI_V][4];
 #pragma unroll
-        for (int u = 0; u < TW * TW / 256; ++u) {
-            const int e = tid + u * 256, c = e / TW, i = e % TW;
-            Us[i][c] = v[u];
-        }
+    for (int q = 0; q < TRI_V; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[q][i] = base[std::min(v0 + 4 * q, m - 1) * vs + (l16 + 16 * i) * es];
+    const T zero = CX<T>::make(0, 0);
+    if (UPPER && tid < TW) rd[tid] = trecip(top[tid * (TW + 1)]);
+#pragma unroll
+    for (int u = 0; u < TW * TW / 256; ++u) {         // top: column e / 64, row e % 64; M[k][c]: element c's multiple of
+        const int e = tid + u * 256, c = e / TW, i = e % TW;      // element k, zero for c <= k
+        if (UPPER) M[i][c] = csel(i < c, v[u], zero);
+        else M[c][i] = csel(i > c, v[u], zero);
     }
     __syncthreads();
-    if (tid < TW) rd[tid] = tid < jb ? trecip(Us[tid][tid]) : CX<T>::make(1, 0);
-    __syncthreads();
-    const long r = r0 + bx * 256 + tid;
-    if (r >= r0 + m) return;
-    T *row = A + j0 * lda + r;                  // element (r, j0 + c) at row[c * lda]
-    auto half = [&](auto hc) __attribute__((always_inline)) {
-        constexpr int h = decltype(hc)::value;
-        RowH<T> x;
-        auto ld = [&](auto jc) __attribute__((always_inline)) {
-            constexpr int j = decltype(jc)::value;
-            x.set(j, ldz(32 * h + j < jb, row + (long)(32 * h + j) * lda));
-        };
-        Unroll<0, TH>::run(ld);
-        if (h == 1) {                           // the first half's solution, final, from the previous pass
-            for (int k0 = 0; k0 < 32 && k0 < jb; k0 += 8) {
-                T xk[8];                        // eight of its values read together
+    auto step = [&](auto kc) __attribute__((always_inline)) {
+        constexpr int k = decltype(kc)::value, ik = k / 16;
+        T x[TRI_V];
 #pragma unroll
-                for (int u = 0; u < 8; ++u) xk[u] = ldz(k0 + u < jb, row + (long)(k0 + u) * lda);
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const int k = k0 + u;
-                    if (k >= jb) break;
-                    auto up = [&](auto jc) __attribute__((always_inline)) {
-                        constexpr int j = decltype(jc)::value;
-                        x.set(j, tsub(x.get(j), tmul(xk[u], Us[k][32 + j])));
-                    };
-                    Unroll<0, TH>::run(up);
-                }
-            }
+        for (int q = 0; q < TRI_V; ++q) {
+            x[q] = CX<T>::make(row_bcast<k % 16>(a[q][ik].x), row_bcast<k % 16>(a[q][ik].y));
+            if (UPPER) x[q] = tmul(x[q], rd[k]);
         }
-        auto solve = [&](auto jc) __attribute__((always_inline)) {
-            constexpr int j = decltype(jc)::value;
-            if (32 * h + j < jb) {
-                T v = x.get(j), v1 = CX<T>::make(0, 0);      // two partial sums: half the dependent chain
-                auto sub = [&](auto kc) __attribute__((always_inline)) {
-                    constexpr int k = decltype(kc)::value;
-                    if constexpr (k % 2 == 0) v = tsub(v, tmul(x.get(k), Us[32 * h + k][32 * h + j]));
-                    else v1 = tadd(v1, tmul(x.get(k), Us[32 * h + k][32 * h + j]));
-                };
-                Unroll<0, j>::run(sub);
-                x.set(j, tmul(tsub(v, v1), rd[32 * h + j]));
-            }
-        };
-        Unroll<0, TH>::run(solve);
-        auto st = [&](auto jc) __attribute__((always_inline)) {
-            constexpr int j = decltype(jc)::value;
-            if (32 * h + j < jb) row[(long)(32 * h + j) * lda] = x.get(j);
-        };
-        Unroll<0, TH>::run(st);
+#pragma unroll
+        for (int i = ik; i < 4; ++i) {
+            const T mk = M[k][l16 + 16 * i];
+#pragma unroll
+            for (int q = 0; q < TRI_V; ++q) a[q][i] = tfms(a[q][i], x[q], mk);
+        }
     };
-    Unroll<0, 2>::run(half);
+    Unroll<0, TW - 1>::run(step);
+#pragma unroll
+    for (int q = 0; q < TRI_V; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (v0 + 4 * q < m)
+                base[(v0 + 4 * q) * vs + (l16 + 16 * i) * es] = UPPER ? tmul(a[q][i], rd[l16 + 16 * i]) : a[q][i];
+}
+
+// workgroup bx of 2 nb21: the first half L21, the other U12
+template <typename T>
+__device__ __forceinline__ void tri_body(T *A, long lda, long j0, long m, const T *top, long bx, long nb21)
+{
+    __shared__ T M[TW][TW + 1];
+    __shared__ T rd[TW];
+    if (bx < nb21) tri_vectors<T, true>(A, lda, j0, m, top, bx, M, rd);
+    else tri_vectors<T, false>(A, lda, j0, m, top, bx - nb21, M, rd);
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_l21(T *A, long lda, long r0, long m, long j0, int jb, const T *top)
+__global__ __launch_bounds__(256) void k_tri(T *A, long lda, long j0, long m, const T *top)
 {
-    l21_body<T>(A, lda, r0, m, j0, jb, top, blockIdx.x);
+    tri_body<T>(A, lda, j0, m, top, blockIdx.x, (long)gridDim.x / 2);
 }
 
 // The panel's row moves on columns [c0, c0 + nc): a column per 128 threads, every source read before any write;
@@ -1008,7 +977,7 @@ int getrf_t(T *A, long n, long lda, int *ipiv, int *info, void *work, size_t wby
         if (c0 < n) {
             {
                 TimedLaunch tl(s, M25X_K_TRSM, dt, 2.0 * es * (n - c0) * jb, 4.0 * (n - c0) * jb * jb);
-                hipLaunchKernelGGL((k_trsm<T, NB>), dim3(blocks(n - c0, TC)), dim3(256), 0, s, A, lda, n, j0, jb, c0);
+                hipLaunchKernelGGL(k_trsm<T>, dim3(blocks(n - c0, TC)), dim3(256), 0, s, A, lda, n, j0, jb, c0);
             }
             if (int rc = check_launch("getrf/trsm")) return rc;
             const long M = n - c0;
@@ -1060,6 +1029,13 @@ template <typename T> size_t tour_work_bytes(long n)
     return nn * sizeof(TNode<T>) + (size_t)TW * TW * sizeof(T) + sizeof(int) * ((size_t)nn + 4 * TW + 64);
 }
 
+// L21 and U12 of a panel of TW columns, m rows and columns beyond it: one launch
+template <typename T> void launch_tri(hipStream_t s, T *A, long lda, long j0, long m, const T *top)
+{
+    TimedLaunch tl(s, M25X_K_L21, dtype_of<T>(), 4.0 * sizeof(T) * m * TW, 8.0 * m * TW * TW);
+    hipLaunchKernelGGL(k_tri<T>, dim3(2 * blocks(m, TRI_N)), dim3(256), 0, s, A, lda, j0, m, top);
+}
+
 // The tournament LU with one panel of look-ahead (see LookAhead): the same kernels and arithmetic as the plain loop
 // (each trailing update split by columns into two launches), so the factor is the same bit for bit. The caller's
 // stream runs the row moves, L21, U12 and the update, stream p the tournaments; events order them.
@@ -1092,24 +1068,15 @@ int getrf_tp_lookahead(T *A, long n, long lda, int *ipiv, int *perm, int *info, 
     if (int rc = tournament(0)) return rc;
     for (long j0 = 0; j0 < n; j0 += TW) {
         const int jb = (int)std::min((long)TW, n - j0);
-        const long m = n - j0;
         if (hipStreamWaitEvent(g, panel, 0) != hipSuccess) return fail(M25X_EHIP, "getrf: wait");
         {
             TimedLaunch tl(g, M25X_K_APPLY_MOVES, dt, 2.0 * es * 2 * jb * n, 0.0);
             hipLaunchKernelGGL(k_apply_moves<T>, dim3(blocks(n, 8) + (perm ? 1 : 0)), dim3(256), 0, g, A, lda, 0L, n,
                                (const int *)pairs, j0, jb, (const T *)top, perm);
         }
-        if (m > jb) {
-            TimedLaunch tl(g, M25X_K_L21, dt, 2.0 * es * (m - jb) * jb, 4.0 * (m - jb) * jb * jb);
-            hipLaunchKernelGGL(k_l21<T>, dim3(blocks(m - jb, 256)), dim3(256), 0, g, A, lda, j0 + jb, m - jb, j0, jb,
-                               (const T *)top);
-        }
         const long c0 = j0 + jb;
         if (c0 < n) {
-            {
-                TimedLaunch tl(g, M25X_K_TRSM, dt, 2.0 * es * (n - c0) * jb, 4.0 * (n - c0) * jb * jb);
-                hipLaunchKernelGGL((k_trsm<T, TW>), dim3(blocks(n - c0, TC)), dim3(256), 0, g, A, lda, n, j0, jb, c0);
-            }
+            launch_tri(g, A, lda, j0, n - c0, (const T *)top);
             const long c1 = std::min(n, c0 + TW);
             update(j0, jb, c0, c0, c1);                                   // the next panel's columns
             if (hipEventRecord(next, g) != hipSuccess || hipStreamWaitEvent(p, next, 0) != hipSuccess)
@@ -1160,18 +1127,10 @@ int getrf_tp(T *A, long n, long lda, int *ipiv, int *perm, int *info, void *work
                                (const int *)pairs, j0, jb, (const T *)top, perm);
         }
         if (int rc = check_launch("getrf/panel")) return rc;
-        if (m > jb) {   // L21 = A21 U11^-1
-            TimedLaunch tl(s, M25X_K_L21, dt, 2.0 * es * (m - jb) * jb, 4.0 * (m - jb) * jb * jb);
-            hipLaunchKernelGGL(k_l21<T>, dim3(blocks(m - jb, 256)), dim3(256), 0, s, A, lda, j0 + jb, m - jb, j0, jb,
-                               (const T *)top);
-        }
         const long c0 = j0 + jb;
-        if (c0 < n) {   // U12 = L11^-1 A12, A22 -= L21 U12
+        if (c0 < n) {   // L21 = A21 U11^-1 and U12 = L11^-1 A12, then A22 -= L21 U12
             T *A12 = A + c0 * lda + j0;
-            {
-                TimedLaunch tl(s, M25X_K_TRSM, dt, 2.0 * es * (n - c0) * jb, 4.0 * (n - c0) * jb * jb);
-                hipLaunchKernelGGL((k_trsm<T, TW>), dim3(blocks(n - c0, TC)), dim3(256), 0, s, A, lda, n, j0, jb, c0);
-            }
+            launch_tri(s, A, lda, j0, n - c0, (const T *)top);
             const long M = n - c0;
             TimedLaunch tl(s, M25X_K_GEMM, dt, es * (2.0 * M * M + 2.0 * M * jb), 8.0 * M * M * jb);
             launch_update<T>(s, dim3(blocks(M, GM), blocks(M, GN)), A + c0 * lda + c0, lda, (const T *)(A + j0 * lda + c0),
@@ -1300,28 +1259,13 @@ __global__ __launch_bounds__(256) void k_apply_moves_b(const m25x_lu_item *items
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_l21_b(const m25x_lu_item *items, long j0)
+__global__ __launch_bounds__(256) void k_tri_b(const m25x_lu_item *items, long j0)
 {
     const m25x_lu_item it = items[blockIdx.y];
-    const long n = it.n;
-    if (j0 >= n) return;
-    const int jb = (int)std::min((long)TW, n - j0);
-    const long rows = n - j0 - jb;
-    if (rows <= 0 || (long)blockIdx.x * 256 >= rows) return;
-    const TourWork<T> w = tour_carve<T>(it.work, n);
-    l21_body<T>((T *)it.A, it.lda, j0 + jb, rows, j0, jb, (const T *)w.top, blockIdx.x);
-}
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_trsm_b(const m25x_lu_item *items, long j0)
-{
-    const m25x_lu_item it = items[blockIdx.y];
-    const long n = it.n;
-    if (j0 >= n) return;
-    const int jb = (int)std::min((long)TW, n - j0);
-    const long c0 = j0 + jb;
-    if (c0 >= n || (long)blockIdx.x * TC >= n - c0) return;
-    trsm_body<T, TW>((T *)it.A, it.lda, n, j0, jb, c0, blockIdx.x);
+    const long m = it.n - j0 - TW, nb21 = (m + TRI_N - 1) / TRI_N;
+    if (m <= 0 || (long)blockIdx.x >= 2 * nb21) return;
+    const TourWork<T> w = tour_carve<T>(it.work, it.n);
+    tri_body<T>((T *)it.A, it.lda, j0, m, (const T *)w.top, blockIdx.x, nb21);
 }
 
 template <typename T, int KS, typename AC = double2>
@@ -1379,10 +1323,9 @@ int getrf_batched_t(int nitems, const m25x_lu_item *h, const m25x_lu_item *d, hi
                 return rc;
         }
         hipLaunchKernelGGL(k_apply_moves_b<T>, dim3(blocks(nbig, 8) + 1, na), dim3(256), 0, s, d, j0);
-        if (mbig > TW) hipLaunchKernelGGL(k_l21_b<T>, dim3(blocks(mbig - TW, 256), na), dim3(256), 0, s, d, j0);
         if (int rc = check_launch("getrf_batched/panel")) return rc;
         if (mbig > TW) {
-            hipLaunchKernelGGL((k_trsm_b<T>), dim3(blocks(mbig - TW, TC), na), dim3(256), 0, s, d, j0);
+            hipLaunchKernelGGL(k_tri_b<T>, dim3(2 * blocks(mbig - TW, TRI_N), na), dim3(256), 0, s, d, j0);
             TimedLaunch tl(s, M25X_K_GEMM, dt, 0.0, flops);
             const dim3 grid(blocks(mbig - TW, GM), blocks(mbig - TW, GN), na);
             const bool f32 = sizeof(T) == 8 && g_update_fp32.load(std::memory_order_relaxed);
