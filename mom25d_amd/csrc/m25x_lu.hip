@@ -266,129 +266,140 @@ __global__ __launch_bounds__(256) void k_trsm(T *A, long lda, long n, long j0, i
     }
 }
 
-// ---- C -= A B (SUB) or C = A B on the matrix cores -------------------------------------------------------
-// C (M x N), A (M x K), B (K x N), column-major, complex. C = A B may overwrite A or B in place when a workgroup
-// tile's output depends on nothing another workgroup writes (M <= 64 with C = B, or N <= 64 with C = A): every
-// workgroup reads all of its K range before it stores. Workgroup tile 64 x 64, four waves of 32 x 32, each
-// 2 x 2 blocks of 16 x 16 with a real and an imaginary accumulator. The MFMA's first operand is B (its rows are
-// C's columns), its second A, so a lane's outputs run down C's columns (coalesced stores).
-constexpr int GM = 64, GN = 64, GK = 8;
+// ---- C -= A B on the matrix cores ---------------------------------------------------------------------------
+// C (M x N), A (M x K), B (K x N), column-major, complex; K a multiple of KS. Workgroup tile 64 x 64, eight waves of 32 x
+// 16, each 2 blocks of 16 x 16 with a real and an imaginary accumulator. The MFMA's first operand is B (its rows are
+// C's columns), its second A, so a lane's outputs run down C's columns (coalesced stores). At K = 64 an update moves as
+// much time's worth of C as it computes (c128: 32 B an entry for 512 flops), so the two have to overlap: a tile's C is
+// asked for first and met last, the stages of A and B alternate between two LDS buffers with one barrier a stage, and
+// the tiles are small and the waves narrow so that four and more a SIMD are at different points of theirs. Loads past
+// the matrix read its last row or column instead of branching (what they feed is never stored). Workgroups are dealt to
+// the eight XCDs round robin; XCD x takes the x-th run of tiles, columns of tiles in order, so its L2 keeps its part of
+// B and the rows of A it meets. Measured at M = 7735, K = 64: 77 -> 89 TFLOP/s (complex64), 37 -> 52 (complex128); tiles of
+// 128 x 64 and 128 x 128, 16-column stages and a persistent grid keeping A's tile measured slower (47 to 87, 30 to 51).
+constexpr int GM = 64, GN = 64, GK = 8, GT = 512;
+constexpr int GWR = 2, GWC = 4;                 // waves down and across a tile
 
-template <typename T, bool SUB, typename AC = T, int KS = GK>
+template <typename T, typename AC = T, int KS = GK>
 __device__ __forceinline__ void gemm_body(T *C, long ldc, const T *A, long lda, const T *B, long ldb, long M, long N,
                                           long K, long bx, long by)
 {
     typedef typename CX<AC>::R R;           // the matrix cores' type: products and sums in it, one rounding to T
     typedef typename CX<T>::R TR;
     typedef typename CX<AC>::acc4 acc4;
-    constexpr int LA = GM * KS / 256, LB = KS * GN / 256;   // a thread's elements of A and of B a stage
-    __shared__ T As[KS][GM];         // As[p][i] = A[i][p]
-    __shared__ T Bs[KS][GN + 1];     // Bs[p][j] = B[p][j]
+    constexpr int LA = GM * KS / GT, LB = KS * GN / GT;     // a thread's elements of A and of B a stage
+    constexpr int FA = GM / GWR / 16, FB = GN / GWC / 16;   // a wave's 16 x 16 blocks
+    __shared__ T As[2][KS][GM];         // As[s][p][i] = A[i][p]
+    __shared__ T Bs[2][KS][GN + 1];     // Bs[s][p][j] = B[p][j]
     const long m0 = bx * GM, n0 = by * GN;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int wm = (wv & 1) * 32, wn = (wv >> 1) * 32;     // wave tile origin in the workgroup tile
+    const int wm = (wv % GWR) * (GM / GWR), wn = (wv / GWR) * (GN / GWC);     // wave tile origin in the workgroup tile
     const int li = lane & 15, kk = lane >> 4, part = kk & 1, ph = kk >> 1;
-    acc4 cr[2][2], ci[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) { cr[a][b][r] = 0; ci[a][b][r] = 0; }
-    // a stage's A (GM x KS) and B (KS x GN) elements of the thread, zero outside, read into registers one stage
-    // ahead: the loads of stage s + 1 are in flight while stage s is multiplied
-    T ra[LA], rb[LB];
+    // (complex values held in registers are kept as separate real and imaginary arrays: an array of the vector type
+    // goes to scratch memory for complex128)
+    TR rax[LA], ray[LA], rbx[LB], rby[LB];
     auto fetch = [&](long k0) __attribute__((always_inline)) {
 #pragma unroll
         for (int it = 0; it < LA; ++it) {
-            const int idx = tid + it * 256, i = idx % GM, p = idx / GM;
-            const long gi = m0 + i, gp = k0 + p;
-            ra[it] = ldz(gi < M && gp < K, A + gp * lda + gi);
+            const int idx = tid + it * GT, i = idx % GM, p = idx / GM;
+            const T v = A[(k0 + p) * lda + std::min(m0 + i, M - 1)];
+            rax[it] = v.x; ray[it] = v.y;
         }
 #pragma unroll
         for (int it = 0; it < LB; ++it) {
-            const int idx = tid + it * 256, p = idx % KS, j = idx / KS;
-            const long gp = k0 + p, gj = n0 + j;
-            rb[it] = ldz(gp < K && gj < N, B + gj * ldb + gp);
+            const int idx = tid + it * GT, p = idx % KS, j = idx / KS;
+            const T v = B[std::min(n0 + j, N - 1) * ldb + k0 + p];
+            rbx[it] = v.x; rby[it] = v.y;
         }
     };
-    fetch(0);
-    for (long k0 = 0; k0 < K; k0 += KS) {
+    auto stage = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
         for (int it = 0; it < LA; ++it) {
-            const int idx = tid + it * 256;
-            As[idx / GM][idx % GM] = ra[it];
+            const int idx = tid + it * GT;
+            As[s][idx / GM][idx % GM] = CX<T>::make(rax[it], ray[it]);
         }
 #pragma unroll
         for (int it = 0; it < LB; ++it) {
-            const int idx = tid + it * 256;
-            Bs[idx % KS][idx / KS] = rb[it];
+            const int idx = tid + it * GT;
+            Bs[s][idx % KS][idx / KS] = CX<T>::make(rbx[it], rby[it]);
         }
-        __syncthreads();
-        if (k0 + KS < K) fetch(k0 + KS);
+    };
+    // lane (li, kk), register r: C row m0 + wm + a*16 + li, column n0 + wn + b*16 + out_row(kk, r)
+    auto row_of = [&](int a) { return m0 + wm + a * 16 + li; };
+    auto col_of = [&](int b, int r) { return n0 + wn + b * 16 + CX<AC>::out_row(kk, r); };
+    fetch(0);
+    TR cx[FB][FA][4], cy[FB][FA][4];
+#pragma unroll
+    for (int b = 0; b < FB; ++b)
+#pragma unroll
+        for (int a = 0; a < FA; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const T v = C[std::min(col_of(b, r), N - 1) * ldc + std::min(row_of(a), M - 1)];
+                cx[b][a][r] = v.x; cy[b][a][r] = v.y;
+            }
+    acc4 cr[FB][FA], ci[FB][FA];
+#pragma unroll
+    for (int b = 0; b < FB; ++b)
+#pragma unroll
+        for (int a = 0; a < FA; ++a)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) { cr[b][a][r] = 0; ci[b][a][r] = 0; }
+    stage(0);
+    __syncthreads();
+    int s = 0;
+    for (long k0 = 0; k0 < K; k0 += KS, s ^= 1) {
+        const bool more = k0 + KS < K;
+        if (more) fetch(k0 + KS);
 #pragma unroll
         for (int ks = 0; ks < KS / 2; ++ks) {
             const int p = 2 * ks + ph;
-            R av[2], br[2], bi[2];
+            R av[FA], br[FB], bi[FB];
 #pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                const T x = As[p][wm + a * 16 + li];
-                av[a] = (R)(part ? x.y : x.x);
-            }
+            for (int a = 0; a < FA; ++a) av[a] = (R)((const TR *)&As[s][p][wm + a * 16 + li])[part];
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const T y = Bs[p][wn + b * 16 + li];
+            for (int b = 0; b < FB; ++b) {
+                const T y = Bs[s][p][wn + b * 16 + li];
                 br[b] = (R)(part ? -y.y : y.x);
                 bi[b] = (R)(part ? y.x : y.y);
             }
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+            for (int b = 0; b < FB; ++b)
 #pragma unroll
-                for (int a = 0; a < 2; ++a) {
+                for (int a = 0; a < FA; ++a) {
                     cr[b][a] = CX<AC>::mfma(br[b], av[a], cr[b][a]);
                     ci[b][a] = CX<AC>::mfma(bi[b], av[a], ci[b][a]);
                 }
         }
+        if (more) stage(s ^ 1);
         __syncthreads();
     }
-    // lane (li, kk), register r: C row m0 + wm + a*16 + li, column n0 + wn + b*16 + out_row(kk, r); for C -= A B
-    // the thread's entries of C are all read first (in flight together), then written
-    T cv[2][2][4];
-    if (SUB) {
+    const bool whole = m0 + GM <= M && n0 + GN <= N;
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < FB; ++b)
 #pragma unroll
-            for (int a = 0; a < 2; ++a)
+        for (int a = 0; a < FA; ++a)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const long gi = m0 + wm + a * 16 + li, gj = n0 + wn + b * 16 + CX<AC>::out_row(kk, r);
-                    cv[b][a][r] = ldz(gi < M && gj < N, C + gj * ldc + gi);
-                }
-    }
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const long gi = m0 + wm + a * 16 + li, gj = n0 + wn + b * 16 + CX<AC>::out_row(kk, r);
-                if (gi < M && gj < N) {
-                    T *c = C + gj * ldc + gi;
-                    if (SUB) {
-                        const T v = cv[b][a][r];
-                        *c = CX<T>::make((TR)((R)v.x - cr[b][a][r]), (TR)((R)v.y - ci[b][a][r]));
-                    } else {
-                        *c = CX<T>::make((TR)cr[b][a][r], (TR)ci[b][a][r]);
-                    }
-                }
-            }
+            for (int r = 0; r < 4; ++r)
+                if (whole || (row_of(a) < M && col_of(b, r) < N))
+                    C[col_of(b, r) * ldc + row_of(a)] = CX<T>::make((TR)((R)cx[b][a][r] - cr[b][a][r]),
+                                                                    (TR)((R)cy[b][a][r] - ci[b][a][r]));
 }
 
-template <typename T, bool SUB, typename AC = T, int KS = GK>
-__global__ __launch_bounds__(256) void k_gemm(T *C, long ldc, const T *A, long lda, const T *B, long ldb, long M,
-                                              long N, long K)
+inline unsigned gemm_grid(long M, long N)
 {
-    gemm_body<T, SUB, AC, KS>(C, ldc, A, lda, B, ldb, M, N, K, blockIdx.x, blockIdx.y);
+    const long t = ((M + GM - 1) / GM) * ((N + GN - 1) / GN);
+    return (unsigned)(8 * ((t + 7) / 8));
+}
+
+// one workgroup a tile of gemm_grid(M, N); the XCD (workgroup i runs on XCD i % 8) takes its run of the tiles
+template <typename T, typename AC = T, int KS = GK>
+__global__ __launch_bounds__(GT) void k_gemm(T *C, long ldc, const T *A, long lda, const T *B, long ldb, long M,
+                                             long N, long K)
+{
+    const long tm = (M + GM - 1) / GM, t = (blockIdx.x & 7) * (long)(gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (t >= tm * ((N + GN - 1) / GN)) return;
+    gemm_body<T, AC, KS>(C, ldc, A, lda, B, ldb, M, N, K, t % tm, t / tm);
 }
 
 // The depth of the K stages of the tournament LU's trailing update (8, 16 or 32: the number of columns of L21 and
@@ -401,27 +412,26 @@ std::atomic<int> g_gemm_stage{8};
 std::atomic<int> g_update_fp32{1};
 
 template <typename T, typename AC>
-void launch_update_ac(hipStream_t s, dim3 grid, T *C, long ldc, const T *A, long lda, const T *B, long ldb, long M,
-                      long N, long K)
+void launch_update_ac(hipStream_t s, T *C, long ldc, const T *A, long lda, const T *B, long ldb, long M, long N, long K)
 {
+    const dim3 grid(gemm_grid(M, N));
     switch (g_gemm_stage.load(std::memory_order_relaxed)) {
-    case 16: hipLaunchKernelGGL((k_gemm<T, true, AC, 16>), grid, dim3(256), 0, s, C, ldc, A, lda, B, ldb, M, N, K); break;
-    case 32: hipLaunchKernelGGL((k_gemm<T, true, AC, 32>), grid, dim3(256), 0, s, C, ldc, A, lda, B, ldb, M, N, K); break;
-    default: hipLaunchKernelGGL((k_gemm<T, true, AC, 8>), grid, dim3(256), 0, s, C, ldc, A, lda, B, ldb, M, N, K);
+    case 16: hipLaunchKernelGGL((k_gemm<T, AC, 16>), grid, dim3(GT), 0, s, C, ldc, A, lda, B, ldb, M, N, K); break;
+    case 32: hipLaunchKernelGGL((k_gemm<T, AC, 32>), grid, dim3(GT), 0, s, C, ldc, A, lda, B, ldb, M, N, K); break;
+    default: hipLaunchKernelGGL((k_gemm<T, AC, 8>), grid, dim3(GT), 0, s, C, ldc, A, lda, B, ldb, M, N, K);
     }
 }
 
 template <typename T>
-void launch_update(hipStream_t s, dim3 grid, T *C, long ldc, const T *A, long lda, const T *B, long ldb, long M,
-                   long N, long K)
+void launch_update(hipStream_t s, T *C, long ldc, const T *A, long lda, const T *B, long ldb, long M, long N, long K)
 {
     if constexpr (sizeof(T) == 8) {
         if (g_update_fp32.load(std::memory_order_relaxed)) {
-            launch_update_ac<T, float2>(s, grid, C, ldc, A, lda, B, ldb, M, N, K);
+            launch_update_ac<T, float2>(s, C, ldc, A, lda, B, ldb, M, N, K);
             return;
         }
     }
-    launch_update_ac<T, double2>(s, grid, C, ldc, A, lda, B, ldb, M, N, K);
+    launch_update_ac<T, double2>(s, C, ldc, A, lda, B, ldb, M, N, K);
 }
 
 // ---- the interchanges as a permutation: perm = the swaps of ipiv applied in order to 0..n-1 ------------------
@@ -981,10 +991,9 @@ int getrf_t(T *A, long n, long lda, int *ipiv, int *info, void *work, size_t wby
             }
             if (int rc = check_launch("getrf/trsm")) return rc;
             const long M = n - c0;
-            dim3 grid(blocks(M, GM), blocks(M, GN));
             {
                 TimedLaunch tl(s, M25X_K_GEMM, dt, es * (2.0 * M * M + 2.0 * M * jb), 8.0 * M * M * jb);
-                hipLaunchKernelGGL((k_gemm<T, true>), grid, dim3(256), 0, s, A + c0 * lda + c0, lda, A + j0 * lda + c0,
+                hipLaunchKernelGGL((k_gemm<T>), dim3(gemm_grid(M, M)), dim3(GT), 0, s, A + c0 * lda + c0, lda, A + j0 * lda + c0,
                                    lda, A + c0 * lda + j0, lda, M, M, (long)jb);
             }
             if (int rc = check_launch("getrf/gemm")) return rc;
@@ -1062,7 +1071,7 @@ int getrf_tp_lookahead(T *A, long n, long lda, int *ipiv, int *perm, int *info, 
     auto update = [&](long j0, int jb, long c0, long c1, long c2) {       // A22[c0:, c1:c2] -= L21 U12[:, c1:c2]
         const long M = n - c0, N = c2 - c1;
         TimedLaunch tl(g, M25X_K_GEMM, dt, es * (2.0 * M * N + (M + N) * jb), 8.0 * M * N * jb);
-        launch_update<T>(g, dim3(blocks(M, GM), blocks(N, GN)), A + c1 * lda + c0, lda,
+        launch_update<T>(g, A + c1 * lda + c0, lda,
                          (const T *)(A + j0 * lda + c0), lda, (const T *)(A + c1 * lda + j0), lda, M, N, (long)jb);
     };
     if (int rc = tournament(0)) return rc;
@@ -1133,7 +1142,7 @@ int getrf_tp(T *A, long n, long lda, int *ipiv, int *perm, int *info, void *work
             launch_tri(s, A, lda, j0, n - c0, (const T *)top);
             const long M = n - c0;
             TimedLaunch tl(s, M25X_K_GEMM, dt, es * (2.0 * M * M + 2.0 * M * jb), 8.0 * M * M * jb);
-            launch_update<T>(s, dim3(blocks(M, GM), blocks(M, GN)), A + c0 * lda + c0, lda, (const T *)(A + j0 * lda + c0),
+            launch_update<T>(s, A + c0 * lda + c0, lda, (const T *)(A + j0 * lda + c0),
                              lda, (const T *)A12, lda, M, M, (long)jb);
         }
         if (int rc = check_launch("getrf/update")) return rc;
@@ -1269,7 +1278,7 @@ __global__ __launch_bounds__(256) void k_tri_b(const m25x_lu_item *items, long j
 }
 
 template <typename T, int KS, typename AC = double2>
-__global__ __launch_bounds__(256) void k_gemm_b(const m25x_lu_item *items, long j0)
+__global__ __launch_bounds__(GT) void k_gemm_b(const m25x_lu_item *items, long j0)
 {
     const m25x_lu_item it = items[blockIdx.z];
     const long n = it.n;
@@ -1279,7 +1288,7 @@ __global__ __launch_bounds__(256) void k_gemm_b(const m25x_lu_item *items, long 
     if (M <= 0 || (long)blockIdx.x * GM >= M || (long)blockIdx.y * GN >= M) return;
     T *A = (T *)it.A;
     const long lda = it.lda;
-    gemm_body<T, true, AC, KS>(A + c0 * lda + c0, lda, A + j0 * lda + c0, lda, A + c0 * lda + j0, lda, M, M, jb,
+    gemm_body<T, AC, KS>(A + c0 * lda + c0, lda, A + j0 * lda + c0, lda, A + c0 * lda + j0, lda, M, M, jb,
                                blockIdx.x, blockIdx.y);
 }
 
@@ -1331,16 +1340,16 @@ int getrf_batched_t(int nitems, const m25x_lu_item *h, const m25x_lu_item *d, hi
             const bool f32 = sizeof(T) == 8 && g_update_fp32.load(std::memory_order_relaxed);
             switch (g_gemm_stage.load(std::memory_order_relaxed)) {
             case 16:
-                if (f32) hipLaunchKernelGGL((k_gemm_b<T, 16, float2>), grid, dim3(256), 0, s, d, j0);
-                else hipLaunchKernelGGL((k_gemm_b<T, 16>), grid, dim3(256), 0, s, d, j0);
+                if (f32) hipLaunchKernelGGL((k_gemm_b<T, 16, float2>), grid, dim3(GT), 0, s, d, j0);
+                else hipLaunchKernelGGL((k_gemm_b<T, 16>), grid, dim3(GT), 0, s, d, j0);
                 break;
             case 32:
-                if (f32) hipLaunchKernelGGL((k_gemm_b<T, 32, float2>), grid, dim3(256), 0, s, d, j0);
-                else hipLaunchKernelGGL((k_gemm_b<T, 32>), grid, dim3(256), 0, s, d, j0);
+                if (f32) hipLaunchKernelGGL((k_gemm_b<T, 32, float2>), grid, dim3(GT), 0, s, d, j0);
+                else hipLaunchKernelGGL((k_gemm_b<T, 32>), grid, dim3(GT), 0, s, d, j0);
                 break;
             default:
-                if (f32) hipLaunchKernelGGL((k_gemm_b<T, 8, float2>), grid, dim3(256), 0, s, d, j0);
-                else hipLaunchKernelGGL((k_gemm_b<T, 8>), grid, dim3(256), 0, s, d, j0);
+                if (f32) hipLaunchKernelGGL((k_gemm_b<T, 8, float2>), grid, dim3(GT), 0, s, d, j0);
+                else hipLaunchKernelGGL((k_gemm_b<T, 8>), grid, dim3(GT), 0, s, d, j0);
             }
         }
         if (int rc = check_launch("getrf_batched/update")) return rc;
