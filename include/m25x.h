@@ -145,10 +145,20 @@ int m25x_near_values(const m25x_mesh *g, const int *P, const int *Q, const doubl
 
 /* Y (+)= A X for a CSR matrix (rowptr: nrow + 1 int32, col int32, vals complex128), X and Y complex128 row-major
  * with k columns (add = 1 adds to Y, 0 overwrites it). With m25x_near_values' entries: near_matvec
- * (src/mom25d/core/mom25d_core.cpp:539-556), deterministic (one thread a row and column, the row's entries in
- * order). */
+ * (src/mom25d/core/mom25d_core.cpp:539-556), deterministic (a wave a row, fixed
+ * summation order). */
 int m25x_csr_matvec(const int *rowptr, const int *col, const double *vals, long nrow, const double *X, int k, long ldx,
                     double *Y, long ldy, int add, void *stream);
+
+/* Workspace bytes of m25x_via_matvec for nv via chains and k columns. */
+size_t m25x_via_matvec_work_bytes(int nv, int k);
+
+/* The via rows and columns of the operator: Y[e] += sum_v B[e, v] X[ne + v] for the ne edge rows (their far and near
+ * parts in Y already), Y[ne + v] = sum_e B[e, v] X[e] + sum_u C[v, u] X[ne + u] for the nv via rows. B (ne x nv), C (nv x
+ * nv) complex128 row-major and contiguous; X and Y (ne + nv) x k, leading dimensions ldx, ldy. Deterministic. The via
+ * part of matvec_exact (src/mom25d/fast.py:571-586). */
+int m25x_via_matvec(const double *B, const double *C, long ne, int nv, const double *X, int k, long ldx, double *Y,
+                    long ldy, void *work, size_t work_bytes, void *stream);
 
 /* Near triangle pairs rho^2 + dz^2 < (fac max(size_p, size_q))^2, sorted by (p, q). Two calls: with P == NULL
  * the count is written to *count (synchronous); then the pairs (int32) are written. Replaces near_pairs

@@ -72,6 +72,8 @@ _SIGS = {
     'm25x_matvec_far': ([P, I, L, P, P, D, P, L, P, S, P], I),
     'm25x_near_values': ([P, P, P, P, L, P, P, D, P, P], I),
     'm25x_csr_matvec': ([P, P, P, L, P, I, L, P, L, I, P], I),
+    'm25x_via_matvec_work_bytes': ([I, I], S),
+    'm25x_via_matvec': ([P, P, L, I, P, I, L, P, L, P, S, P], I),
     'm25x_fan_q': ([P, P, P, I, P, P], I),
     'm25x_radial_table_sum': ([P, P, P, L, L, P, P, L, P, L, D, P, P], I),
     'm25x_hankel': ([P, I, P, I, P, I, P, P], I),

@@ -676,9 +676,20 @@ __global__ __launch_bounds__(MV_P) void k_mv_pairs(DMesh g, DTab T, const double
         if (c < k) { o[3 * c] = ax[c]; o[3 * c + 1] = ay[c]; o[3 * c + 2] = aq[c]; }
 }
 
+// The slices of part summed in slice order, into slice 0: one thread a value. (As a part of the edges' pass, whose
+// threads each walked six values' slices, the sums took 27 us at 2560 triangles and 4 columns; 11 us and 3 us apart.)
+__global__ void k_mv_slices(double2 *part, int nslice, long nv)
+{
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i >= nv) return;
+    double2 v = part[i];
+    for (int sl = 1; sl < nslice; ++sl) v = cadd(v, part[sl * nv + i]);
+    part[i] = v;
+}
+
 // Y[e, c] = sum over the halves (t, alpha, v) of alpha area_t [jw ((c_t - v) . vA_t) + 4 wQ_t / (jw)]
-// (mom25d_core.cpp:300-311), vA and wQ summed over the slices in order
-__global__ void k_mv_out(DMesh g, const double2 *part, int nslice, int k, double w, double2 *Y, long ldy)
+// (mom25d_core.cpp:300-311)
+__global__ void k_mv_out(DMesh g, const double2 *part, int k, double w, double2 *Y, long ldy)
 {
     const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (idx >= (long)g.Ne * k) return;
@@ -690,11 +701,8 @@ __global__ void k_mv_out(DMesh g, const double2 *part, int nslice, int k, double
         const double f = (h ? g.am[e] : g.ap[e]) * g.area[t];
         const double *v = (h ? g.vm : g.vp) + 2 * (size_t)e;
         const double dx = g.cent[2 * t] - v[0], dy = g.cent[2 * t + 1] - v[1];
-        double2 vx = {0, 0}, vy = {0, 0}, wq = {0, 0};
-        for (int sl = 0; sl < nslice; ++sl) {
-            const double2 *o = part + (((size_t)sl * g.Nt + t) * k + c) * 3;
-            vx = cadd(vx, o[0]); vy = cadd(vy, o[1]); wq = cadd(wq, o[2]);
-        }
+        const double2 *o = part + ((size_t)t * k + c) * 3;
+        const double2 vx = o[0], vy = o[1], wq = o[2];
         const double2 u = make_double2(dx * vx.x + dy * vy.x, dx * vx.y + dy * vy.y);
         // jw u + 4 wQ / (jw)
         const double2 z = make_double2(-w * u.y + 4.0 * wq.y * iw, w * u.x - 4.0 * wq.x * iw);
@@ -721,18 +729,90 @@ __global__ __launch_bounds__(256) void k_near_values(DMesh g, const int *P, cons
     vals[e] = acc;
 }
 
-// Y[r, c] (+)= sum over the entries of row r of vals[e] X[col[e], c]; one thread a (row, column)
-__global__ void k_csr_matvec(const int *rowptr, const int *col, const double2 *vals, long nrow, const double2 *X,
-                             int k, long ldx, double2 *Y, long ldy, int add)
+// Y[r, c] (+)= sum over the entries of row r of vals[e] X[col[e], c]: a wave a row, its lanes over the row's entries (so
+// vals and col are read in order), all KM columns at once, the lanes' sums added by a fixed exchange. A thread a (row,
+// column) walked 300 entries one after the other: 109 us at 3512 rows and 4 columns, 12 us so.
+template <int KM>
+__global__ __launch_bounds__(256) void k_csr_matvec(const int *rowptr, const int *col, const double2 *vals, long nrow,
+                                                    const double2 *X, int k, long ldx, double2 *Y, long ldy, int add)
+{
+    const long r = blockIdx.x * 4L + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (r >= nrow) return;
+    double sx[KM], sy[KM];
+#pragma unroll
+    for (int c = 0; c < KM; ++c) sx[c] = sy[c] = 0.0;
+    const int e1 = rowptr[r + 1];
+    for (int e = rowptr[r] + lane; e < e1; e += 64) {
+        const double2 a = vals[e];
+        const double2 *x = X + (size_t)col[e] * ldx;
+#pragma unroll
+        for (int c = 0; c < KM; ++c)
+            if (c < k) {
+                const double2 p = cmul(a, x[c]);
+                sx[c] += p.x; sy[c] += p.y;
+            }
+    }
+#pragma unroll
+    for (int c = 0; c < KM; ++c) {
+        for (int o = 32; o > 0; o >>= 1) { sx[c] += __shfl_xor(sx[c], o); sy[c] += __shfl_xor(sy[c], o); }
+        if (lane == c && c < k) {
+            double2 *y = Y + r * ldy + c;
+            const double2 s = make_double2(sx[c], sy[c]);
+            *y = add ? cadd(*y, s) : s;
+        }
+    }
+}
+
+// ---- the via rows and columns of the operator ---------------------------------------------------------------
+// B (ne x nv) couples the edges and the via chains, C (nv x nv) the chains (row-major). The chains' rows
+// Y[ne + v] = sum_e B[e, v] X[e] + sum_u C[v, u] X[ne + u] in two passes: a workgroup a chain and one of VB blocks of the
+// edges, then the blocks in order with the edges' rows Y[e] += sum_v B[e, v] X[ne + v]. The product with B^T has few
+// outputs and thousands of terms each: a library product gave it one workgroup (384 us at 3512 edges, 4 chains and 4
+// columns; 8 us so).
+constexpr int VB = 32;
+template <int KM>
+__global__ __launch_bounds__(256) void k_via_rows(const double2 *B, long ne, int nv, const double2 *X, int k, long ldx,
+                                                  double2 *part)
+{
+    const int v = blockIdx.y, b = blockIdx.x, tid = threadIdx.x;
+    const long rows = (ne + VB - 1) / VB, r0 = b * rows, r1 = min(ne, r0 + rows);
+    double sx[KM], sy[KM];
+#pragma unroll
+    for (int c = 0; c < KM; ++c) sx[c] = sy[c] = 0.0;
+    for (long e = r0 + tid; e < r1; e += 256) {
+        const double2 a = B[e * nv + v];
+#pragma unroll
+        for (int c = 0; c < KM; ++c)
+            if (c < k) {
+                const double2 p = cmul(a, X[e * ldx + c]);
+                sx[c] += p.x; sy[c] += p.y;
+            }
+    }
+    __shared__ double2 red[4][KM];
+#pragma unroll
+    for (int c = 0; c < KM; ++c) {
+        for (int o = 32; o > 0; o >>= 1) { sx[c] += __shfl_xor(sx[c], o); sy[c] += __shfl_xor(sy[c], o); }
+        if ((tid & 63) == 0) red[tid >> 6][c] = make_double2(sx[c], sy[c]);
+    }
+    __syncthreads();
+    if (tid < k) part[((size_t)v * VB + b) * k + tid] = cadd(cadd(red[0][tid], red[1][tid]), cadd(red[2][tid], red[3][tid]));
+}
+
+__global__ void k_via_out(const double2 *B, const double2 *C, long ne, int nv, const double2 *X, int k, long ldx,
+                          const double2 *part, double2 *Y, long ldy)
 {
     const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (idx >= nrow * k) return;
+    if (idx >= (ne + nv) * k) return;
     const long r = idx / k;
     const int c = (int)(idx % k);
-    double2 acc = add ? Y[r * ldy + c] : make_double2(0, 0);
-    double2 sum = {0, 0};
-    for (int e = rowptr[r]; e < rowptr[r + 1]; ++e) sum = cadd(sum, cmul(vals[e], X[(size_t)col[e] * ldx + c]));
-    Y[r * ldy + c] = cadd(acc, sum);
+    const double2 *a = r < ne ? B + r * nv : C + (r - ne) * nv;
+    double2 s = {0, 0};
+    for (int u = 0; u < nv; ++u) s = cadd(s, cmul(a[u], X[(ne + u) * ldx + c]));
+    if (r < ne) s = cadd(Y[r * ldy + c], s);
+    else
+        for (int b = 0; b < VB; ++b) s = cadd(s, part[((size_t)(r - ne) * VB + b) * k + c]);
+    Y[r * ldy + c] = s;
 }
 
 }  // namespace
@@ -834,8 +914,10 @@ int m25x_matvec_far(const double *X, int k, long ldx, const m25x_mesh *g, const 
         hipLaunchKernelGGL(k_mv_pairs<MV_KMAX>, grid, dim3(MV_P), 0, s, m, dtab(tb), (const double2 *)S,
                            (const int *)act, k, qper, part);
     if (int rc = check_launch("matvec_far")) return rc;
-    hipLaunchKernelGGL(k_mv_out, dim3(blocks((long)g->Ne * k, 256)), dim3(256), 0, s, m, (const double2 *)part,
-                       nslice, k, w, (double2 *)Y, ldy);
+    if (nslice > 1)
+        hipLaunchKernelGGL(k_mv_slices, dim3(blocks(3L * g->Nt * k, 256)), dim3(256), 0, s, part, nslice, 3L * g->Nt * k);
+    hipLaunchKernelGGL(k_mv_out, dim3(blocks((long)g->Ne * k, 256)), dim3(256), 0, s, m, (const double2 *)part, k, w,
+                       (double2 *)Y, ldy);
     return check_launch("matvec_far");
 }
 
@@ -856,9 +938,51 @@ int m25x_csr_matvec(const int *rowptr, const int *col, const double *vals, long 
     if (!rowptr || nrow < 0 || k < 1 || ldx < k || ldy < k || !X || !Y)
         return fail(M25X_EINVAL, "csr_matvec: bad arguments");
     if (nrow == 0) return M25X_OK;
-    hipLaunchKernelGGL(k_csr_matvec, dim3(blocks(nrow * k, 256)), dim3(256), 0, (hipStream_t)stream, rowptr, col,
-                       (const double2 *)vals, nrow, (const double2 *)X, k, ldx, (double2 *)Y, ldy, add);
+    hipStream_t s = (hipStream_t)stream;
+    const double2 *v = (const double2 *)vals, *x = (const double2 *)X;
+    double2 *y = (double2 *)Y;
+    for (int c0 = 0; c0 < k; c0 += MV_KMAX) {       // columns MV_KMAX at a time
+        const int kc = k - c0 < MV_KMAX ? k - c0 : MV_KMAX;
+        if (kc <= 1)
+            hipLaunchKernelGGL(k_csr_matvec<1>, dim3(blocks(nrow, 4)), dim3(256), 0, s, rowptr, col, v, nrow, x + c0, kc,
+                               ldx, y + c0, ldy, add);
+        else if (kc <= 4)
+            hipLaunchKernelGGL(k_csr_matvec<4>, dim3(blocks(nrow, 4)), dim3(256), 0, s, rowptr, col, v, nrow, x + c0, kc,
+                               ldx, y + c0, ldy, add);
+        else
+            hipLaunchKernelGGL(k_csr_matvec<MV_KMAX>, dim3(blocks(nrow, 4)), dim3(256), 0, s, rowptr, col, v, nrow,
+                               x + c0, kc, ldx, y + c0, ldy, add);
+    }
     return check_launch("csr_matvec");
+}
+
+size_t m25x_via_matvec_work_bytes(int nv, int k)
+{
+    return nv > 0 && k > 0 ? sizeof(double2) * (size_t)VB * nv * (k < MV_KMAX ? k : MV_KMAX) : 16;
+}
+
+int m25x_via_matvec(const double *B, const double *C, long ne, int nv, const double *X, int k, long ldx, double *Y,
+                    long ldy, void *work, size_t work_bytes, void *stream)
+{
+    if (ne < 0 || nv < 0 || k < 1 || ldx < k || ldy < k || !X || !Y || (nv && (!B || !C)))
+        return fail(M25X_EINVAL, "via_matvec: bad arguments");
+    if (nv == 0) return M25X_OK;
+    if (!work || work_bytes < m25x_via_matvec_work_bytes(nv, k))
+        return fail(M25X_EINVAL, "via_matvec: workspace of %zu bytes, %zu needed", work_bytes,
+                    m25x_via_matvec_work_bytes(nv, k));
+    hipStream_t s = (hipStream_t)stream;
+    const double2 *b = (const double2 *)B, *c = (const double2 *)C, *x = (const double2 *)X;
+    double2 *y = (double2 *)Y, *part = (double2 *)work;
+    for (int c0 = 0; c0 < k; c0 += MV_KMAX) {
+        const int kc = k - c0 < MV_KMAX ? k - c0 : MV_KMAX;
+        if (kc <= 4)
+            hipLaunchKernelGGL(k_via_rows<4>, dim3(VB, nv), dim3(256), 0, s, b, ne, nv, x + c0, kc, ldx, part);
+        else
+            hipLaunchKernelGGL(k_via_rows<MV_KMAX>, dim3(VB, nv), dim3(256), 0, s, b, ne, nv, x + c0, kc, ldx, part);
+        hipLaunchKernelGGL(k_via_out, dim3(blocks((ne + nv) * kc, 256)), dim3(256), 0, s, b, c, ne, nv, x + c0, kc, ldx,
+                           (const double2 *)part, y + c0, ldy);
+    }
+    return check_launch("via_matvec");
 }
 
 int m25x_near_coo(const m25x_mesh *g, const int *P, const int *Q, const double *M, long n, double w, int *ri, int *ci,

@@ -239,24 +239,37 @@ def csr_matvec(plan, vals, X, Y=None):
     return out[:, 0] if one and not add else out
 
 
-def matvec_far(X, mesh, tabs, w):
-    """Y = Z_far X (device complex128 (Ne,) or (Ne, k)) without forming Z; columns 8 at a time."""
+def matvec_far(X, mesh, tabs, w, out=None):
+    """Y = Z_far X (device complex128 (Ne,) or (Ne, k)) without forming Z; columns 8 at a time. out: a contiguous
+    (Ne, k) complex128 tensor to write (a new one when None)."""
     one = X.dim() == 1
-    X = X.reshape(X.shape[0], -1).to(c128)
+    X = X.reshape(X.shape[0], -1).to(c128).contiguous()
     if X.shape[0] != mesh.Ne:
         raise ValueError("matvec_far: X must have Ne rows")
     k = X.shape[1]
-    Y = torch.empty((mesh.Ne, k), dtype=c128, device=X.device)
+    Y = torch.empty((mesh.Ne, k), dtype=c128, device=X.device) if out is None else out
+    if Y.shape != (mesh.Ne, k) or Y.dtype != c128 or not Y.is_contiguous():
+        raise ValueError("matvec_far: out must be a contiguous complex128 (Ne, k) tensor")
     for c0 in range(0, k, 8):
         kc = min(8, k - c0)
-        Xc = X[:, c0:c0 + kc].contiguous()
-        Yc = torch.empty((mesh.Ne, kc), dtype=c128, device=X.device)
         wb = L.lib().m25x_matvec_far_work_bytes(mesh.Nt, kc)
         work = torch.empty(wb, dtype=torch.uint8, device=X.device)
-        L.call('m25x_matvec_far', ptr(Xc), kc, kc, C.byref(mesh.struct), C.byref(tabs.struct), float(w), ptr(Yc), kc,
-               ptr(work), wb, stream())
-        Y[:, c0:c0 + kc] = Yc
+        L.call('m25x_matvec_far', C.c_void_p(X.data_ptr() + 16 * c0), kc, k, C.byref(mesh.struct),
+               C.byref(tabs.struct), float(w), C.c_void_p(Y.data_ptr() + 16 * c0), k, ptr(work), wb, stream())
     return Y[:, 0] if one else Y
+
+
+def via_matvec(B, Cv, X, Y):
+    """The via rows and columns of Z X: Y[:Ne] += B X[Ne:], Y[Ne:] = B^T X[:Ne] + Cv X[Ne:], with B (Ne, Nv) and Cv
+    (Nv, Nv); X and Y contiguous complex128 (Ne + Nv, k)."""
+    ne, nv = B.shape
+    if X.shape != Y.shape or X.shape[0] != ne + nv or Cv.shape != (nv, nv) or not (
+            X.is_contiguous() and Y.is_contiguous() and X.dtype == Y.dtype == B.dtype == Cv.dtype == c128):
+        raise ValueError("via_matvec: X, Y contiguous complex128 (Ne + Nv, k), B (Ne, Nv), C (Nv, Nv) complex128")
+    B, Cv, k = B.contiguous(), Cv.contiguous(), X.shape[1]
+    wb = L.lib().m25x_via_matvec_work_bytes(nv, k)
+    work = torch.empty(wb, dtype=torch.uint8, device=X.device)
+    L.call('m25x_via_matvec', ptr(B), ptr(Cv), ne, nv, ptr(X), k, k, ptr(Y), k, ptr(work), wb, stream())
 
 
 def near_coo(mesh, plan, M, w):

@@ -136,18 +136,14 @@ class FastOperator:
         and columns and the lumped elements. X: device (N,) or (N, k)."""
         op, Ne = self._op, self.sim.Ne
         one = X.dim() == 1
-        X = X.reshape(X.shape[0], -1).to(dv.c128)
+        X = X.reshape(X.shape[0], -1).to(dv.c128).contiguous()
         if op.get('vals') is None:
             op['vals'] = dv.near_values(self.mesh, self.plan, op['M'], op['w'])
         Y = torch.empty_like(X)
-        Xe = X[:Ne].contiguous()
-        Ye = dv.matvec_far(Xe, self.mesh, self.tabs, op['w'])
-        dv.csr_matvec(self.plan, op['vals'], Xe, Ye)
-        Y[:Ne] = Ye
+        dv.matvec_far(X[:Ne], self.mesh, self.tabs, op['w'], out=Y[:Ne])
+        dv.csr_matvec(self.plan, op['vals'], X[:Ne], Y[:Ne])
         if self.sim.Nv:
-            B, C, Xv = op['B'], op['C'], X[Ne:]
-            Y[:Ne] += B @ Xv
-            Y[Ne:] = B.T @ Xe + C @ Xv
+            dv.via_matvec(op['B'], op['C'], X, Y)
         if op['lumped'] is not None:
             r, c, v = op['lumped']
             Y.index_add_(0, r, v[:, None] * X[c])
