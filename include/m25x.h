@@ -237,8 +237,8 @@ size_t m25x_getrs_work_bytes(int dtype, long n, long ldb);
 
 /* Solves with the factor of m25x_getrf: trans = 1: Z X = B (A^T X = B, lu_solve(..., trans=1)), trans = 0:
  * A X = B. B: n x nrhs row-major (leading dimension ldb >= nrhs, 1 <= nrhs <= 8), the factor's dtype, overwritten
- * with X. perm: m25x_getrf's (or m25x_ipiv_perm's, or NULL: computed here). Diagonal blocks by substitution, as
- * LAPACK's: the accuracy of a factor with small pivots is kept. Every wait between the solve's workgroups is
+ * with X. perm: m25x_getrf's (or m25x_ipiv_perm's, or NULL: computed here). The accuracy of a factor with small
+ * pivots is kept: complex128 diagonal blocks by substitution, as LAPACK's, complex64 ones as FP64 products. Every wait between the solve's workgroups is
  * bounded: the int at work + (work_bytes - 256, rounded down to a multiple of 4), with the work_bytes passed, is
  * nonzero after a call in which one ran out (X is then not the solution), zero otherwise; it is zeroed once per
  * call, so it covers every right-hand side of the call. Replaces the backend's solve (src/mom25d/gpu.py:76-80; src/mom25d/gpu_vk.py:650-678)

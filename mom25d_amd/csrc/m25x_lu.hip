@@ -461,11 +461,7 @@ __global__ void k_perm(const int *ipiv, long n, int *perm)
     }
 }
 
-// ---- triangular solves, one workgroup a 64-row block, ready flags between blocks ---------------------------
-// B: n x nrhs row-major (ldb). The blocks of the solution are published in order; block b takes the contributions
-// of the blocks before it as their flags come up, and solves its diagonal block by substitution (one wave, a row a
-// lane): an explicit inverse of a diagonal block loses the accuracy of a factor with small pivots, which the
-// refinement needs.
+// rows of a block of the triangular solves, and their most right-hand sides
 constexpr int SB = 64;
 constexpr int MAXRHS = 8;
 
@@ -600,15 +596,6 @@ __global__ __launch_bounds__(256) void k_apply_moves(T *A, long lda, long c0, lo
     apply_moves_body<T>(A, lda, c0, nc, pairs, j0, jb, top, perm, blockIdx.x, (long)gridDim.x - 1);
 }
 
-// kind 0: U^T y = b (forward); 1: L^T z = y (backward); 2: L y = b (forward); 3: U x = y (backward).
-// Operator entry (row i, column k): kinds 0, 1 read LU[i * lda + k] (U[k][i], L[k][i]); kinds 2, 3 LU[k * lda + i].
-__host__ __device__ inline bool kind_fwd(int kind) { return kind == 0 || kind == 2; }
-
-__device__ inline float2 readlane_c(float2 v, int l)
-{
-    return make_float2(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.x), l)),
-                       __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v.y), l)));
-}
 __device__ inline double readlane_d(double v, int l)
 {
     const long long b = __double_as_longlong(v);
@@ -616,16 +603,6 @@ __device__ inline double readlane_d(double v, int l)
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 __device__ inline double2 readlane_c(double2 v, int l) { return make_double2(readlane_d(v.x, l), readlane_d(v.y, l)); }
-
-// t - m y with four fused multiply-adds
-__device__ inline float2 cfms(float2 t, float2 m, float2 y)
-{
-    return make_float2(fmaf(-m.x, y.x, fmaf(m.y, y.y, t.x)), fmaf(-m.y, y.x, fmaf(-m.x, y.y, t.y)));
-}
-__device__ inline double2 cfms(double2 t, double2 m, double2 y)
-{
-    return make_double2(fma(-m.x, y.x, fma(m.y, y.y, t.x)), fma(-m.y, y.x, fma(-m.x, y.y, t.y)));
-}
 
 // ---- values that carry their own ready mark ----------------------------------------------------------------
 // The solves hand results between workgroups through buffers filled beforehand with all-ones 64-bit words (a NaN
@@ -673,24 +650,519 @@ template <typename T> __device__ inline bool take(const T *p, T &v)
 }
 __device__ inline bool wave_all(bool c) { return __builtin_amdgcn_ballot_w64(!c) == 0; }
 
-// ---- the triangular solve ----------------------------------------------------------------------------------
+// ---- the triangular solves ---------------------------------------------------------------------------------
+// One launch solves both triangles for all right-hand sides, two to a chain: workgroup q of a chain's pass owns the q-th
+// 64-row diagonal block in solve order and hands its solution to the workgroups after it; the second pass's workgroups
+// take the first one's solution as their right-hand side. The chains of a call run side by side (a solve is bound by the
+// latency from block to block, not by the chip), the workgroups of one block in one XCD so that its L2 serves the
+// block's rows to all of them, and the second pass's workgroups prepare their blocks while the first pass runs.
+// Workgroup q waits only on workgroups before it, which start no later, so the launch makes progress with any number
+// of them resident.
+//
+// y travels as self-marking values (put / take) in dst, chain after chain, the pair of a row side by side: a reader
+// spins on the values themselves, every lane on its own when the block is one of the two before its own (the chain
+// waits on it), one lane with growing naps first otherwise.
 constexpr int TB = 512;                  // threads of a solve workgroup: 8 waves
 constexpr int NWV = TB / 64;
 constexpr int TE = SB * SB / TB;         // entries of a 64 x 64 tile a thread takes: 8
-template <typename T> struct TrsvDepth { static constexpr int D = 3; };  // tiles a workgroup keeps in flight
-template <> struct TrsvDepth<double2> { static constexpr int D = 2; };      // ahead of the values they meet
-template <typename T> struct TrsvMaxRhs { static constexpr int NR = 8; };    // right-hand sides a launch takes
-template <> struct TrsvMaxRhs<double2> { static constexpr int NR = 4; };
+constexpr int CR = 2;                    // right-hand sides of a chain
 
-// Unit-lower (FWD) or unit-upper substitution of NW right-hand sides, lane i row i, with the block's operator Ms
-// in LDS (rows pre-scaled to a unit diagonal; the diagonal, the other triangle and the padding zero): step k
-// broadcasts y_k and every lane subtracts its multiple, the zeros leaving the finished rows alone. After each 8
-// steps the 8 rows they finished (lanes [lo, lo + 8)) are final: pub(lo) hands them on while the rest go on. The
-// row's operator entries are read from LDS one group of 8 steps ahead.
-template <bool FWD, int NW, typename T, class Pub>
-__device__ __attribute__((always_inline)) void subst(T (&t)[NW], const T (*Ms)[SB + 1], int lane, Pub &pub)
+template <typename T> struct Tri {       // one chain's solve of one triangle
+    const T *LU;
+    long lda, n;
+    const T *src;                        // right-hand side: row i at src[(sperm ? sperm[i] : i) * lds + r]
+    long lds;
+    const int *sperm;
+    bool wait;                           // src holds self-marking values
+    T *dst;                              // n x CR solution values, UNSET words before the launch
+    T *out;                              // if given, the solution again: row i at out[(operm ? operm[i] : i) * ldo + r]
+    long ldo;
+    const int *operm;
+    int kc;                              // right-hand sides in use (1 or 2; the other one solves for zero)
+    bool fwd, unit;                      // rows in ascending order (else descending); unit diagonal
+    int *abort;                          // raised if a wait exceeds its bound (the result is then garbage, not a hang)
+};
+
+// workgroup -> (pass, block in solve order, chain): the chains of block q are 8 apart, in q's XCD, and every block
+// before q, and the pass before, has lower numbers
+struct ChainPos {
+    int pass, q, chain;
+};
+__host__ __device__ inline int chain_wgs(int nb, int nchain) { return (nb + 7) / 8 * 8 * nchain; }      // of a pass
+__device__ inline ChainPos chain_pos(int wg, int nb, int nchain)
 {
-    T mk[2][8];
+    const int per = chain_wgs(nb, nchain), pass = wg / per, w = wg - pass * per, t = w / 8;
+    return ChainPos{pass, t / nchain * 8 + w % 8, t % nchain};
+}
+
+template <typename T> __device__ inline void to_out(const Tri<T> &c, long gi, long go, int r, T v)
+{
+    put(c.dst + gi * CR + r, v);
+    if (c.out && r < c.kc) c.out[go * c.ldo + r] = v;
+}
+
+// Polls until the condition holds in every lane of the wave (ok, then what attempt() returns), or the bound is reached
+// (abort raised).
+template <bool NAP, class Try> __device__ __forceinline__ void wave_wait(bool ok, int *abort, Try &&attempt)
+{
+    long spins = 0;
+    while (!wave_all(ok)) {
+        if (NAP) __builtin_amdgcn_s_sleep(1);
+        if (++spins > (1L << 22)) {
+            __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+        }
+        if (!ok) ok = attempt();
+    }
+}
+// d blocks from the chain one lane watches a value, with naps that grow to d / 16 of a us: every later workgroup reads
+// the chain's newest values, and tight polls of all of them on one line would hold up the one that the chain waits for
+template <typename T> __device__ __forceinline__ void nap_wait(const T *w0, int d, int *abort)
+{
+    T v;
+    long spins = 0;
+    const int most = std::min(d, 64);
+    int nap = 1 + most / 8;
+    while (!take(w0, v)) {
+        for (int z = 0; z < nap; ++z) __builtin_amdgcn_s_sleep(2);
+        nap = std::min(2 * nap, most);
+        if (++spins > (1L << 22)) {
+            __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+        }
+    }
+}
+// row gi of the chain's right-hand sides (every lane of the wave calls)
+template <typename T> __device__ __forceinline__ void rhs_row(const Tri<T> &c, long gi, T (&b)[CR])
+{
+    if (c.wait) {
+        const T *p = c.src + gi * CR;
+        auto attempt = [&]() {
+            const bool a0 = take(p, b[0]), a1 = take(p + 1, b[1]);
+            return a0 && a1;
+        };
+        const bool ok = attempt();
+        if (!wave_all(ok)) {
+            if ((threadIdx.x & 63) == 0) nap_wait(p, 64, c.abort);
+            wave_wait<true>(ok, c.abort, attempt);
+        }
+        return;
+    }
+    const T *p = c.src + (c.sperm ? (long)c.sperm[gi] : gi) * c.lds;
+    b[0] = p[0];
+    b[1] = csel(c.kc > 1, p[c.kc > 1 ? 1 : 0], CX<T>::make(0, 0));
+}
+
+// sums within groups of lanes by DPP moves: quad_perm [1,0,3,2] (0xB1), quad_perm [2,3,0,1] (0x4E), row_half_mirror
+// (0x141); and over the halves and quarters of a wave by lane swaps
+template <int CTRL> __device__ __forceinline__ float dpp_of(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL> __device__ __forceinline__ double dpp_of(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | lo);
+}
+__device__ __forceinline__ float swap32_add(float a, float b)     // lanes 0-31: a over both halves; 32-63: b
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap16_add(float a, float b)     // even rows of 16 lanes: a over the pair; odd: b
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double join(unsigned lo, unsigned hi) { return __longlong_as_double(((long long)hi << 32) | lo); }
+__device__ __forceinline__ double swap32_add(double a, double b)
+{
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return join(lo[0], hi[0]) + join(lo[1], hi[1]);
+}
+__device__ __forceinline__ double swap16_add(double a, double b)
+{
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return join(lo[0], hi[0]) + join(lo[1], hi[1]);
+}
+
+// ---- the blocks before a workgroup's own: sum_a Op_qa y_a ----
+// Lane (rl, cq) of wave wv takes rows row(u) and columns 8 wv + 2 cq + v of a 64 x 64 tile, u < 4, v < 2: its loads of 16
+// bytes cover whole lines in either order (row-major: 4 lanes a row; column-major: 16 lanes a column) and it polls y of
+// its own two columns. (A row a lane, as the diagonal block is read, touches 64 lines a load in a row-major factor: of a
+// complex128 solve at N = 7799 it took 0.4 ms.) Tiles are loaded two (complex128) or three blocks ahead of the y they
+// meet.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(8)));    // two complex64, 8-byte aligned
+template <typename T> struct Depth { static constexpr int D = 3; };
+template <> struct Depth<double2> { static constexpr int D = 2; };
+template <typename T> struct Tile {      // entry 2 u + v: row(u), column 2 cq + v
+    typename CX<T>::R r[TE], i[TE];
+    __device__ __forceinline__ void set(int e, T w)
+    {
+        r[e] = w.x;
+        i[e] = w.y;
+    }
+};
+// column-major complex64 rows come in pairs (a load holds two)
+template <typename T, bool RM> __device__ inline int tile_row(int rl, int u)
+{
+    return RM || sizeof(T) == 16 ? rl + 16 * u : 2 * rl + (u & 1) + 32 * (u >> 1);
+}
+
+template <typename T, bool RM>
+__device__ __forceinline__ void load_tile(Tile<T> &t, const Tri<T> &c, long r0, int m, long k0, int rl, int cq)
+{
+    const long gk = k0 + 2 * cq;
+    const bool whole = k0 + TE <= c.n && m == SB;
+    if (whole && sizeof(T) == 8) {
+#pragma unroll
+        for (int h = 0; h < 4; ++h) {    // row-major: two columns of row h; column-major: two rows of a column
+            const T *p = RM ? c.LU + (r0 + rl + 16 * h) * c.lda + gk
+                            : c.LU + (gk + (h & 1)) * c.lda + r0 + 2 * rl + 32 * (h >> 1);
+            const f4u w = *(const f4u *)p;
+            const int e0 = RM ? 2 * h : 4 * (h >> 1) + (h & 1), e1 = RM ? 2 * h + 1 : e0 + 2;
+            t.r[e0] = w.x; t.i[e0] = w.y; t.r[e1] = w.z; t.i[e1] = w.w;
+        }
+        return;
+    }
+    // rows past the block read its last row (their sums are not used), columns past the matrix its last column (y = 0)
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const long gi = r0 + std::min(tile_row<T, RM>(rl, u), m - 1), g = std::min(gk + v, c.n - 1);
+            t.set(2 * u + v, RM ? c.LU[gi * c.lda + g] : c.LU[g * c.lda + gi]);
+        }
+}
+
+// The first D tiles of the sum over blocks 0 .. nfar - 1 of the solve order.
+template <typename T, bool RM, int D, class Order>
+__device__ __forceinline__ void far_begin(Tile<T> (&t)[D], const Tri<T> &c, int nfar, long r0, int m, int wv, int lane,
+                                          Order &&order)
+{
+    const int rl = RM ? lane >> 2 : lane & 15, cq = RM ? lane & 3 : lane >> 4;
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < nfar) load_tile<T, RM>(t[d], c, r0, m, (long)order(d) * SB + wv * TE, rl, cq);
+}
+// o: minus the wave's part of the sum for one row a lane (re and im of the right-hand sides); returns the row. q: the
+// workgroup's own place in the order (how urgent a value is).
+template <typename T, bool RM, int D, class Order>
+__device__ __forceinline__ int far_sum(typename CX<T>::R (&o)[2 * CR], Tile<T> (&t)[D], const Tri<T> &c, int q, int nfar,
+                                       long r0, int m, int wv, int lane, Order &&order)
+{
+    typedef typename CX<T>::R R;
+    const int rl = RM ? lane >> 2 : lane & 15, cq = RM ? lane & 3 : lane >> 4;
+    const long n = c.n;
+    R sr[4][CR], si[4][CR];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int r = 0; r < CR; ++r) sr[u][r] = si[u][r] = 0;
+    // y of a block for this lane, (column v, right-hand side r) at 2 v + r, asked for a step ahead and before the step's
+    // tile: loads return in order, and a poll behind a tile's loads would wait for them
+    T yn[4];
+    auto ask = [&](int p) __attribute__((always_inline)) {
+        const long gk = (long)order(p) * SB + wv * TE + 2 * cq;
+        bool all = true;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) all &= take(c.dst + std::min(gk + e / 2, n - 1) * CR + e % 2, yn[e]);
+        return all;
+    };
+    if (nfar > 0) ask(0);
+    auto step = [&](int p, Tile<T> &tp) __attribute__((always_inline)) {
+        const long k0 = (long)order(p) * SB + wv * TE, gk = k0 + 2 * cq;
+        bool ok = true;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ok &= is_set(yn[e]);
+        ok |= !(gk < n);
+        if (!wave_all(ok)) {
+            if (q - p > 2) {
+                if (lane == 0 && k0 < n) nap_wait(c.dst + k0 * CR, q - p, c.abort);
+                wave_wait<true>(ok, c.abort, [&]() { return ask(p); });
+            } else {
+                wave_wait<false>(ok, c.abort, [&]() { return ask(p); });
+            }
+        }
+        T y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = csel(gk + e / 2 < n, yn[e], CX<T>::make(0, 0));
+        if (p + 1 < nfar) ask(p + 1);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int v = 0; v < 2; ++v)
+#pragma unroll
+                for (int r = 0; r < CR; ++r) {
+                    const T w = tfms(CX<T>::make(sr[u][r], si[u][r]), CX<T>::make(tp.r[2 * u + v], tp.i[2 * u + v]),
+                                     y[2 * v + r]);
+                    sr[u][r] = w.x;
+                    si[u][r] = w.y;
+                }
+        if (p + D < nfar) load_tile<T, RM>(tp, c, r0, m, (long)order(p + D) * SB + wv * TE, rl, cq);
+    };
+    for (int p = 0; p < nfar; p += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (p + d < nfar) step(p + d, t[d]);
+    }
+    // the four lanes of a row exchange: each ends with row(cq)'s sum
+#pragma unroll
+    for (int e = 0; e < 2 * CR; ++e) {
+        const R a0 = e & 1 ? si[0][e / 2] : sr[0][e / 2], a1 = e & 1 ? si[1][e / 2] : sr[1][e / 2],
+                a2 = e & 1 ? si[2][e / 2] : sr[2][e / 2], a3 = e & 1 ? si[3][e / 2] : sr[3][e / 2];
+        if (RM) {
+            const bool b0 = cq & 1, b1 = cq & 2;
+            const R k0 = (b0 ? a1 : a0) + dpp_of<0xB1>(b0 ? a0 : a1);
+            const R k1 = (b0 ? a3 : a2) + dpp_of<0xB1>(b0 ? a2 : a3);
+            o[e] = (b1 ? k1 : k0) + dpp_of<0x4E>(b1 ? k0 : k1);
+        } else {
+            o[e] = swap16_add(swap32_add(a0, a2), swap32_add(a1, a3));
+        }
+    }
+    return tile_row<T, RM>(rl, cq);
+}
+
+// -- complex64 --
+// The block's own triangle is inverted in FP64 when the workgroup starts, and the inverse multiplied into the tile of
+// the block before it (W = inv(Op_qq) Op_q,q-1, FP64 too): a block's step is then y_q = z_q - W y_q-1, one product,
+// with z_q = inv(Op_qq) (b_q - sum over a < q - 1 of Op_qa y_a) formed while y_q-1 is still on its way. Substitution
+// needs 64 dependent steps instead, 1.4 us at 52 cycles (a broadcast and two dependent multiply-adds): the block's step
+// went from 3.0 to 1.5 us (hand-off 0.6, meeting at the barrier 0.15, the product 0.35, its sums over lanes 0.15, and
+// z_q not ready before) and a solve of N = 7799, 4 right-hand sides from 739 to 452 us. The products in FP64 with the
+// inverse in FP64 keep what substitution in FP32 gives and more: an inverse's error, eps64 cond(Op_qq), stays under
+// eps32 up to condition 5e8, and measured against FP64 solves of the same factor the solution's error is
+// 1.3e-7 against the substitution's 3.9e-7 on a board-like system of N = 3001, 6e-5 against 1e-4 on a random one (an
+// inverse or W rounded to FP32 is not good enough: a factor whose pivots span 1e7 then preconditions poorly).
+// The first blocks of a chain take the tile before theirs as any other one: W is ready 10 us after the inverse, and until
+// then the longer step (2.4 us, without W) is the shorter way (N = 905: 109 us with W from the start, 89 so).
+constexpr int FIRST = 6;
+constexpr int S_LD = SB + 1;
+constexpr size_t C64_LDS = 2 * SB * S_LD * sizeof(double2) + SB * sizeof(double2);
+
+__device__ __forceinline__ void zfma(double &r, double &i, double2 a, double2 b)      // (r, i) += a b
+{
+    r = fma(a.x, b.x, fma(-a.y, b.y, r));
+    i = fma(a.y, b.x, fma(a.x, b.y, i));
+}
+
+// X21 = -X22 (S21 X11) for the pairs of H x H blocks of S along the diagonal, X11 and X22 in place of theirs: NO rows of
+// a column a thread, H / NO apart. S21 lies in S; the product S21 X11 goes there first.
+template <int H> __device__ __forceinline__ void invert_level(double2 (*S)[S_LD], int tid)
+{
+    constexpr int NO = H == 32 ? 4 : H == 16 ? 2 : 1, NT = 32 * H / NO, ST = H / NO;
+    const int p = tid / (NT / (SB / 2 / H)), x = tid % (NT / (SB / 2 / H)), i = x / H, j = x % H;
+    double2(*M)[S_LD] = S + p * 2 * H;                       // the pair's corner
+    const int c0 = p * 2 * H;
+    double xr[NO], xi[NO];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        if (tid < NT) {
+#pragma unroll
+            for (int e = 0; e < NO; ++e) xr[e] = xi[e] = 0.0;
+#pragma unroll 4
+            for (int k = 0; k < H; ++k) {                    // triangular factors: zeros past the diagonal
+                const double2 b = half ? M[H + k][c0 + j] : M[k][c0 + j];
+#pragma unroll
+                for (int e = 0; e < NO; ++e) zfma(xr[e], xi[e], M[H + i + ST * e][half ? c0 + H + k : c0 + k], b);
+            }
+        }
+        __syncthreads();
+        if (tid < NT) {
+#pragma unroll
+            for (int e = 0; e < NO; ++e)
+                M[H + i + ST * e][c0 + j] = half ? make_double2(-xr[e], -xi[e]) : make_double2(xr[e], xi[e]);
+        }
+        __syncthreads();
+    }
+}
+
+// The inverse of the lower triangular S (64 x 64, zeros above the diagonal) in place, rd holding the reciprocals of its
+// diagonal: 8 x 8 blocks by substitution, a column a lane, then the blocks off the diagonal.
+__device__ __forceinline__ void invert_lower(double2 (*S)[S_LD], const double2 *rd, int tid)
+{
+    if (tid < 64) {
+        const int o = tid & ~7, j = tid & 7;
+        double xr[8], xi[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            double sr = i == j ? 1.0 : 0.0, si = 0.0;
+#pragma unroll
+            for (int k = 0; k < i; ++k) {
+                const double2 a = S[o + i][o + k];
+                sr = fma(-a.x, xr[k], fma(a.y, xi[k], sr));
+                si = fma(-a.y, xr[k], fma(-a.x, xi[k], si));
+            }
+            const double2 d = rd[o + i];
+            xr[i] = sr * d.x - si * d.y;
+            xi[i] = sr * d.y + si * d.x;
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const bool in = i >= j;
+            S[o + i][o + j] = make_double2(in ? xr[i] : 0.0, in ? xi[i] : 0.0);
+        }
+    }
+    __syncthreads();
+    invert_level<8>(S, tid);
+    invert_level<16>(S, tid);
+    invert_level<32>(S, tid);
+}
+
+// (ar, ai)[r] += sum over the lane's columns c8 + 8 v of (wr, wi)[v] x[column][r]
+__device__ __forceinline__ void rows_product(double (&ar)[CR], double (&ai)[CR], const double (&wr)[TE],
+                                             const double (&wi)[TE], const double2 (*x)[CR], int c8)
+{
+#pragma unroll
+    for (int v = 0; v < TE; ++v)
+#pragma unroll
+        for (int r = 0; r < CR; ++r) zfma(ar[r], ai[r], make_double2(wr[v], wi[v]), x[c8 + 8 * v][r]);
+}
+
+template <bool RM>
+__device__ __forceinline__ void chain_of(const Tri<float2> &c, int q)
+{
+    __shared__ __align__(16) unsigned char lds[C64_LDS];
+    double2(*S)[S_LD] = (double2(*)[S_LD])lds;               // the triangle, then its inverse (solve order, lower)
+    double2(*N)[S_LD] = S + SB;                              // the tile of the block before (rows in solve order)
+    double2 *rd = (double2 *)(N + SB);
+    const long n = c.n;
+    const int nb = (int)((n + SB - 1) / SB);
+    if (q >= nb) return;
+    const bool fwd = c.fwd, unit = c.unit;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto order = [&](int p) { return fwd ? p : nb - 1 - p; };
+    auto flip = [&](int i) { return fwd ? i : SB - 1 - i; };               // local row <-> its place in solve order
+    const long r0 = (long)order(q) * SB;
+    const int m = (int)std::min((long)SB, n - r0);                         // rows of this block inside the matrix
+    const bool near = q > FIRST;
+    const int nfar = near ? q - 1 : q;
+
+    // the diagonal block and the tile before it, whole lines a load; indices clamped into the matrix
+    float2 md[TE], mn[TE];
+    const long kn = (long)order(near ? q - 1 : 0) * SB;
+#pragma unroll
+    for (int u = 0; u < TE; ++u) {
+        const int i = RM ? wv * TE + u : lane, k = RM ? lane : wv * TE + u;
+        const long gi = r0 + std::min(i, m - 1), gk = r0 + std::min(k, m - 1), gn = std::min(kn + k, n - 1);
+        md[u] = RM ? c.LU[gi * c.lda + gk] : c.LU[gk * c.lda + gi];
+        mn[u] = RM ? c.LU[gi * c.lda + gn] : c.LU[gn * c.lda + gi];
+    }
+    // the lane's row of the products below: waves w and w + 4 share a SIMD, and W's rows take more the later they are
+    const int li = 8 * (wv < 4 ? wv : 11 - wv) + (lane >> 3), c8 = lane & 7, gl = flip(li);
+    const bool inrow = gl < m;
+    const long grow = r0 + std::min(gl, m - 1);
+    const long orow = c.out && c.operm ? c.operm[grow] : grow;
+    constexpr int D = Depth<float2>::D;
+    Tile<float2> t[D];
+    far_begin<float2, RM>(t, c, nfar, r0, m, wv, lane, order);
+#pragma unroll
+    for (int u = 0; u < TE; ++u) {       // rows and columns past the matrix: those of the unit matrix
+        const int i = RM ? wv * TE + u : lane, k = RM ? lane : wv * TE + u, si = flip(i), sk = flip(k);
+        const bool in = i < m && k < m && (sk < si || (sk == si && !unit));
+        double2 v = make_double2(in ? (double)md[u].x : 0.0, in ? (double)md[u].y : 0.0);
+        if (si == sk) {
+            if (!in) v.x = 1.0;
+            rd[si] = trecip(v);
+        }
+        S[si][sk] = v;
+        N[si][k] = make_double2(i < m ? (double)mn[u].x : 0.0, i < m ? (double)mn[u].y : 0.0);
+    }
+    __syncthreads();
+    invert_lower(S, rd, tid);
+    double vr[TE], vi[TE], wr[TE], wi[TE];                                 // row li of the inverse, and of -W
+#pragma unroll
+    for (int v = 0; v < TE; ++v) {
+        const double2 a = S[li][c8 + 8 * v];
+        vr[v] = a.x;
+        vi[v] = a.y;
+        wr[v] = wi[v] = 0.0;
+    }
+    if (near) {
+        const int kend = 8 * (wv < 4 ? wv : 11 - wv) + 8;                  // the inverse is zero past its diagonal
+#pragma unroll 2
+        for (int k = 0; k < kend; ++k) {
+            const double2 a = S[li][k];
+            const double2 na = make_double2(-a.x, -a.y);
+#pragma unroll
+            for (int v = 0; v < TE; ++v) zfma(wr[v], wi[v], na, N[k][c8 + 8 * v]);
+        }
+    }
+    __syncthreads();
+    float4(*red)[SB] = (float4(*)[SB])lds;                                 // [wave][row]: partial sums of the pair
+    double2(*vb)[CR] = (double2(*)[CR])(red + NWV);                        // the block's right-hand sides
+    double2(*yb)[CR] = vb + SB;                                            // y of the block before
+    float2 bx[CR];
+    rhs_row(c, grow, bx);
+    {
+        float o[2 * CR];
+        const int i = far_sum<float2, RM>(o, t, c, q, nfar, r0, m, wv, lane, order);
+        red[wv][flip(i)] = make_float4(o[0], o[1], o[2], o[3]);
+    }
+    __syncthreads();
+    {                                    // the 8 waves' sums of row li meet in its 8 lanes
+        const float4 g = red[c8][li];
+        float h[2 * CR] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+        for (int e = 0; e < 2 * CR; ++e) {
+            h[e] += dpp_of<0xB1>(h[e]);
+            h[e] += dpp_of<0x4E>(h[e]);
+            h[e] += dpp_of<0x141>(h[e]);
+        }
+        if (c8 < CR)
+            vb[li][c8] = make_double2(inrow ? (double)((c8 ? bx[1].x : bx[0].x) + (c8 ? h[2] : h[0])) : 0.0,
+                                      inrow ? (double)((c8 ? bx[1].y : bx[0].y) + (c8 ? h[3] : h[1])) : 0.0);
+    }
+    __syncthreads();
+    // the block before: lanes 0-15 of wave wv poll its rows 8 wv .. 8 wv + 7, first while z is formed
+    const long gk = kn + 8 * wv + lane / CR;
+    const bool need = near && lane < 8 * CR && gk < n;
+    float2 y = make_float2(0.f, 0.f);
+    auto attempt = [&]() { return take(c.dst + gk * CR + lane % CR, y); };
+    __builtin_amdgcn_s_setprio(3);
+    if (need) y = fetch(c.dst + gk * CR + lane % CR);
+    __builtin_amdgcn_sched_barrier(0);
+    double ar[CR] = {0.0, 0.0}, ai[CR] = {0.0, 0.0};
+    rows_product(ar, ai, vr, vi, vb, c8);
+    __builtin_amdgcn_sched_barrier(0);       // y is looked at after the product
+    if (near) {
+        wave_wait<false>(is_set(y), c.abort, attempt);
+        if (lane < 8 * CR)
+            yb[8 * wv + lane / CR][lane % CR] = make_double2(need ? (double)y.x : 0.0, need ? (double)y.y : 0.0);
+        __syncthreads();
+        rows_product(ar, ai, wr, wi, yb, c8);
+    }
+    // the sums over the row's 8 lanes: each keeps one right-hand side (its lowest bit)
+    const bool b0 = c8 & 1;
+    double xr = (b0 ? ar[1] : ar[0]) + dpp_of<0xB1>(b0 ? ar[0] : ar[1]);
+    double xi = (b0 ? ai[1] : ai[0]) + dpp_of<0xB1>(b0 ? ai[0] : ai[1]);
+    xr += dpp_of<0x4E>(xr);
+    xi += dpp_of<0x4E>(xi);
+    // the two quads of a row: the half mirror pairs lane c8 with 7 - c8, the other right-hand side; a quad swap
+    // within it puts that right
+    xr += dpp_of<0x141>(dpp_of<0xB1>(xr));
+    xi += dpp_of<0x141>(dpp_of<0xB1>(xi));
+    if (inrow && c8 < CR) to_out(c, grow, orow, c8, make_float2((float)xr, (float)xi));
+}
+
+// -- complex128 --
+// The diagonal blocks by substitution (an inverse in the same precision as the factor would lose the accuracy of one
+// with small pivots). Unit-lower (FWD) or unit-upper substitution of one right-hand side, lane i row i, with the
+// block's operator Ms in LDS (rows pre-scaled to a unit diagonal; the diagonal, the other triangle and the padding
+// zero): step k broadcasts y_k and every lane subtracts its multiple, the zeros leaving the finished rows alone. After
+// each 8 steps the 8 rows they finished (lanes [lo, lo + 8)) are final: pub(lo) hands them on while the rest go on. The
+// row's operator entries are read from LDS one group of 8 steps ahead.
+template <bool FWD, class Pub>
+__device__ __attribute__((always_inline)) void subst(double2 &t, const double2 (*Ms)[SB + 1], int lane, Pub &pub)
+{
+    double2 mk[2][8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) mk[0][j] = Ms[lane][FWD ? j : SB - 1 - j];
 #pragma unroll
@@ -703,223 +1175,132 @@ __device__ __attribute__((always_inline)) void subst(T (&t)[NW], const T (*Ms)[S
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int k = FWD ? s0 + j : SB - 1 - s0 - j;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) t[w] = cfms(t[w], mk[g][j], readlane_c(t[w], k));
+            t = tfms(t, mk[g][j], readlane_c(t, k));
         }
         pub(FWD ? s0 : SB - 8 - s0);
     }
 }
 
-// One launch of nb workgroups of 512 threads solves one triangle for nrhs <= NR right-hand sides. Workgroup q
-// owns the q-th 64-row diagonal block in solve order (the chain passes from workgroup to workgroup):
-//  - at its start it stages its diagonal block's operator in LDS (strict triangle, rows scaled by 1 / U_ii) and
-//    reads its right-hand sides;
-//  - it then meets the earlier blocks a in order: thread (row lane, columns 8 wv + u of block a) holds its
-//    entries of Op_qa, loaded TrsvDepth blocks ahead, and subtracts Op_qa y_a from its partial sums once y_a is
-//    out (fused multiply-subtracts: four per complex term);
-//  - after the last one (a = q - 1) the partial sums meet in LDS, waves 0-3 form the block's right-hand side
-//    (wave w takes right-hand sides w and, for NR = 8, w + 4; lane i row i), substitute, and publish y_q eight
-//    rows at a time as the substitution finishes them: the next workgroup's wave that takes those rows starts its
-//    product with them while the substitution goes on, so the chain's hand-off overlaps the substitution.
-// y travels as self-marking values (put / take) in dst: a reader spins on the values themselves, every lane on its
-// own when the block is one of the two before its own (the chain waits on it), one lane with growing naps first
-// otherwise. Workgroup q waits only on workgroups before it, which start no later, so the launch makes progress
-// with any number of them resident.
-//
-// rdg: 1 / U_ii (read for the kinds with U only: L is unit). src: n x nrhs (leading dimension lds); dst: n x nrhs
-// (leading dimension nrhs) filled with UNSET words beforehand. abort: raised if a wait exceeds its bound (the result
-// is then garbage, not a hang). NR: 4 (nrhs <= 4) or 8.
-template <typename T, int NR>
-__device__ __forceinline__ void trsv_body(const T *LU, long lda, long n, const T *rdg, const T *src, long lds, T *dst,
-                                          int nrhs, int kind, int *abort, int q)
+// Workgroup q stages its diagonal block's operator in LDS (strict triangle, rows scaled by 1 / U_ii), sums the earlier
+// blocks' part, and waves 0 and 1 form the block's right-hand sides (one each; lane i row i), substitute, and publish y_q
+// eight rows at a time as the substitution finishes them: the next workgroup's wave that takes those rows starts its
+// product with them while the substitution goes on, so the chain's hand-off overlaps the substitution.
+// Two right-hand sides to a chain: a call of 5 to 8 ran as two calls of 4 one after the other, and the products of 4
+// took 0.25 us more of a block's step than those of 2. N = 3001, 7 right-hand sides: 650 -> 333 us, 3.3 us
+// a block, of which the substitution is 1.8.
+template <bool RM>
+__device__ __forceinline__ void chain_of(const Tri<double2> &c, int q)
 {
-    constexpr int NW = NR / 4;               // right-hand sides a solver wave takes
-    constexpr int D = TrsvDepth<T>::D;
+    typedef double2 T;
     __shared__ T Ms[SB][SB + 1];             // the diagonal block's operator
-    __shared__ T red[NWV][NR][SB];           // the waves' partial sums
-    __shared__ T yb[NWV][64];                // each wave's y values of the block it meets
+    __shared__ T red[NWV][CR][SB];           // the waves' partial sums
+    // the right-hand sides and 1 / U_ii of the rows (past n: zeroed where used), parked in LDS until the substitution:
+    // held in registers across the loop they are spilled to scratch, and reloading them would put a memory round trip
+    // into every step of the chain
+    __shared__ T bxs[CR][SB], rds[SB];
+    const T *LU = c.LU;
+    const long n = c.n, lda = c.lda;
     const int nb = (int)((n + SB - 1) / SB);
     if (q >= nb) return;
-    const bool fwd = kind_fwd(kind), rowmajor = kind <= 1, unit = kind == 1 || kind == 2;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const T zero = CX<T>::make(0, 0), one = CX<T>::make(1, 0);
+    const bool fwd = c.fwd, unit = c.unit;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const T zero = make_double2(0, 0), one = make_double2(1, 0);
     auto order = [&](int p) { return fwd ? p : nb - 1 - p; };
-    auto opp = [&](long gi, long gk) { return rowmajor ? LU + gi * lda + gk : LU + gk * lda + gi; };
-    const long kstep = rowmajor ? 1 : lda;   // address step along a row of the operator
-    const int b = order(q);
-    const long r0 = (long)b * SB;
+    auto opp = [&](long gi, long gk) { return RM ? LU + gi * lda + gk : LU + gk * lda + gi; };
+    const long r0 = (long)order(q) * SB;
     const int m = (int)std::min((long)SB, n - r0);          // rows of this block inside the matrix
 
     // the diagonal block: thread (rows 8 wv + u, column lane) of a row-major operator, (row lane, columns 8 wv + u)
     // of a column-major one, so that every load reads whole lines; indices clamped into the block, the entries
     // outside it or outside the strict triangle zeroed when staged
-    T md[TE], mr[TE];
+    T md[TE];
 #pragma unroll
     for (int u = 0; u < TE; ++u) {
-        const int i = rowmajor ? wv * TE + u : lane, k = rowmajor ? lane : wv * TE + u;
-        const long gi = r0 + std::min(i, m - 1), gk = r0 + std::min(k, m - 1);
-        md[u] = *opp(gi, gk);
-        mr[u] = rdg[gi];                     // read either way: a select of values, not of addresses
+        const int i = RM ? wv * TE + u : lane, k = RM ? lane : wv * TE + u;
+        md[u] = *opp(r0 + std::min(i, m - 1), r0 + std::min(k, m - 1));
     }
-    // the solver waves' right-hand sides and 1 / U_ii of the lane's row (rows past n: zeroed where used), parked in
-    // LDS until the substitution: held in registers across the loop they are spilled to scratch for complex128, and
-    // reloading them would put a memory round trip into every step of the chain
-    __shared__ T bxs[NR][SB], rds[SB];
-    int rr[NW];
-#pragma unroll
-    for (int w = 0; w < NW; ++w) rr[w] = (wv & 3) + 4 * w;
-    if (wv < 4) {
-        const long gi = r0 + std::min(lane, m - 1);
-#pragma unroll
-        for (int w = 0; w < NW; ++w) bxs[rr[w]][lane] = src[gi * lds + std::min(rr[w], nrhs - 1)];
-        if (wv == 0) rds[lane] = csel(unit, one, rdg[gi]);
-    }
-
-    // the earlier blocks' entries: thread (row lane, columns 8 wv + u of block a); a row past the matrix reads the
-    // last row (its sums are never used), columns past it meet zero y
-    auto load_tile = [&](T (&mt)[TE], int a) __attribute__((always_inline)) {
-        const long gi = r0 + std::min(lane, m - 1), k0 = (long)a * SB + wv * TE;
-        const T *p = opp(gi, k0);
-        if (k0 + TE <= n) {
-#pragma unroll
-            for (int u = 0; u < TE; ++u) mt[u] = p[u * kstep];
-        } else {                             // columns from n on read column n - 1 (ul < 0 past the matrix)
-            const int ul = (int)(n - 1 - k0);
-#pragma unroll
-            for (int u = 0; u < TE; ++u) mt[u] = p[(u < ul ? u : ul) * kstep];
-        }
-    };
-    auto stage = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < TE; ++u) {
-            const int i = rowmajor ? wv * TE + u : lane, k = rowmajor ? lane : wv * TE + u;
-            const bool in = i < m && k < m && (fwd ? k < i : k > i);
-            Ms[i][k] = csel(in, csel(unit, md[u], tmul(md[u], mr[u])), zero);
-        }
-    };
-    // complex128 stages the diagonal block before its first tiles are asked for (registers), complex64 after
-    if constexpr (sizeof(T) == 16) stage();
-    T m0[TE], m1[TE], m2[TE];
-    if (q > 0) load_tile(m0, order(0));
-    if (q > 1) load_tile(m1, order(1));
-    if (D > 2 && q > 2) load_tile(m2, order(2));
-    if constexpr (sizeof(T) != 16) stage();
-
-    T s[NR];                                 // minus the wave's share of the products
-#pragma unroll
-    for (int r = 0; r < NR; ++r) s[r] = zero;
-    // lane l < 8 NR of wave wv takes y of row 8 wv + l / NR of block a, right-hand side l % NR (zero for the
-    // right-hand sides past nrhs)
-    const int lu_ = lane / NR, lr = lane % NR;
-    T *ybw = yb[wv];
-    auto step = [&](int p, T (&mt)[TE]) __attribute__((always_inline)) {
-        const int a = order(p);
-        const long g0 = (long)a * SB + wv * TE, gk = g0 + lu_;
-        const bool need = lane < TE * NR && lr < nrhs && gk < n;
-        if (q - p > 2 && lane == 0 && g0 < n) {   // far from the chain: one lane watches the slice's first value
-            const T *w0 = dst + g0 * nrhs;         // with growing naps first (a slice past n needs none)
-            T v;
-            long spins = 0;
-            int nap = 1;
-            while (!take(w0, v)) {
-                for (int z = 0; z < nap; ++z) __builtin_amdgcn_s_sleep(2);
-                nap = nap < 8 ? 2 * nap : 8;
-                if (++spins > (1L << 22)) {
-                    __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-            }
-        }                                          // near it, every lane polls its own value from the start
-        T yv = zero;
-        bool ok = !need || take(dst + gk * nrhs + lr, yv);
-        long spins = 0;
-        while (!wave_all(ok)) {
-            __builtin_amdgcn_s_sleep(1);
-            if (++spins > (1L << 22)) {
-                __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                break;
-            }
-            if (!ok) ok = take(dst + gk * nrhs + lr, yv);
-        }
-        if (!need) yv = zero;
-        ybw[lane] = yv;
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int u = 0; u < TE; ++u) {
-#pragma unroll
-            for (int r = 0; r < NR; ++r) s[r] = cfms(s[r], mt[u], ybw[u * NR + r]);
-            if constexpr (sizeof(T) == 16) __builtin_amdgcn_sched_barrier(0);     // y read as it is used
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (p + D < q) load_tile(mt, order(p + D));
-    };
-    for (int p = 0; p < q; p += D) {
-        step(p, m0);
-        if (p + 1 < q) step(p + 1, m1);
-        if (D > 2 && p + 2 < q) step(p + 2, m2);
-    }
-#pragma unroll
-    for (int r = 0; r < NR; ++r) red[wv][r][lane] = s[r];
+    const long grow = r0 + std::min(lane, m - 1);
+    if (wv == 0) rds[lane] = csel(unit, one, trecip(*opp(grow, grow)));
+    constexpr int D = Depth<T>::D;
+    Tile<T> t[D];
+    far_begin<T, RM>(t, c, q, r0, m, wv, lane, order);
     __syncthreads();
-    if (wv >= 4) return;
-    const bool inrow = lane < m;
-    T t[NW];
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        T h[NWV];                            // the 8 waves' partial sums, added as a tree (depth 3)
-#pragma unroll
-        for (int sl = 0; sl < NWV; ++sl) h[sl] = red[sl][rr[w]][lane];
-#pragma unroll
-        for (int st = 1; st < NWV; st *= 2)
-#pragma unroll
-            for (int sl = 0; sl + st < NWV; sl += 2 * st) h[sl] = tadd(h[sl], h[sl + st]);
-        const T v = h[0];
-        t[w] = csel(inrow && rr[w] < nrhs, tmul(tadd(bxs[rr[w]][lane], v), rds[lane]), zero);
+    for (int u = 0; u < TE; ++u) {
+        const int i = RM ? wv * TE + u : lane, k = RM ? lane : wv * TE + u;
+        const bool in = i < m && k < m && (fwd ? k < i : k > i);
+        Ms[i][k] = csel(in, csel(unit, md[u], tmul(md[u], rds[i])), zero);
     }
-    auto pub = [&](int lo) __attribute__((always_inline)) {
-        if (lane >= lo && lane < lo + 8 && inrow) {
+    if (wv == 0) {
+        T b[CR];
+        rhs_row(c, grow, b);
+        bxs[0][lane] = b[0];
+        bxs[1][lane] = b[1];
+    }
+    {
+        double o[2 * CR];
+        const int i = far_sum<T, RM>(o, t, c, q, q, r0, m, wv, lane, order);
+        red[wv][0][i] = make_double2(o[0], o[1]);
+        red[wv][1][i] = make_double2(o[2], o[3]);
+    }
+    __syncthreads();
+    if (wv >= CR) return;
+    const bool inrow = lane < m;
+    T h[NWV];                                // the 8 waves' partial sums, added as a tree (depth 3)
 #pragma unroll
-            for (int w = 0; w < NW; ++w)
-                if (rr[w] < nrhs) put(dst + (r0 + lane) * nrhs + rr[w], t[w]);
-        }
+    for (int sl = 0; sl < NWV; ++sl) h[sl] = red[sl][wv][lane];
+#pragma unroll
+    for (int st = 1; st < NWV; st *= 2)
+#pragma unroll
+        for (int sl = 0; sl + st < NWV; sl += 2 * st) h[sl] = tadd(h[sl], h[sl + st]);
+    T y = csel(inrow, tmul(tadd(bxs[wv][lane], h[0]), rds[lane]), zero);
+    auto pub = [&](int lo) __attribute__((always_inline)) {
+        if (lane >= lo && lane < lo + 8 && inrow) put(c.dst + grow * CR + wv, y);
     };
-    if (fwd) subst<true, NW>(t, Ms, lane, pub);
-    else subst<false, NW>(t, Ms, lane, pub);
+    if (fwd) subst<true>(y, Ms, lane, pub);
+    else subst<false>(y, Ms, lane, pub);
+    if (inrow && c.out && wv < c.kc) c.out[(c.operm ? (long)c.operm[grow] : grow) * c.ldo + wv] = y;
 }
 
-template <typename T, int NR>
-__global__ __launch_bounds__(TB) void k_trsv(const T *LU, long lda, long n, const T *rdg, const T *src, long lds,
-                                             T *dst, int nrhs, int kind, int *abort)
-{
-    trsv_body<T, NR>(LU, lda, n, rdg, src, lds, dst, nrhs, kind, abort, blockIdx.x);
-}
-
-// 1 / U_ii for the substitutions with U and U^T
+// the chain's part of one call: pass 0 reads B, pass 1 the solution of pass 0 and also writes B (every workgroup that
+// reads a row of B has done so before the second pass has a solution for it: that needs the first pass's last block)
 template <typename T>
-__global__ void k_rdiag(const T *LU, long lda, long n, T *rd)
+__device__ __forceinline__ Tri<T> chain_args(const T *LU, long lda, long n, T *B, long ldb, const int *perm, T *W1, T *W2,
+                                             int nrhs, int trans, const ChainPos &at, int *abort)
+{
+    Tri<T> c;
+    const int pass = at.pass;
+    T *Bc = B + at.chain * CR;
+    c.LU = LU; c.lda = lda; c.n = n;
+    c.kc = std::min(CR, nrhs - at.chain * CR);
+    c.fwd = pass == 0;                       // U^T, then L^T (row-major: RM); or L, then U
+    c.unit = pass == trans;
+    c.abort = abort;
+    c.wait = pass;
+    c.src = pass ? W1 + at.chain * CR * n : Bc;
+    c.lds = ldb;
+    c.sperm = pass || trans ? nullptr : perm;
+    c.dst = (pass ? W2 : W1) + at.chain * CR * n;
+    c.out = pass ? Bc : nullptr;
+    c.ldo = ldb;
+    c.operm = pass && trans ? perm : nullptr;
+    return c;
+}
+
+// RM: the operator's rows are contiguous (trans = 1: U^T then L^T in the factor's row-major buffer)
+template <typename T, bool RM>
+__global__ __launch_bounds__(TB) void k_trsv(const T *LU, long lda, long n, T *B, long ldb, const int *perm, T *W1, T *W2,
+                                             int nrhs, int *abort)
+{
+    const ChainPos at = chain_pos(blockIdx.x, (int)((n + SB - 1) / SB), (nrhs + CR - 1) / CR);
+    chain_of<RM>(chain_args(LU, lda, n, B, ldb, perm, W1, W2, nrhs, (int)RM, at, abort), at.q);
+}
+
+// UNSET words to the first n words of each of gridDim.y buffers
+__global__ void k_fill_unset(u64 *p, long pitch, long n)
 {
     const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i < n) rd[i] = trecip(LU[i * lda + i]);
-}
-
-// out[perm[i]] = in[i] (scatter, trans) or out[i] = in[perm[i]] (gather); perm NULL: a copy. Leading dimensions
-// ldi (in) and ldo (out).
-template <typename T>
-__global__ void k_permute(const T *in, long ldi, T *out, long ldo, long n, int nrhs, const int *perm, int scatter)
-{
-    const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (idx >= n * nrhs) return;
-    const long i = idx / nrhs;
-    const int r = (int)(idx % nrhs);
-    const long p = perm ? (long)perm[i] : i;
-    if (scatter) out[p * ldo + r] = in[i * ldi + r];
-    else out[i * ldo + r] = in[p * ldi + r];
-}
-
-__global__ void k_fill_unset(unsigned long long *p, long n)
-{
-    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i < n) p[i] = ~0ull;
+    if (i < n) p[blockIdx.y * pitch + i] = UNSET;
 }
 
 inline unsigned blocks(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -1150,80 +1531,52 @@ int getrf_tp(T *A, long n, long lda, int *ipiv, int *perm, int *info, void *work
     return M25X_OK;
 }
 
-// Solve workspace: y of the two solves (W1, W2), written as self-marking values over UNSET words; the gathered
-// right-hand sides (W0); 1 / U_ii; the permutation, the abort word (at the passed work_bytes - 256, rounded down
-// to an int: callers read it there)
-// and 63 spare ints.
+// Solve workspace: y of the two solves (W1, W2: n x MAXRHS each), written as self-marking values over UNSET words;
+// a third such buffer and n values that the solves no longer use (the size is part of the interface); the
+// permutation, the abort word (at the passed work_bytes - 256, rounded down to an int: callers read it there) and 63
+// spare ints.
 template <typename T> size_t getrs_work(long n, long)
 {
     return sizeof(T) * (3 * (size_t)n * MAXRHS + (size_t)n) + sizeof(int) * ((size_t)n + 64);
 }
-
-template <typename T>
-int trsv_launch(hipStream_t s, int nb, const T *LU, long lda, long n, const T *rd, const T *src, long lds, T *dst,
-                int nrhs, int kind, int *abort)
+template <typename T> struct RsWork {
+    T *W1, *W2;
+    int *perm;
+};
+template <typename T> __host__ __device__ inline RsWork<T> rs_carve(void *work, long n)
 {
-    const double tri = kind_fwd(kind) ? 0.5 * n * (n - 1) : 0.5 * n * (n + 1);
-    TimedLaunch tl(s, M25X_K_TRSV, dtype_of<T>(), (tri + 2.0 * n * nrhs) * sizeof(T), 8.0 * tri * nrhs);
-    if (nrhs <= 4)
-        hipLaunchKernelGGL((k_trsv<T, 4>), dim3(nb), dim3(TB), 0, s, LU, lda, n, rd, src, lds, dst, nrhs, kind, abort);
+    const size_t wn = (size_t)n * MAXRHS;
+    T *w = (T *)work;
+    return RsWork<T>{w, w + wn, (int *)(w + 3 * wn + n)};
+}
+
+// The solve with the buffers at buf (getrs_work(n) - 256 bytes) and the abort word given (not reset here).
+template <typename T>
+int getrs_noreset(const T *LU, long n, long lda, const int *ipiv, const int *perm, T *B, long ldb, int nrhs, int trans,
+                  char *buf, int *abort, hipStream_t s)
+{
+    trans = trans != 0;
+    const RsWork<T> w = rs_carve<T>(buf, n);
+    const int nb = (int)((n + SB - 1) / SB), nchain = (nrhs + CR - 1) / CR;
+    if (!perm) {
+        hipLaunchKernelGGL(k_perm, dim3(1), dim3(256), 0, s, ipiv, n, w.perm);
+        perm = w.perm;
+    }
+    const long words = (long)(nchain * CR * sizeof(T) / 8) * n;
+    hipLaunchKernelGGL(k_fill_unset, dim3(blocks(words, 256), 2), dim3(256), 0, s, (u64 *)w.W1,
+                       (long)((w.W2 - w.W1) * sizeof(T) / 8), words);
+    if (int rc = check_launch("getrs")) return rc;
+    TimedLaunch tl(s, M25X_K_TRSV, dtype_of<T>(), ((double)n * n + 4.0 * n * nrhs) * sizeof(T), 8.0 * n * n * nrhs);
+    const dim3 grid(2 * chain_wgs(nb, nchain));
+    if (trans)
+        hipLaunchKernelGGL((k_trsv<T, true>), grid, dim3(TB), 0, s, LU, lda, n, B, ldb, perm, w.W1, w.W2, nrhs, abort);
     else
-        hipLaunchKernelGGL((k_trsv<T, TrsvMaxRhs<T>::NR>), dim3(nb), dim3(TB), 0, s, LU, lda, n, rd, src, lds, dst,
-                           nrhs, kind, abort);
+        hipLaunchKernelGGL((k_trsv<T, false>), grid, dim3(TB), 0, s, LU, lda, n, B, ldb, perm, w.W1, w.W2, nrhs, abort);
     return check_launch("getrs/trsv");
 }
 
-// One solve of at most TrsvMaxRhs<T>::NR right-hand sides; the abort word is the caller's (zeroed once per call).
-template <typename T>
-int getrs_part(const T *LU, long n, long lda, const int *perm_in, T *B, long ldb, int nrhs, int trans, T *W1, T *W2,
-               T *W0, const T *rd, int *abort, hipStream_t s)
-{
-    const int nb = (int)((n + SB - 1) / SB);
-    const size_t wn = (size_t)n * MAXRHS;
-    const long words = (long)(2 * wn * sizeof(T) / 8);
-    hipLaunchKernelGGL(k_fill_unset, dim3(blocks(words, 256)), dim3(256), 0, s, (unsigned long long *)W1, words);
-    if (int rc = check_launch("getrs")) return rc;
-    const unsigned pg = blocks(n * nrhs, 256);
-    int rc;
-    if (trans) {
-        if ((rc = trsv_launch<T>(s, nb, LU, lda, n, rd, B, ldb, W1, nrhs, 0, abort))) return rc;
-        if ((rc = trsv_launch<T>(s, nb, LU, lda, n, rd, W1, nrhs, W2, nrhs, 1, abort))) return rc;
-        hipLaunchKernelGGL(k_permute<T>, dim3(pg), dim3(256), 0, s, (const T *)W2, (long)nrhs, B, ldb, n, nrhs, perm_in, 1);
-    } else {
-        hipLaunchKernelGGL(k_permute<T>, dim3(pg), dim3(256), 0, s, (const T *)B, ldb, W0, (long)nrhs, n, nrhs, perm_in, 0);
-        if ((rc = trsv_launch<T>(s, nb, LU, lda, n, rd, W0, nrhs, W1, nrhs, 2, abort))) return rc;
-        if ((rc = trsv_launch<T>(s, nb, LU, lda, n, rd, W1, nrhs, W2, nrhs, 3, abort))) return rc;
-        hipLaunchKernelGGL(k_permute<T>, dim3(pg), dim3(256), 0, s, (const T *)W2, (long)nrhs, B, ldb, n, nrhs,
-                           (const int *)nullptr, 0);
-    }
-    return check_launch("getrs");
-}
-
-// The solve with the buffers at buf (getrs_work(n) - 256 bytes: W1, W2, W0, 1 / U_ii, the permutation) and the
-// abort word given (not reset here): in parts of at most TrsvMaxRhs<T>::NR right-hand sides.
-template <typename T>
-int getrs_noreset(const T *LU, long n, long lda, const int *ipiv, const int *perm_in, T *B, long ldb, int nrhs,
-                  int trans, char *buf, int *abort, hipStream_t s)
-{
-    const size_t wn = (size_t)n * MAXRHS;
-    T *W1 = (T *)buf, *W2 = W1 + wn, *W0 = W2 + wn, *rd = W0 + wn;
-    int *perm = (int *)(rd + n);
-    hipLaunchKernelGGL(k_rdiag<T>, dim3(blocks(n, 256)), dim3(256), 0, s, LU, lda, n, rd);
-    if (!perm_in) {
-        hipLaunchKernelGGL(k_perm, dim3(1), dim3(256), 0, s, ipiv, n, perm);
-        perm_in = perm;
-    }
-    if (int rc = check_launch("getrs")) return rc;
-    for (int c0 = 0; c0 < nrhs; c0 += TrsvMaxRhs<T>::NR) {
-        const int kc = std::min(TrsvMaxRhs<T>::NR, nrhs - c0);
-        if (int rc = getrs_part<T>(LU, n, lda, perm_in, B + c0, ldb, kc, trans, W1, W2, W0, rd, abort, s)) return rc;
-    }
-    return M25X_OK;
-}
-
-// The solve: buffers carved from `work` (W1, W2, W0: n x MAXRHS each; 1 / U_ii; the permutation), the abort word
-// at work + wbytes - 256 (rounded down to an int), zeroed once here and raised by any part whose wait ran out.
-// More right-hand sides than the solve kernel holds are solved in parts that share the word.
+// The solve: buffers carved from `work`, the abort word at work + wbytes - 256 (rounded down to an int), zeroed once
+// here and raised by any chain whose wait ran out.
 template <typename T>
 int getrs_t(const T *LU, long n, long lda, const int *ipiv, const int *perm_in, T *B, long ldb, int nrhs, int trans,
             void *work, size_t wbytes, hipStream_t s)
@@ -1357,79 +1710,35 @@ int getrf_batched_t(int nitems, const m25x_lu_item *h, const m25x_lu_item *d, hi
     return M25X_OK;
 }
 
-// the solve's buffers in an item's workspace (as getrs_noreset carves them)
-template <typename T> struct RsWork {
-    T *W1, *W2, *W0, *rd;
-};
-template <typename T> __device__ inline RsWork<T> rs_carve(void *work, long n)
-{
-    RsWork<T> w;
-    const size_t wn = (size_t)n * MAXRHS;
-    w.W1 = (T *)work;
-    w.W2 = w.W1 + wn;
-    w.W0 = w.W2 + wn;
-    w.rd = w.W0 + wn;
-    return w;
-}
-
-// W1, W2 filled with UNSET words; with rdiag, 1 / U_ii too
+// W1, W2 of every item filled with UNSET words
 template <typename T>
-__global__ void k_rs_prep_b(const m25x_rs_item *items, int c0, int rdiag)
+__global__ void k_rs_prep_b(const m25x_rs_item *items)
 {
     const m25x_rs_item it = items[blockIdx.y];
-    if (c0 >= it.nrhs) return;
     const RsWork<T> w = rs_carve<T>(it.work, it.n);
-    const long words = (long)(2 * (size_t)it.n * MAXRHS * sizeof(T) / 8);
+    const long words = (long)((it.nrhs + CR - 1) / CR * CR * sizeof(T) / 8) * it.n;
     const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (i < words) ((unsigned long long *)w.W1)[i] = ~0ull;
-    if (rdiag && i < it.n) {
-        const T *LU = (const T *)it.LU;
-        w.rd[i] = trecip(LU[i * it.lda + i]);
-    }
+    if (i < words) ((u64 *)w.W1)[i] = ((u64 *)w.W2)[i] = UNSET;
 }
 
-// the right-hand sides of part c0 in or out through the permutation: mode 0 B -> W0 gathered by perm (trans 0),
-// mode 1 W2 -> B scattered by perm (trans 1), mode 2 W2 -> B as is (trans 0)
-template <typename T>
-__global__ void k_rs_move_b(const m25x_rs_item *items, int c0, int NR, int mode)
+// Both triangles of every item: workgroup g is workgroup g / nitems of item g % nitems (the chains side by side; a
+// workgroup waits only on workgroups of its own item before it, which have smaller g). nb, nchain: the most blocks and
+// chains of an item.
+template <typename T, bool RM>
+__global__ __launch_bounds__(TB) void k_trsv_b(const m25x_rs_item *items, int nitems, int nb, int nchain, int *abort)
 {
-    const m25x_rs_item it = items[blockIdx.y];
-    if (c0 >= it.nrhs) return;
-    const int kc = std::min(NR, it.nrhs - c0);
-    const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (idx >= it.n * kc) return;
-    const long i = idx / kc;
-    const int r = (int)(idx % kc);
+    const m25x_rs_item it = items[blockIdx.x % nitems];
+    const ChainPos at = chain_pos(blockIdx.x / nitems, nb, nchain);
+    if (at.chain * CR >= it.nrhs) return;
     const RsWork<T> w = rs_carve<T>(it.work, it.n);
-    T *B = (T *)it.B + c0;
-    if (mode == 0) w.W0[i * kc + r] = B[(long)it.perm[i] * it.ldb + r];
-    else if (mode == 1) B[(long)it.perm[i] * it.ldb + r] = w.W2[i * kc + r];
-    else B[i * it.ldb + r] = w.W2[i * kc + r];
-}
-
-// one triangle of every item's part c0: workgroup g is block g / nitems of item g % nitems (the chains side by
-// side; a workgroup waits only on blocks of its own item with smaller indices, which have smaller g)
-template <typename T, int NR>
-__global__ __launch_bounds__(TB) void k_trsv_b(const m25x_rs_item *items, int nitems, int c0, int kind, int *abort)
-{
-    const int item = blockIdx.x % nitems, q = blockIdx.x / nitems;
-    const m25x_rs_item it = items[item];
-    if (c0 >= it.nrhs || q >= (int)((it.n + SB - 1) / SB)) return;
-    const int kc = std::min(NR, it.nrhs - c0);
-    const RsWork<T> w = rs_carve<T>(it.work, it.n);
-    const T *src;
-    long lds;
-    T *dst;
-    if (kind == 0) { src = (const T *)it.B + c0; lds = it.ldb; dst = w.W1; }
-    else if (kind == 2) { src = w.W0; lds = kc; dst = w.W1; }
-    else { src = w.W1; lds = kc; dst = w.W2; }
-    trsv_body<T, NR>((const T *)it.LU, it.lda, it.n, w.rd, src, lds, dst, kc, kind, abort, q);
+    chain_of<RM>(chain_args((const T *)it.LU, it.lda, it.n, (T *)it.B, it.ldb, it.perm, w.W1, w.W2, it.nrhs, (int)RM, at,
+                            abort), at.q);
 }
 
 template <typename T>
 int getrs_batched_t(int nitems, const m25x_rs_item *h, const m25x_rs_item *d, int trans, int *status, hipStream_t s)
 {
-    constexpr int NR = TrsvMaxRhs<T>::NR;
+    trans = trans != 0;
     long nmax = 0;
     int rmax = 0, nbmax = 0;
     for (int i = 0; i < nitems; ++i) {
@@ -1448,36 +1757,20 @@ int getrs_batched_t(int nitems, const m25x_rs_item *h, const m25x_rs_item *d, in
     hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, status, 1);
     if (int rc = check_launch("getrs_batched")) return rc;
     if (nitems == 0 || nmax == 0) return M25X_OK;
-    const long words = (long)(2 * (size_t)nmax * MAXRHS * sizeof(T) / 8);
-    const int dt = dtype_of<T>();
-    for (int c0 = 0; c0 < rmax; c0 += NR) {
-        hipLaunchKernelGGL(k_rs_prep_b<T>, dim3(blocks(std::max(words, nmax), 256), nitems), dim3(256), 0, s, d, c0,
-                           (int)(c0 == 0));
-        const dim3 mg(blocks(nmax * std::min(NR, rmax - c0), 256), nitems);
-        if (!trans) hipLaunchKernelGGL(k_rs_move_b<T>, mg, dim3(256), 0, s, d, c0, NR, 0);
-        if (int rc = check_launch("getrs_batched")) return rc;
-        const int kmax = std::min(NR, rmax - c0);
-        for (int pass = 0; pass < 2; ++pass) {
-            const int kind = trans ? pass : 2 + pass;
-            double bytes = 0, flops = 0;
-            for (int i = 0; i < nitems; ++i)
-                if (c0 < h[i].nrhs) {
-                    const double n = h[i].n, tri = kind_fwd(kind) ? 0.5 * n * (n - 1) : 0.5 * n * (n + 1);
-                    const int kc = std::min(NR, h[i].nrhs - c0);
-                    bytes += (tri + 2.0 * n * kc) * sizeof(T);
-                    flops += 8.0 * tri * kc;
-                }
-            TimedLaunch tl(s, M25X_K_TRSV, dt, bytes, flops);
-            if (kmax <= 4)
-                hipLaunchKernelGGL((k_trsv_b<T, 4>), dim3(nbmax * nitems), dim3(TB), 0, s, d, nitems, c0, kind, status);
-            else
-                hipLaunchKernelGGL((k_trsv_b<T, NR>), dim3(nbmax * nitems), dim3(TB), 0, s, d, nitems, c0, kind, status);
-            if (int rc = check_launch("getrs_batched/trsv")) return rc;
-        }
-        hipLaunchKernelGGL(k_rs_move_b<T>, mg, dim3(256), 0, s, d, c0, NR, trans ? 1 : 2);
-        if (int rc = check_launch("getrs_batched")) return rc;
+    const int nchain = (rmax + CR - 1) / CR, dt = dtype_of<T>();
+    hipLaunchKernelGGL(k_rs_prep_b<T>, dim3(blocks((long)(nchain * CR * sizeof(T) / 8) * nmax, 256), nitems), dim3(256), 0,
+                       s, d);
+    if (int rc = check_launch("getrs_batched")) return rc;
+    double bytes = 0, flops = 0;
+    for (int i = 0; i < nitems; ++i) {
+        bytes += ((double)h[i].n * h[i].n + 4.0 * h[i].n * h[i].nrhs) * sizeof(T);
+        flops += 8.0 * h[i].n * h[i].n * h[i].nrhs;
     }
-    return M25X_OK;
+    TimedLaunch tl(s, M25X_K_TRSV, dt, bytes, flops);
+    const dim3 grid(2 * chain_wgs(nbmax, nchain) * nitems);
+    if (trans) hipLaunchKernelGGL((k_trsv_b<T, true>), grid, dim3(TB), 0, s, d, nitems, nbmax, nchain, status);
+    else hipLaunchKernelGGL((k_trsv_b<T, false>), grid, dim3(TB), 0, s, d, nitems, nbmax, nchain, status);
+    return check_launch("getrs_batched/trsv");
 }
 
 // ---- the solve without allocation ------------------------------------------------------------------------
@@ -1514,7 +1807,7 @@ int getrs_noalloc_t(const T *LU, long n, long lda, const int *ipiv, const int *p
 {
     if (nrhs < 1 || nrhs > MAXRHS) return fail(M25X_EINVAL, "getrs_noalloc: 1 to %d right-hand sides, not %d", MAXRHS, nrhs);
     if (ldb < nrhs) return fail(M25X_EINVAL, "getrs_noalloc: ldb < nrhs");
-    // the buffers getrs_noreset carves (W1, W2, W0, 1 / U_ii, the permutation): getrs_work less its 256-byte tail
+    // the buffers getrs_noreset carves: getrs_work less its 256-byte tail
     const size_t need = getrs_work<T>(n, ldb) - 256;
     if (need > (size_t)M25X_GETRS_SCRATCH_BYTES)
         return fail(M25X_EINVAL, "getrs_noalloc: n = %ld needs %zu bytes of workspace, more than the %u held per device",
