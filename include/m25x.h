@@ -266,10 +266,12 @@ int m25x_getrs_noalloc(int dtype, const void *LU, long n, long lda, const int *i
 int m25x_lu_set_gemm_stage(int ks);
 int m25x_lu_gemm_stage(void);
 
-/* Look-ahead of the tournament LU (m25x_getrf, one matrix), 1 on, 0 off (the default): the next panel's tournament
- * runs on a second stream of the library's (one per device, the default priority) beside the rest of the trailing
- * update on the caller's stream. The factor is the same bit for bit either way (the same kernels; each update
- * split by columns). No counterpart in the reference (its LU is LAPACK's or a vendor library's). */
+/* Look-ahead of the tournament LU (m25x_getrf, one matrix), 1 on (the default), 0 off: for large matrices the next
+ * panel's columns are updated first and its tournament runs on the caller's stream beside the rest of the trailing
+ * update on a stream of the library's (at most four per device, the default priority, one call at a time on each; the
+ * caller's stream waits for it before the call's last kernels, and a call on a stream that is being captured uses the
+ * caller's stream alone). The factor is the same bit for bit either way (the same kernels; each update split by
+ * columns). No counterpart in the reference (its LU is LAPACK's or a vendor library's). */
 int m25x_lu_set_lookahead(int on);
 int m25x_lu_lookahead(void);
 

@@ -1385,33 +1385,86 @@ int getrf_t(T *A, long n, long lda, int *ipiv, int *info, void *work, size_t wby
 
 // ---- look-ahead: the next panel's tournament beside the trailing update -----------------------------------
 // The tournament of panel j + 1 needs only panel j + 1's columns updated, so the update of step j is split: the next
-// panel's 64 columns first, then the rest, and the tournament runs on a second stream beside the rest (its waves
-// raise their own issue priority on the SIMDs they share with the update, s_setprio; both streams keep the default
-// queue priority). Off by default (m25x_lu_set_lookahead): one extra stream per device, created once.
-std::atomic<int> g_lookahead{0};
+// panel's 64 columns first, on the caller's stream, with the tournament right behind them, and the rest on a side stream
+// that waits for those columns. A tournament workgroup takes all registers of a CU, so it can start only on an empty
+// one: in this order its workgroups are there before the rest of the update is let go. (The other way round, the
+// tournament on the side stream, it waits for the update's thousands of workgroups to drain and nothing is gained.)
+// N = 7799: complex64 43.3 -> 36.5 ms, complex128 58.7 -> 49.3; N = 14 000, complex64: 139 -> 120 ms. Beside the update
+// a tournament takes 1.5 to 1.7 times as long (the clock falls to 2.2 GHz, 1.95 for complex128, and its 53 KB of code
+// share an instruction cache with the update on the CU next to it) and the update 1.2 times.
+// On by default (m25x_lu_set_lookahead).
+std::atomic<int> g_lookahead{1};
 
-struct LookAhead {
-    hipStream_t p = nullptr;                  // the panel stream; the update runs on the caller's
-    hipEvent_t ev[4] = {};
-    bool ok = false;
+// A side stream and its events, leased to one call at a time (what a call has enqueued keeps its order on the stream
+// when the next lease goes on). At most MAX_SIDE a device, made as calls need them and kept.
+struct Side {
+    hipStream_t s = nullptr;
+    hipEvent_t next = nullptr, done = nullptr;
+};
+constexpr int MAX_SIDE = 4, SIDE_DEVICES = 64;
+struct SidePool {
+    std::mutex mu;
+    Side side[MAX_SIDE];
+    int made = 0;
+    unsigned busy = 0;
+};
+SidePool side_pool[SIDE_DEVICES];
+
+class SideLease {
+public:
+    // For work on `caller`; empty (use one stream) if not wanted, look-ahead is off, the caller's stream is being captured (a leased
+    // stream would stay part of the capture after the call), or none is free or can be made.
+    SideLease(hipStream_t caller, bool wanted)
+    {
+        int dev = -1;
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (!wanted || !g_lookahead.load(std::memory_order_relaxed)) return;
+        if (hipStreamIsCapturing(caller, &st) != hipSuccess || st != hipStreamCaptureStatusNone ||
+            hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= SIDE_DEVICES) {
+            (void)hipGetLastError();
+            return;
+        }
+        SidePool &p = side_pool[dev];
+        std::lock_guard<std::mutex> lk(p.mu);
+        for (int i = 0; i < MAX_SIDE; ++i) {
+            if (p.busy >> i & 1) continue;
+            if (i >= p.made) {
+                Side n;
+                if (hipStreamCreateWithFlags(&n.s, hipStreamNonBlocking) != hipSuccess ||
+                    hipEventCreateWithFlags(&n.next, hipEventDisableTiming) != hipSuccess ||
+                    hipEventCreateWithFlags(&n.done, hipEventDisableTiming) != hipSuccess) {
+                    (void)hipGetLastError();
+                    if (n.next) (void)hipEventDestroy(n.next);
+                    if (n.s) (void)hipStreamDestroy(n.s);
+                    return;
+                }
+                p.side[i] = n;
+                p.made = i + 1;
+            }
+            p.busy |= 1u << i;
+            pool = &p;
+            index = i;
+            return;
+        }
+    }
+    ~SideLease()
+    {
+        if (!pool) return;
+        std::lock_guard<std::mutex> lk(pool->mu);
+        pool->busy &= ~(1u << index);
+    }
+    SideLease(const SideLease &) = delete;
+    SideLease &operator=(const SideLease &) = delete;
+    const Side *get() const { return pool ? &pool->side[index] : nullptr; }
+
+private:
+    SidePool *pool = nullptr;
+    int index = 0;
 };
 
-LookAhead *lookahead_streams()
-{
-    static std::mutex mu;
-    static LookAhead la[64];
-    int dev = 0;
-    if (!g_lookahead.load(std::memory_order_relaxed) || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
-        return nullptr;
-    std::lock_guard<std::mutex> lk(mu);
-    LookAhead &L = la[dev];
-    if (L.ok) return &L;
-    if (hipStreamCreateWithFlags(&L.p, hipStreamNonBlocking) != hipSuccess) return nullptr;
-    for (auto &e : L.ev)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return nullptr;
-    L.ok = true;
-    return &L;
-}
+// From this many trailing rows on a step's update is split: below it the update is hardly longer than what the split
+// costs (the extra launch and two events, about 25 us; at 2500 rows 7.48 ms without and 7.38 with it).
+constexpr long LOOK_ROWS = 2048;
 
 template <typename T> size_t tour_work_bytes(long n)
 {
@@ -1424,60 +1477,6 @@ template <typename T> void launch_tri(hipStream_t s, T *A, long lda, long j0, lo
 {
     TimedLaunch tl(s, M25X_K_L21, dtype_of<T>(), 4.0 * sizeof(T) * m * TW, 8.0 * m * TW * TW);
     hipLaunchKernelGGL(k_tri<T>, dim3(2 * blocks(m, TRI_N)), dim3(256), 0, s, A, lda, j0, m, top);
-}
-
-// The tournament LU with one panel of look-ahead (see LookAhead): the same kernels and arithmetic as the plain loop
-// (each trailing update split by columns into two launches), so the factor is the same bit for bit. The caller's
-// stream runs the row moves, L21, U12 and the update, stream p the tournaments; events order them.
-template <typename T>
-int getrf_tp_lookahead(T *A, long n, long lda, int *ipiv, int *perm, int *info, TNode<T> *nodes, int *arrive, T *top,
-                       int *pairs, LookAhead &la, hipStream_t s)
-{
-    constexpr int RL = Tour<T>::RL;
-    const int dt = dtype_of<T>();
-    const double es = sizeof(T);
-    hipStream_t g = s, p = la.p;
-    hipEvent_t start = la.ev[0], panel = la.ev[1], next = la.ev[2], done = la.ev[3];
-    if (hipEventRecord(start, s) != hipSuccess || hipStreamWaitEvent(p, start, 0) != hipSuccess)
-        return fail(M25X_EHIP, "getrf: look-ahead stream");
-    auto tournament = [&](long j0) -> int {
-        const int jb = (int)std::min((long)TW, n - j0);
-        const long m = n - j0;
-        TimedLaunch tl(p, M25X_K_TSLU, dt, es * m * jb, 0.0);
-        if (int rc = launch_tslu((const T *)A, lda, n, j0, jb, (int)tour_leaves(m, RL), nodes, arrive, top, ipiv, pairs,
-                                 info, p))
-            return rc;
-        return hipEventRecord(panel, p) == hipSuccess ? M25X_OK : fail(M25X_EHIP, "getrf: event");
-    };
-    auto update = [&](long j0, int jb, long c0, long c1, long c2) {       // A22[c0:, c1:c2] -= L21 U12[:, c1:c2]
-        const long M = n - c0, N = c2 - c1;
-        TimedLaunch tl(g, M25X_K_GEMM, dt, es * (2.0 * M * N + (M + N) * jb), 8.0 * M * N * jb);
-        launch_update<T>(g, A + c1 * lda + c0, lda,
-                         (const T *)(A + j0 * lda + c0), lda, (const T *)(A + c1 * lda + j0), lda, M, N, (long)jb);
-    };
-    if (int rc = tournament(0)) return rc;
-    for (long j0 = 0; j0 < n; j0 += TW) {
-        const int jb = (int)std::min((long)TW, n - j0);
-        if (hipStreamWaitEvent(g, panel, 0) != hipSuccess) return fail(M25X_EHIP, "getrf: wait");
-        {
-            TimedLaunch tl(g, M25X_K_APPLY_MOVES, dt, 2.0 * es * 2 * jb * n, 0.0);
-            hipLaunchKernelGGL(k_apply_moves<T>, dim3(blocks(n, 8) + (perm ? 1 : 0)), dim3(256), 0, g, A, lda, 0L, n,
-                               (const int *)pairs, j0, jb, (const T *)top, perm);
-        }
-        const long c0 = j0 + jb;
-        if (c0 < n) {
-            launch_tri(g, A, lda, j0, n - c0, (const T *)top);
-            const long c1 = std::min(n, c0 + TW);
-            update(j0, jb, c0, c0, c1);                                   // the next panel's columns
-            if (hipEventRecord(next, g) != hipSuccess || hipStreamWaitEvent(p, next, 0) != hipSuccess)
-                return fail(M25X_EHIP, "getrf: event");
-            if (int rc = tournament(c0)) return rc;                       // beside the rest of the update
-            if (c1 < n) update(j0, jb, c0, c1, n);
-        }
-        if (int rc = check_launch("getrf/look-ahead")) return rc;
-    }
-    (void)done;                               // the last panel's tournament was waited for on the caller's stream
-    return M25X_OK;
 }
 
 template <typename T>
@@ -1497,20 +1496,27 @@ int getrf_tp(T *A, long n, long lda, int *ipiv, int *perm, int *info, void *work
     if (info) hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, info, 1);
     if (perm) hipLaunchKernelGGL(k_iota, dim3(blocks(n, 256)), dim3(256), 0, s, perm, n);
     if (int rc = check_launch("getrf")) return rc;
-    if (n > 2 * TW)
-        if (LookAhead *la = lookahead_streams())
-            return getrf_tp_lookahead<T>(A, n, lda, ipiv, perm, info, nodes, arrive, top, pairs, *la, s);
-    for (long j0 = 0; j0 < n; j0 += TW) {
+    const SideLease lease(s, n - TW >= LOOK_ROWS);
+    const Side *side = lease.get();
+    const int dt = dtype_of<T>();
+    const double es = sizeof(T);
+    auto tournament = [&](long j0) -> int {
         const int jb = (int)std::min((long)TW, n - j0);
         const long m = n - j0;
-        const int P = (int)tour_leaves(m, RL);
-        const int dt = dtype_of<T>();
-        const double es = sizeof(T);
-        {
-            TimedLaunch tl(s, M25X_K_TSLU, dt, es * m * jb, 0.0);
-            if (int rc = launch_tslu((const T *)A, lda, n, j0, jb, P, nodes, arrive, top, ipiv, pairs, info, s))
-                return rc;
-        }
+        TimedLaunch tl(s, M25X_K_TSLU, dt, es * m * jb, 0.0);
+        return launch_tslu((const T *)A, lda, n, j0, jb, (int)tour_leaves(m, RL), nodes, arrive, top, ipiv, pairs, info, s);
+    };
+    auto update = [&](hipStream_t on, long j0, int jb, long c1, long c2) {      // A22[:, c1:c2] -= L21 U12[:, c1:c2]
+        const long c0 = j0 + jb, M = n - c0, N = c2 - c1;
+        TimedLaunch tl(on, M25X_K_GEMM, dt, es * (2.0 * M * N + (double)(M + N) * jb), 8.0 * M * N * jb);
+        launch_update<T>(on, A + c1 * lda + c0, lda, (const T *)(A + j0 * lda + c0), lda, (const T *)(A + c1 * lda + j0),
+                         lda, M, N, (long)jb);
+    };
+    if (int rc = tournament(0)) return rc;
+    bool beside = false;                     // the last update's rest runs on the side stream
+    for (long j0 = 0; j0 < n; j0 += TW) {
+        const int jb = (int)std::min((long)TW, n - j0);
+        if (beside && hipStreamWaitEvent(s, side->done, 0) != hipSuccess) return fail(M25X_EHIP, "getrf: wait");
         {
             TimedLaunch tl(s, M25X_K_APPLY_MOVES, dt, 2.0 * es * 2 * jb * n, 0.0);
             hipLaunchKernelGGL(k_apply_moves<T>, dim3(blocks(n, 8) + (perm ? 1 : 0)), dim3(256), 0, s, A, lda, 0L, n,
@@ -1518,13 +1524,20 @@ int getrf_tp(T *A, long n, long lda, int *ipiv, int *perm, int *info, void *work
         }
         if (int rc = check_launch("getrf/panel")) return rc;
         const long c0 = j0 + jb;
-        if (c0 < n) {   // L21 = A21 U11^-1 and U12 = L11^-1 A12, then A22 -= L21 U12
-            T *A12 = A + c0 * lda + j0;
-            launch_tri(s, A, lda, j0, n - c0, (const T *)top);
-            const long M = n - c0;
-            TimedLaunch tl(s, M25X_K_GEMM, dt, es * (2.0 * M * M + 2.0 * M * jb), 8.0 * M * M * jb);
-            launch_update<T>(s, A + c0 * lda + c0, lda, (const T *)(A + j0 * lda + c0),
-                             lda, (const T *)A12, lda, M, M, (long)jb);
+        if (c0 >= n) break;
+        launch_tri(s, A, lda, j0, n - c0, (const T *)top);   // L21 = A21 U11^-1 and U12 = L11^-1 A12
+        beside = side && n - c0 >= LOOK_ROWS;
+        if (beside) {
+            const long c1 = c0 + TW;
+            update(s, j0, jb, c0, c1);                       // the next panel's columns
+            if (hipEventRecord(side->next, s) != hipSuccess || hipStreamWaitEvent(side->s, side->next, 0) != hipSuccess)
+                return fail(M25X_EHIP, "getrf: look-ahead");
+            if (int rc = tournament(c0)) return rc;          // in place before the rest is let go
+            update(side->s, j0, jb, c1, n);
+            if (hipEventRecord(side->done, side->s) != hipSuccess) return fail(M25X_EHIP, "getrf: look-ahead");
+        } else {
+            update(s, j0, jb, c0, n);
+            if (int rc = tournament(c0)) return rc;
         }
         if (int rc = check_launch("getrf/update")) return rc;
     }
