@@ -183,6 +183,26 @@ int m25x_radial_table_sum(const double *px, const double *py, const double *W, l
 int m25x_hankel(const double *rho, int nr, const double *kr, int nk, const double *W, int ns, double *out,
                 void *stream);
 
+/* The same for several sets of distances at once, each over rows of W of its own: set q transforms rows
+ * [row, row + rows) of W (nrows x nk) at its `count` distances, the sets covering rho[0 .. nr) in order, into
+ * out + out (complex values; rows x count), every sum divided by scale. sets: on the host, at most M25X_HANKEL_SETS. */
+#define M25X_HANKEL_SETS 32
+typedef struct { int first, count, row, rows; long out; } m25x_hankel_set;
+int m25x_hankel_sets(const double *rho, int nr, const m25x_hankel_set *sets, int nsets, double scale, const double *kr,
+                     int nk, const double *W, int nrows, double *out, long nout, void *stream);
+
+/* Complex rows y (rows x nc) on a coarse grid to nfine points by a real operator given transposed (St: nc x nfine):
+ * out[row][i] = sum_j St[j][i] y[row][j]; pairs: out[row / 2][i][row % 2] instead. The spline of the radial tables
+ * (src/mom25d/via.py:111-123), whose action is linear in its data. */
+int m25x_resample(const double *St, int nc, int nfine, const double *y, int rows, int pairs, double *out, void *stream);
+
+/* The nodes kr and weights dk (complex128, device) of a Sommerfeld contour (src/mom25d/via.py:36-53): nq nodes x and
+ * weights wq (host, on [-1, 1]) a panel; `near` panels evenly from 0 to t1, lifted into Im kr > 0 by
+ * lift sin(pi t / t1); `far` panels of `step` from t1 on and one to K, real: (near + far + 1) nq nodes. */
+#define M25X_CONTOUR_NQ 8
+int m25x_contour(int nq, const double *x, const double *wq, int near, int far, double t1, double lift, double step, double K,
+                 double *kr, double *dk, void *stream);
+
 /* The spectra of nreq requests at the npts nodes of a Sommerfeld contour (kr, dk: npts complex128 nodes and
  * weights, device), each times kr dk (the Hankel weights of m25x_hankel): W (nrows x npts complex128, device), a
  * request's values in its output row(s). req_i / req_d: the requests on the device; req_i_host: the same ints on the
@@ -195,6 +215,24 @@ int m25x_spectra(const m25x_stack *st, double w, const double *kr, const double 
 /* G~_A and G~_q between interfaces o and s at one complex kr, on the host (synchronous): out = (Re G~_A, Im G~_A,
  * Re G~_q, Im G~_q). The extraction coefficients' single evaluations (src/mom25d/multilayer.py:279-282, 288-291). */
 int m25x_spectral_point(const m25x_stack *st, double w, double kr_re, double kr_im, int o, int s, double *out);
+
+/* What the via blocks need of a mesh's vias, device arrays (once per mesh): F the nF fan triangles and dF (nF x Nv)
+ * the fans' charge operator; per chain its axis (vx, vy) and span; per edge its triangles and +-l / A; pair (Nv x Nv):
+ * the entry of R for a pair of chains or -1; the near pairs' part of the fan moments: QF[fan_row, fan_col] +=
+ * qc[fan_sel]. */
+typedef struct {
+    int Ne, Nt, Nv, nF, nlayer, nfine;
+    long nfan;
+    const int *F, *span, *tp, *tm, *pair, *fan_sel, *fan_row, *fan_col;
+    const double *dF, *vx, *vy, *wp, *wm;
+} m25x_via;
+
+/* The via blocks B (Ne x Nv) and C (Nv x Nv) at w: QF (Nt x nF, m25x_fan_q's; corrected in place), the smooth kernels
+ * D (spans x layers, nfine each, step dr), the reactions R, the rest of C in C0; X: Nt x Nv values of workspace.
+ * (src/mom25d/sim.py:816-872) */
+int m25x_via_blocks(const m25x_via *v, const m25x_mesh *g, const m25x_quad *q, double w, double *QF, const double *qc,
+                    const double *D, double dr, const double *R, const double *C0, double *X, double *B, double *Cv,
+                    void *stream);
 
 /* J_n(z), complex z, n = 0, 1, 2, elementwise. Replaces bessel_jn_complex
  * (src/mom25d/core/mom25d_core.cpp:1510-1558). */

@@ -53,6 +53,20 @@ class Mesh(C.Structure):
                 ('cent', C.c_void_p), ('area', C.c_void_p), ('ta', C.c_void_p), ('tv', C.c_void_p)]
 
 
+class HankelSet(C.Structure):
+    _fields_ = [('first', C.c_int), ('count', C.c_int), ('row', C.c_int), ('rows', C.c_int), ('out', C.c_long)]
+
+
+HANKEL_SETS = 32
+
+
+class Via(C.Structure):
+    _fields_ = [('Ne', C.c_int), ('Nt', C.c_int), ('Nv', C.c_int), ('nF', C.c_int), ('nlayer', C.c_int),
+                ('nfine', C.c_int), ('nfan', C.c_long)] + \
+               [(k, C.c_void_p) for k in ('F', 'span', 'tp', 'tm', 'pair', 'fan_sel', 'fan_row', 'fan_col',
+                                          'dF', 'vx', 'vy', 'wp', 'wm')]
+
+
 class Quad(C.Structure):
     _fields_ = [('nodes', C.c_void_p), ('tris', C.c_void_p), ('P3', C.c_void_p), ('W3', C.c_void_p),
                 ('P6', C.c_void_p), ('W6', C.c_void_p)]
@@ -77,6 +91,10 @@ _SIGS = {
     'm25x_fan_q': ([P, P, P, I, P, P], I),
     'm25x_radial_table_sum': ([P, P, P, L, L, P, P, L, P, L, D, P, P], I),
     'm25x_hankel': ([P, I, P, I, P, I, P, P], I),
+    'm25x_hankel_sets': ([P, I, P, I, D, P, I, P, I, P, L, P], I),
+    'm25x_resample': ([P, I, I, P, I, I, P, P], I),
+    'm25x_contour': ([I, P, P, I, I, D, D, D, D, P, P, P], I),
+    'm25x_via_blocks': ([P, P, P, D, P, P, P, D, P, P, P, P, P, P], I),
     'm25x_bessel_jn_complex': ([I, P, L, P, P], I),
     'm25x_spectra': ([P, D, P, P, I, P, P, I, P, P, L, P], I),
     'm25x_spectral_point': ([P, D, D, D, I, I, P], I),

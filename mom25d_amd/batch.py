@@ -81,9 +81,9 @@ class SweepBatch:
         t0 = time.perf_counter()
         pts = self.points
         Zs, Z64s, ds, Bs, ks = [], [], [], [], []
-        # every point's host-side parts first (tables, moments, via blocks: these wait for the device), then every
-        # Z, equilibration and copy queued with nothing waiting, so the fills run back to back on the device
-        prep = [(sim.fast.prepare(f), torch.from_numpy(sim.excitation()).to(dv.device())) for sim, f in pts]
+        # every point's host-side parts first (tables, moments, via blocks), then every Z, equilibration and copy,
+        # with nothing waiting for the device
+        prep = [(sim.fast.prepare(f), dv.upload(np.asarray(sim.excitation(), np.complex128))[0]) for sim, f in pts]
         for (sim, f), (st, E) in zip(pts, prep):
             Z = sim.fast.assemble(st)
             d = dv.diag_scales(Z)

@@ -499,13 +499,24 @@ __global__ void k_bessel(int n, const double2 *z, long total, double2 *o)
 }
 
 // out[s, i] = sum_k J0(rho_i kr_k) W[s, k]: one workgroup per rho; the real nodes and the lifted ones summed
-// apart and added at the end, as the reference adds its two parts (via.py:97-101)
+// apart and added at the end, as the reference adds its two parts (via.py:97-101). Several sets of distances, each with
+// rows of its own, go in one launch (a set of 200 or 260 distances alone leaves the chip two thirds empty: a launch of one
+// took 53 us, three of them in one launch take 64).
 constexpr int HS = 4;
-__global__ __launch_bounds__(256) void k_hankel(const double *rho, int nr, const double2 *kr, int nk,
-                                                const double2 *W, int ns, double2 *out)
+struct HankelSets {
+    int n;
+    double scale;                               // the sums are divided by it
+    m25x_hankel_set set[M25X_HANKEL_SETS];
+};
+__global__ __launch_bounds__(256) void k_hankel(HankelSets hs, const double *rho, const double2 *kr, int nk,
+                                                const double2 *W, double2 *out)
 {
-    const int i = blockIdx.x;
-    const double r = rho[i];
+    int q = 0;
+    while (q + 1 < hs.n && (int)blockIdx.x >= hs.set[q + 1].first) ++q;
+    const int i = (int)blockIdx.x - hs.set[q].first, nr = hs.set[q].count, ns = hs.set[q].rows;
+    const double r = rho[blockIdx.x];
+    W += (size_t)hs.set[q].row * nk;
+    out += hs.set[q].out;
     __shared__ double2 red[2][HS][256];
     for (int s0 = 0; s0 < ns; s0 += HS) {
         double2 aR[HS], aC[HS];
@@ -538,9 +549,134 @@ __global__ __launch_bounds__(256) void k_hankel(const double *rho, int nr, const
             }
             __syncthreads();
         }
-        if (threadIdx.x < HS && s0 + (int)threadIdx.x < ns)
-            out[(size_t)(s0 + threadIdx.x) * nr + i] = cadd(red[0][threadIdx.x][0], red[1][threadIdx.x][0]);
+        if (threadIdx.x < HS && s0 + (int)threadIdx.x < ns) {
+            const double2 v = cadd(red[0][threadIdx.x][0], red[1][threadIdx.x][0]);
+            out[(size_t)(s0 + threadIdx.x) * nr + i] = make_double2(v.x / hs.scale, v.y / hs.scale);
+        }
         __syncthreads();
+    }
+}
+
+// ---- tables on the uniform grid ------------------------------------------------------------------------------
+// out[row][i] = sum_j S[i][j] y[row][j], S given transposed (nc x nfine) so that a wave's loads of it are whole lines;
+// a lane a fine point, RS rows a thread, a quarter of the nodes a wave whose loads are asked for
+// many at a time. 14 us with S in the caches, 28 without (a point finds it there no more), the rows' coarse values in LDS. pairs: rows 2 t and 2 t + 1 side by side per point
+// (the tables' A and Q). Reading S, 8192 x 260 doubles, bounds it; the library's two real products and the copies into
+// this layout took 60 us more.
+constexpr int RS = 4, RP = 64, RG = 4;       // rows a thread, points and node groups of a workgroup
+constexpr int RN = 512, RU = 22;             // coarse nodes in LDS at a time; loads of S in flight a thread
+__global__ __launch_bounds__(RP * RG) void k_resample(const double *St, int nc, int nfine, const double2 *y, int rows,
+                                                      int pairs, double2 *out)
+{
+    __shared__ double2 yl[RN * RS];             // [node][row]; the groups' sums at the end
+    const int lane = threadIdx.x % RP, g = threadIdx.x / RP;
+    const int i = blockIdx.x * RP + lane, r0 = blockIdx.y * RS, ic = i < nfine ? i : nfine - 1;
+    double2 acc[RS];
+#pragma unroll
+    for (int r = 0; r < RS; ++r) acc[r] = make_double2(0.0, 0.0);
+    for (int j0 = 0; j0 < nc; j0 += RN) {
+        const int nj = nc - j0 < RN ? nc - j0 : RN, per = (nj + RG - 1) / RG;
+        if (j0) __syncthreads();
+        for (int e = threadIdx.x; e < nj * RS; e += RP * RG) {
+            const int r = r0 + e / nj, j = e % nj;
+            yl[j * RS + e / nj] = y[(size_t)(r < rows ? r : rows - 1) * nc + j0 + j];
+        }
+        __syncthreads();
+        const int ja = g * per, jb = ja + per < nj ? ja + per : nj;
+        for (int j = ja; j < jb; j += RU) {
+            double w[RU];                       // the group's next entries of S, all asked for first
+#pragma unroll
+            for (int u = 0; u < RU; ++u) w[u] = St[(size_t)(j0 + (j + u < jb ? j + u : jb - 1)) * nfine + ic];
+#pragma unroll
+            for (int u = 0; u < RU; ++u) {
+                if (j + u >= jb) break;
+#pragma unroll
+                for (int r = 0; r < RS; ++r) acc[r] = cadd(acc[r], cscale(yl[(j + u) * RS + r], w[u]));
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RS; ++r) yl[(g * RS + r) * RP + lane] = acc[r];
+    __syncthreads();
+    const int row = r0 + g;                     // group g adds up row g
+    if (i >= nfine || row >= rows) return;
+    double2 v = yl[g * RP + lane];
+#pragma unroll
+    for (int h = 1; h < RG; ++h) v = cadd(v, yl[(h * RS + g) * RP + lane]);
+    out[pairs ? ((size_t)(row >> 1) * nfine + i) * 2 + (row & 1) : (size_t)row * nfine + i] = v;
+}
+static_assert(RG == RS && RG * RS * RP <= RN * RS, "a group per row, and room for the sums");
+
+// ---- via blocks ----------------------------------------------------------------------------------------------
+// QF += the near pairs' correction of the fan moments
+__global__ void k_fan_add(m25x_via v, const double2 *qc, double2 *QF)
+{
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i >= v.nfan) return;
+    double2 *o = QF + (size_t)v.fan_row[i] * v.nF + v.fan_col[i];
+    *o = cadd(*o, qc[v.fan_sel[i]]);
+}
+
+// X[t, n] = the potential of chain n on triangle t: its end charges' through the fan moments, and its smooth kernel
+// D(layer of t, span of n) over the triangle's six points
+__global__ void k_via_tri(m25x_via v, const int *lt, const double *P6, const double *W6, double w, const double2 *QF,
+                          const double2 *D, double dr, double2 *X)
+{
+    const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (idx >= (long)v.Nt * v.Nv) return;
+    const int t = (int)(idx / v.Nv), c = (int)(idx % v.Nv);
+    double2 pot = {0, 0}, acc = {0, 0};
+    for (int j = 0; j < v.nF; ++j) pot = cadd(pot, cscale(QF[(size_t)t * v.nF + j], v.dF[(size_t)j * v.Nv + c]));
+    const double2 *d = D + (size_t)(v.span[c] * v.nlayer + lt[t]) * v.nfine;
+    const double top = (double)v.nfine - 1.000001;
+    for (int q = 0; q < 6; ++q) {
+        const double rx = P6[(size_t)t * 12 + 2 * q] - v.vx[c], ry = P6[(size_t)t * 12 + 2 * q + 1] - v.vy[c];
+        double u = hypot(rx, ry) / dr;
+        if (!(u <= top)) u = top;
+        const long i = (long)u;
+        const double f = u - (double)i;
+        const double2 a = d[i], b = d[i + 1];
+        acc = cadd(acc, cscale(make_double2(a.x * (1.0 - f) + b.x * f, a.y * (1.0 - f) + b.y * f), W6[(size_t)t * 6 + q]));
+    }
+    X[idx] = make_double2(acc.x + pot.y / w, acc.y - pot.x / w);            // pot / (j w)
+}
+
+// B[e, n] = wp X[T+] + wm X[T-]
+__global__ void k_via_div(m25x_via v, const double2 *X, double2 *B)
+{
+    const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (idx >= (long)v.Ne * v.Nv) return;
+    const int e = (int)(idx / v.Nv), c = (int)(idx % v.Nv);
+    B[idx] = cadd(cscale(X[(size_t)v.tp[e] * v.Nv + c], v.wp[e]), cscale(X[(size_t)v.tm[e] * v.Nv + c], v.wm[e]));
+}
+
+// C[m, n] = C0[m, n] + R[pair(m, n)] + the end charges' part: a wave an entry, a lane a fan triangle (in turns)
+__global__ __launch_bounds__(64) void k_via_c(m25x_via v, double w, const double2 *QF, const double2 *R, const double2 *C0,
+                                              double2 *Cv)
+{
+    const int m = blockIdx.x / v.Nv, c = blockIdx.x % v.Nv;
+    double2 acc = {0, 0};
+    for (int i = threadIdx.x; i < v.nF; i += 64) {
+        const double dm = v.dF[(size_t)i * v.Nv + m];
+        if (dm == 0.0) continue;
+        double2 pot = {0, 0};
+        const double2 *q = QF + (size_t)v.F[i] * v.nF;
+        for (int j = 0; j < v.nF; ++j) pot = cadd(pot, cscale(q[j], v.dF[(size_t)j * v.Nv + c]));
+        acc = cadd(acc, cscale(pot, dm));
+    }
+    __shared__ double2 red[64];
+    red[threadIdx.x] = acc;
+    __syncthreads();
+    for (int st = 32; st > 0; st >>= 1) {
+        if ((int)threadIdx.x < st) red[threadIdx.x] = cadd(red[threadIdx.x], red[threadIdx.x + st]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const int p = v.pair[blockIdx.x];
+        double2 o = C0[blockIdx.x];
+        if (p >= 0) o = cadd(o, R[p]);
+        Cv[blockIdx.x] = make_double2(o.x + red[0].y / w, o.y - red[0].x / w);
     }
 }
 
@@ -1046,14 +1182,66 @@ int m25x_radial_table_sum(const double *px, const double *py, const double *W, l
     return check_launch("radial_table_sum");
 }
 
+int m25x_hankel_sets(const double *rho, int nr, const m25x_hankel_set *sets, int nsets, double scale, const double *kr,
+                     int nk, const double *W, int nrows, double *out, long nout, void *stream)
+{
+    if (nr < 0 || nk < 0 || nrows < 0 || nsets < 0 || nsets > M25X_HANKEL_SETS || (nsets && !sets))
+        return fail(M25X_EINVAL, "hankel: bad sizes (at most %d sets)", M25X_HANKEL_SETS);
+    HankelSets hs;
+    hs.n = nsets;
+    hs.scale = scale;
+    int at = 0;
+    for (int q = 0; q < nsets; ++q) {           // the sets cover the distances in order
+        const m25x_hankel_set &t = hs.set[q] = sets[q];
+        if (t.first != at || t.count < 0 || t.row < 0 || t.rows < 0 || t.row + t.rows > nrows || t.out < 0 ||
+            t.out + (long)t.rows * t.count > nout)
+            return fail(M25X_EINVAL, "hankel: set %d", q);
+        at += t.count;
+    }
+    if (at != nr) return fail(M25X_EINVAL, "hankel: the sets cover %d of %d distances", at, nr);
+    if (nr == 0) return M25X_OK;
+    hipLaunchKernelGGL(k_hankel, dim3(nr), dim3(256), 0, (hipStream_t)stream, hs, rho, (const double2 *)kr, nk,
+                       (const double2 *)W, (double2 *)out);
+    return check_launch("hankel");
+}
+
 int m25x_hankel(const double *rho, int nr, const double *kr, int nk, const double *W, int ns, double *out,
                 void *stream)
 {
     if (nr < 0 || nk < 0 || ns < 0) return fail(M25X_EINVAL, "hankel: bad sizes");
-    if ((long)nr * ns == 0) return M25X_OK;
-    hipLaunchKernelGGL(k_hankel, dim3(nr), dim3(256), 0, (hipStream_t)stream, rho, nr, (const double2 *)kr, nk,
-                       (const double2 *)W, ns, (double2 *)out);
-    return check_launch("hankel");
+    const m25x_hankel_set one = {0, nr, 0, ns, 0};
+    return m25x_hankel_sets(rho, nr, &one, 1, 1.0, kr, nk, W, ns, out, (long)nr * ns, stream);
+}
+
+int m25x_resample(const double *St, int nc, int nfine, const double *y, int rows, int pairs, double *out, void *stream)
+{
+    if (nc < 1 || nfine < 0 || rows < 0 || (pairs && rows % 2))
+        return fail(M25X_EINVAL, "resample: one node or more, an even number of rows for pairs");
+    if (rows == 0 || nfine == 0) return M25X_OK;
+    hipLaunchKernelGGL(k_resample, dim3(blocks(nfine, RP), blocks(rows, RS)), dim3(RP * RG), 0, (hipStream_t)stream,
+                       St, nc, nfine, (const double2 *)y, rows, pairs, (double2 *)out);
+    return check_launch("resample");
+}
+
+int m25x_via_blocks(const m25x_via *v, const m25x_mesh *g, const m25x_quad *q, double w, double *QF, const double *qc,
+                    const double *D, double dr, const double *R, const double *C0, double *X, double *B, double *Cv,
+                    void *stream)
+{
+    if (!v || !g || !q || v->Nv < 1 || v->Ne != g->Ne || v->Nt != g->Nt || v->nF < 0 || v->nfine < 2 || v->nfan < 0 ||
+        !(dr > 0) || !(w > 0))
+        return fail(M25X_EINVAL, "via_blocks: bad arguments");
+    hipStream_t s = (hipStream_t)stream;
+    if (v->nfan)
+        hipLaunchKernelGGL(k_fan_add, dim3(blocks(v->nfan, 256)), dim3(256), 0, s, *v, (const double2 *)qc, (double2 *)QF);
+    if (v->Nt)
+        hipLaunchKernelGGL(k_via_tri, dim3(blocks((long)v->Nt * v->Nv, 256)), dim3(256), 0, s, *v, g->lt, q->P6, q->W6, w,
+                           (const double2 *)QF, (const double2 *)D, dr, (double2 *)X);
+    if (v->Ne)
+        hipLaunchKernelGGL(k_via_div, dim3(blocks((long)v->Ne * v->Nv, 256)), dim3(256), 0, s, *v, (const double2 *)X,
+                           (double2 *)B);
+    hipLaunchKernelGGL(k_via_c, dim3(v->Nv * v->Nv), dim3(64), 0, s, *v, w, (const double2 *)QF, (const double2 *)R,
+                       (const double2 *)C0, (double2 *)Cv);
+    return check_launch("via_blocks");
 }
 
 int m25x_bessel_jn_complex(int n, const double *z, long total, double *out, void *stream)

@@ -220,6 +220,29 @@ __global__ __launch_bounds__(128) void k_spectra(m25x_stack st, double w, const 
     for (int q = 0; q < nout; ++q) W[(size_t)(row + q) * npts + node] = cmul(out[q], wt);
 }
 
+// The nodes and weights of a Sommerfeld contour: panel p of np lies between edges p and p + 1 (near + 1 edges evenly
+// from 0 to t1, then every step, the last at K), nq Gauss-Legendre nodes each, lifted below t1.
+struct Gauss {
+    double x[M25X_CONTOUR_NQ], w[M25X_CONTOUR_NQ];
+};
+__device__ inline double contour_edge(int e, int near, int far, double t1, double step, double K)
+{
+    return e < near ? e * (t1 / near) : e == near ? t1 : e <= near + far ? t1 + (e - near) * step : K;
+}
+__global__ void k_contour(Gauss gl, int nq, int near, int far, double t1, double lift, double step, double K, int npts,
+                          double2 *kr, double2 *dk)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= npts) return;
+    const int p = i / nq, q = i % nq;
+    const double lo = contour_edge(p, near, far, t1, step, K), hi = contour_edge(p + 1, near, far, t1, step, K);
+    const double half = 0.5 * (hi - lo), t = half * gl.x[q] + 0.5 * (lo + hi), wt = half * gl.w[q];
+    const double arc = M_PI * t / t1;
+    const bool on = t < t1;
+    kr[i] = make_double2(t, on ? lift * sin(arc) : 0.0);
+    dk[i] = make_double2(wt, wt * (on ? lift * M_PI / t1 * cos(arc) : 0.0));
+}
+
 int check_stack(const m25x_stack *st)
 {
     if (!st || st->N < 1 || st->N > ML) return fail(M25X_EINVAL, "spectra: 1 to %d layers", ML);
@@ -265,6 +288,22 @@ int m25x_spectra(const m25x_stack *st, double w, const double *kr, const double 
     hipLaunchKernelGGL(k_spectra, dim3((npts + 127) / 128, nreq), dim3(128), 0, (hipStream_t)stream, *st, w,
                        (const double2 *)kr, (const double2 *)dk, npts, req_i, req_d, (double2 *)W);
     return check_launch("spectra");
+}
+
+int m25x_contour(int nq, const double *x, const double *wq, int near, int far, double t1, double lift, double step, double K,
+                 double *kr, double *dk, void *stream)
+{
+    if (nq < 1 || nq > M25X_CONTOUR_NQ || !x || !wq || near < 1 || far < 0 || !(t1 > 0) || !kr || !dk)
+        return fail(M25X_EINVAL, "contour: bad arguments (1 to %d nodes a panel)", M25X_CONTOUR_NQ);
+    Gauss gl = {};
+    for (int q = 0; q < nq; ++q) {
+        gl.x[q] = x[q];
+        gl.w[q] = wq[q];
+    }
+    const int npts = (near + far + 1) * nq;
+    hipLaunchKernelGGL(k_contour, dim3((npts + 127) / 128), dim3(128), 0, (hipStream_t)stream, gl, nq, near, far, t1, lift,
+                       step, K, npts, (double2 *)kr, (double2 *)dk);
+    return check_launch("contour");
 }
 
 int m25x_spectral_point(const m25x_stack *st, double w, double kr_re, double kr_im, int o, int s, double *out)

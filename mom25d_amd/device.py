@@ -17,11 +17,17 @@ f64, i32, c128, c64 = torch.float64, torch.int32, torch.complex128, torch.comple
 
 def device():
     """The current HIP device (RuntimeError without one), initialised for the library."""
-    if not torch.cuda.is_available():
+    if not _DEVICES and not torch.cuda.is_available():
         raise RuntimeError("mom25d_amd: no GPU - the kernels are HIP (gfx950) only")
     idx = torch.cuda.current_device()
-    L.init(idx)
-    return torch.device('cuda', idx)
+    d = _DEVICES.get(idx)
+    if d is None:
+        L.init(idx)
+        d = _DEVICES[idx] = torch.device('cuda', idx)
+    return d
+
+
+_DEVICES = {}                            # the devices initialised so far
 
 
 def stream():
@@ -39,6 +45,27 @@ def on_dev(a, dtype):
     np_dt = {f64: np.float64, i32: np.int32, c128: np.complex128, c64: np.complex64,
              torch.int64: np.int64}[dtype]
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np_dt)).to(device())
+
+
+def upload(*arrays):
+    """Device copies of small NumPy arrays for kernels on the current stream, in one transfer that the host does not
+    wait for (through a pinned buffer, which is not used again before the transfer is done). For data of one call:
+    what is kept and read on other streams later goes through on_dev, which waits."""
+    arrays = [np.ascontiguousarray(a) for a in arrays]
+    at, n = [], 0
+    for a in arrays:
+        at.append(n)
+        n += -(-a.nbytes // 16) * 16
+    host = torch.empty(n, dtype=torch.uint8, pin_memory=True)
+    h = host.numpy()
+    for a, o in zip(arrays, at):
+        h[o:o + a.nbytes] = a.reshape(-1).view(np.uint8)
+    blob = host.to(device(), non_blocking=True)
+    return [blob[o:o + a.nbytes].view(_TORCH_DTYPE[a.dtype.char]).view(a.shape) for a, o in zip(arrays, at)]
+
+
+_TORCH_DTYPE = {np.dtype(a).char: b for a, b in ((np.float64, f64), (np.int32, i32), (np.complex128, c128),
+                                                 (np.int64, torch.int64))}
 
 
 def _cx_pairs(z):
@@ -76,11 +103,9 @@ class DevTables:
         real = np.concatenate([scal['dr'], scal['d'], scal['dimg']]).astype(np.float64)
         cplx = np.concatenate([scal[k] for k in ('cA', 'cq', 'cAi', 'cqi')]).astype(np.complex128)
         ints = np.concatenate([np.asarray(tab, np.int32).ravel(), np.asarray(kind, np.int32)])
-        blob = torch.from_numpy(np.concatenate([real, cplx.view(np.float64)])).to(dv)
-        t.dr, t.d, t.dimg = blob[:n], blob[n:2 * n], blob[2 * n:3 * n]
-        cx = blob[3 * n:].view(4, n, 2)
+        real, cx, iblob = upload(real, cplx.view(np.float64).reshape(4, n, 2), ints)
+        t.dr, t.d, t.dimg = real[:n], real[n:2 * n], real[2 * n:]
         t.cA, t.cq, t.cAi, t.cqi = cx[0], cx[1], cx[2], cx[3]
-        iblob = torch.from_numpy(ints).to(dv)
         t.L = int(np.asarray(tab).shape[0])
         t.tab, t.kind = iblob[:t.L * t.L].view(t.L, t.L), iblob[t.L * t.L:]
         t.sig = np.asarray(kind, np.int32).tobytes() + np.asarray(scal['dimg'], np.float64).tobytes() + \
@@ -330,6 +355,70 @@ def hankel_sum(rho, kr, W):
     out = torch.empty((W.shape[0], len(rho)), dtype=c128, device=device())
     L.call('m25x_hankel', ptr(rho), len(rho), ptr(kr), len(kr), ptr(W), W.shape[0], ptr(out), stream())
     return out
+
+
+def hankel_sets(rho, sets, kr, W, scale=1.0):
+    """Several Hankel sums in one launch: sets [(count, row, rows)] take the distances rho (device float64) in order,
+    each over rows [row, row + rows) of W; every sum divided by scale. Returns one (rows, count) tensor a set."""
+    sizes = [c * r for c, _, r in sets]
+    out = torch.empty(sum(sizes), dtype=c128, device=W.device)
+    views, pos, first, q0 = [], 0, 0, 0
+    tab = []
+    for (c, row, rows), size in zip(sets, sizes):
+        tab.append((first, c, row, rows, pos))
+        views.append(out[pos:pos + size].view(rows, c))
+        first, pos = first + c, pos + size
+    for q0 in range(0, len(tab), L.HANKEL_SETS):
+        part = tab[q0:q0 + L.HANKEL_SETS]
+        lo, hi = part[0][0], part[-1][0] + part[-1][1]
+        arr = (L.HankelSet * len(part))(*[(f - lo, c, row, rows, o) for f, c, row, rows, o in part])
+        L.call('m25x_hankel_sets', C.c_void_p(rho.data_ptr() + 8 * lo), hi - lo, arr, len(part), float(scale), ptr(kr),
+               len(kr), ptr(W), W.shape[0], ptr(out), out.numel(), stream())
+    return views
+
+
+def resample(St, y, pairs=False):
+    """The operator given transposed (St: nc x nfine float64) on complex rows y (rows, nc): (rows, nfine), or with
+    pairs (rows / 2, nfine, 2), two rows side by side per point."""
+    nc, nfine = St.shape
+    y = y.contiguous()
+    rows = y.shape[0]
+    out = torch.empty((rows // 2, nfine, 2) if pairs else (rows, nfine), dtype=c128, device=y.device)
+    L.call('m25x_resample', ptr(St), nc, nfine, ptr(y), rows, int(pairs), ptr(out), stream())
+    return out
+
+
+def via_blocks(via, mesh, w, QF, qc, D, dr, R, C0):
+    """(B, C) of the vias (m25x_via_blocks): via a DevVia, D (spans x layers, nfine), R and C0 complex128."""
+    Ne, Nt, Nv = mesh.Ne, mesh.Nt, via.Nv
+    X = torch.empty((Nt, Nv), dtype=c128, device=D.device)
+    B = torch.empty((Ne, Nv), dtype=c128, device=D.device)
+    Cv = torch.empty((Nv, Nv), dtype=c128, device=D.device)
+    if D.shape != (via.nspan * via.struct.nlayer, via.struct.nfine) or C0.shape != Cv.shape or \
+            QF.shape != (Nt, via.struct.nF) or R.numel() != via.npair or not (QF.is_contiguous() and D.is_contiguous()):
+        raise ValueError("via_blocks: the tables, fan moments or reactions do not fit the vias")
+    L.call('m25x_via_blocks', C.byref(via.struct), C.byref(mesh.struct), C.byref(mesh.quad), float(w), ptr(QF), ptr(qc),
+           ptr(D), float(dr), ptr(R), ptr(C0), ptr(X), ptr(B), ptr(Cv), stream())
+    return B, Cv
+
+
+class DevVia:
+    """The vias' fixed arrays on the device (m25x_via), once per mesh: F (nF,) fan triangles, dF (nF, Nv), the chains'
+    axes x, y and span indices, the edges' triangles tp, tm with their +-l / A (wp, wm), pair (Nv, Nv) into the
+    reactions (npair of them), and the near pairs' part of the fan moments (sel, row, col)."""
+
+    def __init__(self, mesh, nlayer, nfine, F, dF, x, y, span, nspan, tp, tm, wp, wm, pair, npair, fan):
+        sel, row, col = fan
+        self.Nv, self.nspan, self.npair = len(x), nspan, npair
+        keep = dict(F=on_dev(F, i32), dF=on_dev(dF, f64), vx=on_dev(x, f64), vy=on_dev(y, f64), span=on_dev(span, i32),
+                    tp=on_dev(tp, i32), tm=on_dev(tm, i32), wp=on_dev(wp, f64), wm=on_dev(wm, f64),
+                    pair=on_dev(pair, i32), fan_sel=on_dev(sel, i32), fan_row=on_dev(row, i32), fan_col=on_dev(col, i32))
+        s = L.Via()
+        s.Ne, s.Nt, s.Nv, s.nF, s.nfan = mesh.Ne, mesh.Nt, self.Nv, len(F), len(sel)
+        s.nlayer, s.nfine = nlayer, nfine
+        for k, t in keep.items():
+            setattr(s, k, t.data_ptr())
+        self._keep, self.struct = keep, s
 
 
 def bessel_jn_complex(n, z):

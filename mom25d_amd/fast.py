@@ -60,44 +60,51 @@ class FastOperator:
         sim.log.note(f"fast solver: {self.plan.n} near triangle pairs ({self.plan.n / max(1, len(sim.tri_size)):.0f} "
                      f"per triangle), {self.plan.nentry} near entries")
         F = sim.F
-        self._fan = None
+        self._fan, self.fan_pairs = None, (np.zeros(0, int),) * 3
         if len(F):
             dev = dv.device()
             pos = -np.ones(len(sim.tri_size), np.int64)
             pos[F] = np.arange(len(F))
             Pn, Qn = self.plan.P.long().cpu().numpy(), self.plan.Q.long().cpu().numpy()
             sel = np.flatnonzero(pos[Qn] >= 0)
+            self.fan_pairs = sel, Pn[sel], pos[Qn[sel]]
             self._fan = (torch.from_numpy(sel).to(dev), torch.from_numpy(Pn[sel]).to(dev),
                          torch.from_numpy(pos[Qn[sel]]).to(dev))
 
     # ---- set-up and fill ------------------------------------------------------------------------------------
     def setup(self, f):
+        """The frequency's tables; the via kernels made with them, if any (sim.point_tables)."""
         self.f, self.w = f, 2 * np.pi * f
-        self.sim.green_tables(f)
+        kernels = self.sim.point_tables(f)
         self.tabs = self.sim.dev_tables
+        return kernels
 
     def prepare(self, f):
-        """The per-frequency parts of Z that involve the host, computed before any N x N work is queued: the
-        Green's tables, the near pairs' moments, the via blocks B and C (their small dense parts are assembled on
-        the host, which waits for the device there) and the lumped entries, uploaded. Returns the point's state for
-        assemble(); holding it keeps its tables alive, so many points can be prepared before any is assembled."""
+        """The per-frequency parts of Z that involve the host, queued before any N x N work: the Green's tables, the
+        near pairs' moments, the via blocks B and C and the lumped entries. Nothing waits for the device (except
+        where reactions of many chain pairs go through a table). Returns the point's state for assemble(); holding
+        it keeps its tables alive, so many points can be prepared before any is assembled."""
         sim, w = self.sim, 2 * np.pi * f
-        self.setup(f)
-        tabs, dev = self.tabs, dv.device()
+        kernels = self.setup(f)
+        tabs = self.tabs
         with sim.log.timer('near-field moments'):
             M, qc = dv.near_moments(self.mesh, tabs, self.plan, w)
         B = C = lum = None
         if sim.Nv:
             with sim.log.timer('via kernels', f"{sim.Nv} chains"):
-                QF = dv.fan_q(self.mesh, tabs, sim.F)
-                if self._fan is not None:
-                    sel, rows, cols = self._fan
-                    QF[rows, cols] += qc[sel]
-                B, C = sim._via_blocks(f, QF)
+                if kernels is not None:
+                    QF = dv.fan_q(self.mesh, tabs, sim._dev_via()._keep['F'])
+                    B, C = sim.via_blocks(f, QF, qc, kernels)
+                else:
+                    QF = dv.fan_q(self.mesh, tabs, sim.F)
+                    if self._fan is not None:
+                        sel, rows, cols = self._fan
+                        QF[rows, cols] += qc[sel]
+                    B, C = sim._via_blocks(f, QF)
         le = sim.lumped_entries(f)
         if le is not None:
-            r, c, v = (torch.from_numpy(x).to(dev) for x in le)
-            lum = (r, c, v.to(dv.c128))
+            r, c, v = le
+            lum = tuple(dv.upload(np.asarray(r, np.int64), np.asarray(c, np.int64), np.asarray(v, np.complex128)))
         return dict(f=f, w=w, tabs=tabs, M=M, B=B, C=C, lumped=lum)
 
     def assemble(self, st, dtype=dv.c128):

@@ -194,19 +194,32 @@ class LayerStack:
         return complex(out[0], out[1]), complex(out[2], out[3])
 
 
-def sommerfeld_contour(f, stack, rho_max, K=None, nq=8):
-    """(kr, dkr, K): nq-point Gauss-Legendre panels along real t from 0 to K, lifted into Im kr > 0 by
-    lift sin(pi t / t1) up to t1 = 1.5 k_max (clear of the branch points and surface-wave poles), real beyond; the
-    panels are at most min(0.3 k0, 0.8 lift) wide before t1 and 2 pi / rho_max after it (via.py:36-53)."""
+def gauss_legendre(nq, _kept={}):
+    """The nq Gauss-Legendre nodes and weights on [-1, 1] (kept per nq)."""
+    if nq not in _kept:
+        _kept[nq] = np.polynomial.legendre.leggauss(nq)
+    return _kept[nq]
+
+
+def _contour_shape(f, stack, rho_max, K=None):
+    """(t1, lift, K, panels before t1, width of the panels after it) of the contour."""
     k0 = 2 * np.pi * f / C0
     kmax = k0 * np.sqrt(stack.max_er())
     if not K:
         K = max(1e5, 30.0 / stack.hmin) + 40 * kmax
     t1, lift = 1.5 * kmax, min(0.5 * k0, 4.0 / rho_max)
-    near = np.linspace(0, t1, int(np.ceil(t1 / min(0.3 * k0, 0.8 * lift))) + 1)
-    far = np.arange(t1, K, 2 * np.pi / rho_max)[1:]
+    return t1, lift, K, int(np.ceil(t1 / min(0.3 * k0, 0.8 * lift))), 2 * np.pi / rho_max
+
+
+def sommerfeld_contour(f, stack, rho_max, K=None, nq=8):
+    """(kr, dkr, K): nq-point Gauss-Legendre panels along real t from 0 to K, lifted into Im kr > 0 by
+    lift sin(pi t / t1) up to t1 = 1.5 k_max (clear of the branch points and surface-wave poles), real beyond; the
+    panels are at most min(0.3 k0, 0.8 lift) wide before t1 and 2 pi / rho_max after it (via.py:36-53)."""
+    t1, lift, K, near, step = _contour_shape(f, stack, rho_max, K)
+    near = np.linspace(0, t1, near + 1)
+    far = np.arange(t1, K, step)[1:]
     edges = np.concatenate([near, far, [K]])
-    x, wq = np.polynomial.legendre.leggauss(nq)
+    x, wq = gauss_legendre(nq)
     lo, hi = edges[:-1, None], edges[1:, None]
     half, mid = 0.5 * (hi - lo), 0.5 * (lo + hi)
     t, wt = (half * x[None, :] + mid).ravel(), (half * wq[None, :]).ravel()
@@ -217,30 +230,23 @@ def sommerfeld_contour(f, stack, rho_max, K=None, nq=8):
     return t + 1j * lifted, wt * (1 + 1j * slope), K
 
 
-_CONTOURS = {}
-
-
-def device_contour(f, stack, rho_max):
-    """(kr, dkr, K) of sommerfeld_contour on the device, kept for the last few (f, stack, rho_max): the tables and
-    the via kernels of a frequency share one contour."""
-    st = stack.at(f)
-    key = (float(f), float(rho_max), st.key(), torch.cuda.current_device())
-    c = _CONTOURS.get(key)
-    if c is None:
-        kr_h, dk_h, K = sommerfeld_contour(f, st, rho_max)
-        both = dv.on_dev(np.stack([kr_h, dk_h]), dv.c128)
-        c = (both[0], both[1], K)
-        if len(_CONTOURS) >= 4:
-            _CONTOURS.clear()
-        _CONTOURS[key] = c
-    return c
+def device_contour(f, stack, rho_max, nq=8):
+    """(kr, dkr, K) of sommerfeld_contour, computed on the device (m25x_contour)."""
+    t1, lift, K, near, step = _contour_shape(f, stack.at(f), rho_max)
+    # np.arange(t1, K, step)[1:], whose values are t1 + i ((t1 + step) - t1)
+    far = max(0, int(np.ceil((K - t1) / step)) - 1)
+    both = torch.empty((2, (near + far + 1) * nq), dtype=dv.c128, device=dv.device())
+    x, wq = gauss_legendre(nq)
+    L.call('m25x_contour', nq, x.ctypes.data_as(C.c_void_p), wq.ctypes.data_as(C.c_void_p), near, far, float(t1),
+           float(lift), float((t1 + step) - t1), float(K), dv.ptr(both[0]), dv.ptr(both[1]), dv.stream())
+    return both[0], both[1], K
 
 
 _SPLINES = {}
 
 
-def spline_operator(rho_max, nrho, nfine):
-    """The (nfine x nrho) matrix S with S @ y = CubicSpline(rho_max u^2, y)(uniform nfine grid) (not-a-knot, the
+def spline_operator(nrho, nfine):
+    """S^T (nrho x nfine) for the S with S @ y = CubicSpline(rho_max u^2, y)(uniform nfine grid) (not-a-knot, the
     reference's Table1D, via.py:111-123): the spline is linear in its data, so its action is fixed by the grid, and
     a cubic spline is unchanged by a scaling of its abscissae, so one S (built on rho_max = 1) serves every rho_max.
     Built once per (nrho, nfine) on the host, kept on the device."""
@@ -249,14 +255,9 @@ def spline_operator(rho_max, nrho, nfine):
     if S is None:
         rho = np.linspace(0, 1, nrho) ** 2
         fine = np.linspace(0, 1, nfine)
-        S = torch.from_numpy(np.ascontiguousarray(CubicSpline(rho, np.eye(nrho))(fine))).to(dv.device())
+        S = torch.from_numpy(np.ascontiguousarray(CubicSpline(rho, np.eye(nrho))(fine).T)).to(dv.device())
         _SPLINES[key] = S
     return S
-
-
-def resample(S, vals):
-    """S (nfine x n real) applied to complex vals (n, m) on the device."""
-    return torch.complex(S @ vals.real.contiguous(), S @ vals.imag.contiguous())
 
 
 def quad_grid(rho_max, nrho):
@@ -284,8 +285,7 @@ class Requests:
         if not self.ints:
             return W
         ri_h = np.ascontiguousarray(self.ints, dtype=np.int32)
-        ri = torch.from_numpy(ri_h).to(kr.device)
-        rd = torch.from_numpy(np.ascontiguousarray(self.dbls, dtype=np.float64)).to(kr.device)
+        ri, rd = dv.upload(ri_h, np.asarray(self.dbls, dtype=np.float64))
         L.call('m25x_spectra', C.byref(stack.struct(w)), float(w), dv.ptr(kr), dv.ptr(dk), npts, dv.ptr(ri),
                dv.ptr(rd), len(self.ints), ri_h.ctypes.data_as(C.c_void_p), dv.ptr(W), self.rows, dv.stream())
         return W
@@ -372,27 +372,36 @@ class GreenTableML:
         return GA, GQ
 
 
-def _fill_tables(tabs, st, w, contour, rho_max, nrho, nfine):
-    """A_rest and Q_rest of every table in tabs (their extraction set): one spectra launch, one Hankel transform on
-    the quadratic grid, one spline product to the uniform grid."""
-    req = Requests()
+def _request_tables(req, tabs):
+    """The spectra of every table in tabs (their extraction set): two rows of W each, in order from the first on."""
     for t in tabs:
         parts = t.extracted()
         dbl = []
         for d, cA, cq in parts:
             cA, cq = complex(cA), complex(cq)
             dbl += [d, cA.real, cA.imag, cq.real, cq.imag]
-        t._row = req.add(L.SPEC_TABLE, (t.o, t.s, len(parts)), dbl)
-    W = req.run(st, w, contour)
-    rho = dv.on_dev(quad_grid(rho_max, nrho), dv.f64)
-    coarse = hankel(W, contour, rho)                                       # (2 ntab, nrho)
-    fine = resample(spline_operator(rho_max, nrho, nfine), coarse.T)       # (nfine, 2 ntab)
+        req.add(L.SPEC_TABLE, (t.o, t.s, len(parts)), dbl)
+
+
+def _set_tables(tabs, coarse, contour, rho_max, nrho, nfine):
+    """A_rest and Q_rest of the tables from their Hankel transforms coarse (2 ntab, nrho) on the quadratic grid."""
+    fine = dv.resample(spline_operator(nrho, nfine), coarse, pairs=True)   # (ntab, nfine, 2)
     grid = np.linspace(0, rho_max, nfine)
-    for t in tabs:
-        t.A_rest, t.Q_rest = fine[:, t._row], fine[:, t._row + 1]
+    for i, t in enumerate(tabs):
+        t.A_rest, t.Q_rest = fine[i, :, 0], fine[i, :, 1]
         t.rho, t.dr = grid, grid[1]
         t.npts, t.K = int(contour[0].shape[0]), contour[2]
-        t._fine = (fine, t._row)
+        t._fine = (fine, i)
+
+
+def _fill_tables(tabs, st, w, contour, rho_max, nrho, nfine):
+    """A_rest and Q_rest of every table in tabs (their extraction set): one spectra launch, one Hankel transform on
+    the quadratic grid, one spline product to the uniform grid."""
+    req = Requests()
+    _request_tables(req, tabs)
+    W = req.run(st, w, contour)
+    coarse = hankel(W, contour, dv.on_dev(quad_grid(rho_max, nrho), dv.f64))
+    _set_tables(tabs, coarse, contour, rho_max, nrho, nfine)
 
 
 def green_tables(f, stack, layers, rho_max, dmax):
@@ -400,7 +409,13 @@ def green_tables(f, stack, layers, rho_max, dmax):
     3 dmax has its near-singular part extracted, a same-interface pair within 1.5 dmax of a discontinuity its image.
     The tables of a frequency share one contour and are computed in one batch."""
     st, w = stack.at(f), 2 * np.pi * f
-    contour = device_contour(f, stack, rho_max)
+    out = _blank_tables(f, st, w, layers, dmax)
+    if out:
+        _fill_tables(list(out.values()), st, w, device_contour(f, stack, rho_max), rho_max, NRHO, NFINE)
+    return out
+
+
+def _blank_tables(f, st, w, layers, dmax):
     out = {}
     for i, a in enumerate(layers):
         for b in layers[i:]:
@@ -408,8 +423,6 @@ def green_tables(f, stack, layers, rho_max, dmax):
             t._extraction(st, w, cross_sing=a != b and abs(st.z[a] - st.z[b]) < 3 * dmax,
                           image_sing=a == b and st.nearest_discontinuity(a) < 1.5 * dmax)
             out[(a, b)] = t
-    if out:
-        _fill_tables(list(out.values()), st, w, contour, rho_max, NRHO, NFINE)
     return out
 
 
@@ -424,9 +437,8 @@ def device_tables(tables, layers):
         tab[lidx[a], lidx[b]] = tab[lidx[b], lidx[a]] = i
     kind = np.array([0 if a == b else (1 if t.cA != 0 else 2) for (a, b), t in zip(keys, T)], np.int32)
     fine, _ = T[0]._fine
-    if all(t._fine[0] is fine for t in T):
-        cols = torch.tensor(sum(([t._row, t._row + 1] for t in T), []), device=fine.device)
-        AQ = torch.view_as_real(fine[:, cols]).reshape(fine.shape[0], len(T), 4).transpose(0, 1)
+    if fine.shape[0] == len(T) and all(t._fine[0] is fine and t._fine[1] == i for i, t in enumerate(T)):
+        AQ = torch.view_as_real(fine).reshape(len(T), fine.shape[1], 4)
     else:
         AQ = torch.stack([torch.stack([t.A_rest.real, t.A_rest.imag, t.Q_rest.real, t.Q_rest.imag], -1) for t in T])
     scal = dict(dr=np.array([t.dr for t in T]), d=np.array([t.d for t in T], float),

@@ -17,7 +17,7 @@ import torch
 
 from .base import MU0, RWG, geometry, gram_entries
 from .mesh import contains, find_node, tensor_mesh
-from .multilayer import RunLog, device_tables, green_tables
+from .multilayer import NFINE, RunLog, device_tables, green_tables
 from . import device as dv
 
 GPU_MIN_N = 3000          # mixed precision (complex64 LU + FP64 refinement) above this many unknowns
@@ -417,6 +417,64 @@ class Simulation:
 
     VIA_TABLE_PAIRS = 64
 
+    def point_tables(self, f):
+        """green_tables and the via kernels of a frequency in one batch: (D, R) of via.point_kernels, or None where the
+        via blocks compute their own (no vias, or reactions of many chain pairs, which go through a table)."""
+        from .via import point_distances, point_kernels
+        geo = self._via_geometry() if self.Nv else None
+        if geo is None or max(len(dd) for _, _, dd in geo['groups'].values()) > self.VIA_TABLE_PAIRS:
+            self.green_tables(f)
+            return None
+        with self.log.timer('Green tables', f"{len(self.layers)} interfaces @ {f / 1e9:.3f} GHz"):
+            if getattr(self, '_point_rho', None) is None:
+                self._point_rho = point_distances(self.rho_max, geo['groups'])
+            self.tables, D, R = point_kernels(f, self.st, self.layers, self.rho_max, self.dmax, geo['spans'],
+                                              geo['groups'], self._point_rho)
+            self.dev_tables = device_tables(self.tables, self.layers)
+        return D, R
+
+    def via_blocks(self, f, QF, qc, kernels):
+        """_via_blocks on the device alone, from point_tables's kernels: only the K0 parts and the elements are
+        evaluated on the host, and nothing waits for the device. QF: the fans' moments before the near pairs' qc."""
+        from .via import homog
+        st, w, geo = self.st.at(f), 2 * np.pi * f, self._via_geometry()
+        C0 = self._via_elements(f)
+        for (sm, sn), (m, n, dd) in geo['groups'].items():
+            vals = homog(st, w, sm, sn, dd)
+            C0[m, n] += vals
+            off = m != n
+            C0[n[off], m[off]] += vals[off]
+        D, R = kernels
+        C0, = dv.upload(C0)
+        return dv.via_blocks(self._dev_via(), self.fast.mesh, w, QF, qc, D, self._via_dr, R, C0)
+
+    def _via_elements(self, f):
+        """The chains' own part of C: elements in vias and, with metal loss, the barrel's wall loss."""
+        C = np.zeros((self.Nv, self.Nv), complex)
+        zs = self.metal.zs(f) if self.metal is not None else 0.0
+        first = set()
+        for n, (v, lo, hi) in enumerate(self.chains):
+            if v.Z is not None and id(v) not in first:                       # an element: in its lowest chain
+                C[n, n] += v.Z(f)
+            first.add(id(v))
+            C[n, n] += zs * (self.st.z[hi] - self.st.z[lo]) / (2 * np.pi * v.a)
+        return C
+
+    def _dev_via(self):
+        """The vias' fixed arrays for the device (dv.DevVia), once."""
+        if getattr(self, '_devvia', None) is None:
+            geo, r, mesh = self._via_geometry(), self.rwg, self.fast.mesh
+            pair, at = -np.ones((self.Nv, self.Nv), np.int32), 0
+            for m, n, dd in geo['groups'].values():
+                pair[m, n] = pair[n, m] = at + np.arange(len(dd))
+                at += len(dd)
+            span = np.array([geo['spans'].index((lo, hi)) for _, lo, hi in self.chains])
+            self._via_dr = np.linspace(0, self.rho_max, NFINE)[1]
+            self._devvia = dv.DevVia(mesh, len(self.layers), NFINE, self.F, self.dF, geo['x'], geo['y'], span,
+                                     len(geo['spans']), r.tp, r.tm, r.l / r.area[r.tp], -r.l / r.area[r.tm], pair, at,
+                                     self.fast.fan_pairs)
+        return self._devvia
+
     def _via_geometry(self):
         """Geometry of the via blocks, once: each chain's axis, the chains of each span, and every chain pair
         (m <= n) grouped by its two spans with its distance (the barrel radius for two chains of one via, at least
@@ -449,7 +507,7 @@ class Simulation:
         jw = 2j * np.pi * f
         Nt, dev = len(self.rwg.tris), dv.device()
         B = torch.zeros((self.Ne, self.Nv), dtype=dv.c128, device=dev)
-        C = np.zeros((self.Nv, self.Nv), complex)
+        C = self._via_elements(f)
         vk = ViaKernels(f, self.st, [(lo, hi) for _, lo, hi in self.chains], self.layers, self.rho_max)
         geo, div, vd = self._via_geometry(), self._div_ops(), self._via_device()
         if len(self.F):
@@ -469,13 +527,6 @@ class Simulation:
             np.add.at(C, (m, n), vals)
             off = m != n
             np.add.at(C, (n[off], m[off]), vals[off])
-        zs = self.metal.zs(f) if self.metal is not None else 0.0
-        first = set()
-        for n, (v, lo, hi) in enumerate(self.chains):
-            if v.Z is not None and id(v) not in first:                       # an element: in its lowest chain
-                C[n, n] += v.Z(f)
-            first.add(id(v))
-            C[n, n] += zs * (self.st.z[hi] - self.st.z[lo]) / (2 * np.pi * v.a)
         return B, torch.from_numpy(C).to(dev)
 
     def _via_device(self):

@@ -1,0 +1,80 @@
+"""A frequency's preparation in one batch (contour, spectra, Hankel sums, splines and via blocks on the device) against
+the same parts one by one: the host's contour, m25x_hankel, a NumPy spline product and the ViaKernels classes. Both
+sides compute in FP64 with sums in another order: bounds of the number of terms times eps."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(float).eps
+
+
+@pytest.mark.parametrize('f', [1e8, 2.3e9, 4e10])
+def test_contour(gpu, f):
+    from mom25d_amd.multilayer import Layer, LayerStack, device_contour, sommerfeld_contour
+    for top, rho_max in (('open', 0.02), ('open', 1e-4), ('pec', 0.3)):
+        st = LayerStack([Layer(0.2e-3, 4.3, 0.02), Layer(0.5e-3, 3.1, 0.001, fref=1e9)], top=top)
+        kr, dk, K = sommerfeld_contour(f, st.at(f), rho_max)
+        a, b, K2 = device_contour(f, st, rho_max)
+        assert K2 == K and len(a) == len(kr)
+        # edges of the panels are rounded to eps K on both sides; a panel's weights are their differences
+        assert np.abs(a.cpu().numpy() - kr).max() <= 8 * EPS * K
+        assert np.abs(b.cpu().numpy() - dk).max() <= 8 * EPS * K
+
+
+def test_hankel_sets(gpu):
+    dv = gpu
+    rng = np.random.default_rng(1)
+    kr = np.sort(rng.uniform(0, 4e3, 700)) + 1j * np.where(np.arange(700) < 90, 5.0, 0.0)
+    kr, W = dv.on_dev(kr, dv.c128), dv.on_dev(rng.standard_normal((9, 700)) + 1j * rng.standard_normal((9, 700)), dv.c128)
+    for sets in ([(1, 8, 1)], [(260, 0, 4), (200, 4, 5), (3, 8, 1)], [(2, i % 9, 1) for i in range(40)]):
+        rho = dv.on_dev(rng.uniform(0, 0.02, sum(c for c, _, _ in sets)), dv.f64)
+        at = 0
+        for (c, row, rows), got in zip(sets, dv.hankel_sets(rho, sets, kr, W, 2.0)):
+            want = dv.hankel_sum(rho[at:at + c], kr, W[row:row + rows])
+            assert torch.equal(2.0 * got, want)                          # the same kernel, sums halved exactly
+            at += c
+    with pytest.raises(ValueError):
+        dv.hankel_sets(rho, [(80, 8, 2)], kr, W)                         # row 9 of 9
+
+
+@pytest.mark.parametrize('nc, nfine, rows', [(1, 5, 2), (200, 8192, 6), (513, 63, 3), (1025, 65, 8)])
+def test_resample(gpu, nc, nfine, rows):
+    dv = gpu
+    rng = np.random.default_rng(nc)
+    S = rng.standard_normal((nc, nfine))
+    y = rng.standard_normal((rows, nc)) + 1j * rng.standard_normal((rows, nc))
+    want, bound = y @ S, 4 * nc * EPS * (np.abs(y) @ np.abs(S))
+    St, yd = dv.on_dev(S, dv.f64), dv.on_dev(y, dv.c128)
+    got = dv.resample(St, yd).cpu().numpy()
+    assert np.all(np.abs(got - want) <= bound)
+    if rows % 2 == 0:
+        pairs = dv.resample(St, yd, pairs=True).cpu().numpy()
+        assert np.array_equal(pairs.transpose(0, 2, 1).reshape(rows, nfine), got)
+    else:
+        with pytest.raises(ValueError):
+            dv.resample(St, yd, pairs=True)
+
+
+@pytest.mark.parametrize('board', ['microstrip', 'coupled_lines', 'seeded_board'])
+def test_via_blocks_and_tables(gpu, board):
+    from mom25d_amd import boards
+    from mom25d_amd.multilayer import green_tables
+    from mom25d_amd.sim import Simulation
+    dv, f = gpu, 2.3e9
+    st, shapes, ports, vias, kw = getattr(boards, board)(dmax=1.5e-3, ncross=2)
+    sim = Simulation(st, shapes, ports, vias, verbose=False, **kw)
+    state = sim.fast.prepare(f)
+    tables = green_tables(f, sim.st, sim.layers, sim.rho_max, sim.dmax)
+    for key, t in tables.items():
+        for a, b in ((sim.tables[key].A_rest, t.A_rest), (sim.tables[key].Q_rest, t.Q_rest)):
+            assert (a - b).abs().max() <= 1e-13 * b.abs().max()
+    if not sim.Nv:
+        return
+    fo = sim.fast
+    QF = dv.fan_q(fo.mesh, fo.tabs, sim.F)
+    _, qc = dv.near_moments(fo.mesh, fo.tabs, fo.plan, 2 * np.pi * f)
+    sel, rows, cols = fo._fan
+    QF[rows, cols] += qc[sel]
+    for got, want in zip((state['B'], state['C']), sim._via_blocks(f, QF)):
+        assert got.shape == want.shape and (got - want).abs().max() <= 1e-12 * want.abs().max()
