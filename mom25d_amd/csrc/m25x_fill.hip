@@ -41,24 +41,35 @@ template <> __device__ inline void store_c<float2>(float2 *Z, size_t i, double2 
 }
 
 // ---- far field -------------------------------------------------------------------------------------------
-// One 256-thread workgroup per 32 x 32 tile of edge pairs in the upper triangle (tile row <= tile column):
+// One 512-thread workgroup per 32 x 32 tile of edge pairs in the upper triangle (tile row <= tile column):
 // Z[m, n] for m in the row tile, n in the column tile, each the reference's sum over the halves (s, t) of
 //   a_ms a_nt [jw (c_ms - v_ms).(c_nt - v_nt) G_A(r) + 4 G_q(r) / (jw)],  r = |c_ms - c_nt|,
 // (mom25d_core.cpp:152-170), stored at (m, n) and, through LDS, at (n, m): Z is symmetric bit for bit.
+//
+// The kernel's value (square roots, divisions, two interpolations) bounds the fill, and it depends on the two triangles
+// only: edges that follow each other share triangles (32 edges of a mesh have some 33, not 64), so it is computed once
+// for each pair of the tile's triangles and the entries read it from LDS: a quarter of the evaluations, 7799 unknowns
+// 1130 -> 580 us. Where a tile's triangles are too many for the LDS (edges in an order of their own) each entry
+// computes its own four.
 struct Half {
     double a, dx, dy, cx, cy;
-    int lay, pad;
+    int lay, tri;
 };
 
-constexpr int FT = 32;
+constexpr int FT = 32, FTH = 512;         // edges of a tile's side; threads
+constexpr int FP = 1296;                  // triangle pairs that the LDS holds (36 x 36; two workgroups a CU)
 
 template <typename TZ>
-__global__ __launch_bounds__(256) void k_fill_far(TZ *__restrict__ Z, long ld, DMesh g, DTab T, double w)
+__global__ __launch_bounds__(FTH) void k_fill_far(TZ *__restrict__ Z, long ld, DMesh g, DTab T, double w)
 {
     const int ti = blockIdx.y, tj = blockIdx.x;
     if (ti > tj) return;
-    __shared__ Half hr[2][FT], hc[2][FT];
+    __shared__ Half hf[2][2 * FT];                           // [rows, columns][s * 32 + edge]
+    __shared__ __align__(16) int tr[2][2 * FT];              // their triangles
     __shared__ double2 tile[FT][FT + 1];
+    __shared__ double2 KA[FP], KQ[FP];                       // G_A and G_q of a pair of distinct triangles
+    __shared__ unsigned char un[2][2 * FT], rep[2][2 * FT];  // a half's number among its side's distinct triangles, and
+    __shared__ unsigned short firsts[2][4];                  // a distinct triangle's first half; which halves are first
     const int tid = threadIdx.x;
     const int m0 = ti * FT, n0 = tj * FT, Ne = g.Ne;
     if (tid < 4 * FT) {
@@ -66,7 +77,7 @@ __global__ __launch_bounds__(256) void k_fill_far(TZ *__restrict__ Z, long ld, D
         const int edge = (side ? n0 : m0) + e;
         Half h;
         h.a = h.dx = h.dy = h.cx = h.cy = 0.0;
-        h.lay = 0; h.pad = 0;
+        h.lay = 0; h.tri = -1;
         if (edge < Ne) {
             const int tri = s ? g.em[edge] : g.ep[edge];
             const double alpha = s ? g.am[edge] : g.ap[edge];
@@ -75,26 +86,89 @@ __global__ __launch_bounds__(256) void k_fill_far(TZ *__restrict__ Z, long ld, D
             h.cx = g.cent[2 * tri]; h.cy = g.cent[2 * tri + 1];
             h.dx = h.cx - v[0]; h.dy = h.cy - v[1];
             h.lay = g.lt[tri];
+            h.tri = tri;
         }
-        if (side) hc[s][e] = h; else hr[s][e] = h;
+        hf[side][k] = h;
+        tr[side][k] = h.tri;
     }
     __syncthreads();
-    const int c = tid % FT, rg = tid / FT;          // 8 row groups of 4 rows
-    const double iw = 1.0 / w;
-    const Half cn0 = hc[0][c], cn1 = hc[1][c];
+    // the distinct triangles of each side: four lanes a half look for the first half with its triangle
+    const int side = tid >> 8, q = tid & 3, half = (tid >> 2) & 63;
+    int first = half;
+    {
+        const int mine = tr[side][half];
+        const int4 *t4 = (const int4 *)tr[side] + 4 * q;
 #pragma unroll
-    for (int k = 0; k < FT / 8; ++k) {
-        const int r = rg + 8 * k;
+        for (int i = 3; i >= 0; --i) {
+            const int4 v = t4[i];
+            const int b = 16 * q + 4 * i;
+            if (v.w == mine) first = min(first, b + 3);
+            if (v.z == mine) first = min(first, b + 2);
+            if (v.y == mine) first = min(first, b + 1);
+            if (v.x == mine) first = min(first, b);
+        }
+        first = min(first, __builtin_amdgcn_update_dpp(first, first, 0xB1, 0xF, 0xF, false));      // over the quad
+        first = min(first, __builtin_amdgcn_update_dpp(first, first, 0x4E, 0xF, 0xF, false));
+    }
+    {
+        // a wave holds 16 halves, four lanes each: one bit a half
+        unsigned long long m = __builtin_amdgcn_ballot_w64(first == half && q == 0) & 0x1111111111111111ull;
+        m = (m | m >> 3) & 0x0303030303030303ull;
+        m = (m | m >> 6) & 0x000f000f000f000full;
+        m = (m | m >> 12) & 0x000000ff000000ffull;
+        m = (m | m >> 24) & 0xffffull;
+        if ((tid & 63) == 0) firsts[side][(tid >> 6) & 3] = (unsigned short)m;
+    }
+    __syncthreads();
+    unsigned long long fm[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+        fm[d] = (unsigned long long)firsts[d][0] | (unsigned long long)firsts[d][1] << 16 |
+                (unsigned long long)firsts[d][2] << 32 | (unsigned long long)firsts[d][3] << 48;
+    if (q == 0) {
+        const int u = __popcll(fm[side] & ((1ull << first) - 1));
+        un[side][half] = (unsigned char)u;
+        if (first == half) rep[side][u] = (unsigned char)half;
+    }
+    __syncthreads();
+    const int ncol = __popcll(fm[1]), np = __popcll(fm[0]) * ncol;
+    const bool shared = np <= FP;
+    if (shared) {
+        for (int p = tid; p < np; p += FTH) {
+            const int a = p / ncol;
+            const Half &hm = hf[0][rep[0][a]], &hn = hf[1][rep[1][p - a * ncol]];
+            const double ddx = hm.cx - hn.cx, ddy = hm.cy - hn.cy;
+            double2 ga, gq;
+            tab_kern(T, hm.lay, hn.lay, sqrt(ddx * ddx + ddy * ddy), ga, gq);
+            KA[p] = ga;
+            KQ[p] = gq;
+        }
+        __syncthreads();
+    }
+    const int c = tid % FT, rg = tid / FT;          // rows rg and rg + 16
+    const double iw = 1.0 / w;
+    const Half cn0 = hf[1][c], cn1 = hf[1][FT + c];
+    const int u0 = un[1][c], u1 = un[1][FT + c];
+#pragma unroll
+    for (int k = 0; k < FT * FT / FTH; ++k) {
+        const int r = rg + FTH / FT * k;
         double vx = 0.0, vy = 0.0;
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
-            const Half hm = hr[s][r];
+            const Half hm = hf[0][s * FT + r];
+            const int pr = un[0][s * FT + r] * ncol;
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
                 const Half &hn = t ? cn1 : cn0;
-                const double ddx = hm.cx - hn.cx, ddy = hm.cy - hn.cy;
                 double2 ga, gq;
-                tab_kern(T, hm.lay, hn.lay, sqrt(ddx * ddx + ddy * ddy), ga, gq);
+                if (shared) {
+                    const int p = pr + (t ? u1 : u0);
+                    ga = KA[p];
+                    gq = KQ[p];
+                } else {
+                    const double ddx = hm.cx - hn.cx, ddy = hm.cy - hn.cy;
+                    tab_kern(T, hm.lay, hn.lay, sqrt(ddx * ddx + ddy * ddy), ga, gq);
+                }
                 const double wd = w * (hm.dx * hn.dx + hm.dy * hn.dy);
                 const double tx = -wd * ga.y + 4.0 * gq.y * iw, ty = wd * ga.x - 4.0 * gq.x * iw;
                 const double f = hm.a * hn.a;
@@ -106,14 +180,14 @@ __global__ __launch_bounds__(256) void k_fill_far(TZ *__restrict__ Z, long ld, D
     __syncthreads();
     const bool diag = ti == tj;
 #pragma unroll
-    for (int k = 0; k < FT / 8; ++k) {
-        const int r = rg + 8 * k, m = m0 + r, n = n0 + c;
+    for (int k = 0; k < FT * FT / FTH; ++k) {
+        const int r = rg + FTH / FT * k, m = m0 + r, n = n0 + c;
         if (m < Ne && n < Ne) store_c(Z, (size_t)m * ld + n, (diag && r > c) ? tile[c][r] : tile[r][c]);
     }
     if (!diag) {
 #pragma unroll
-        for (int k = 0; k < FT / 8; ++k) {
-            const int r = rg + 8 * k, n = n0 + r, m = m0 + c;
+        for (int k = 0; k < FT * FT / FTH; ++k) {
+            const int r = rg + FTH / FT * k, n = n0 + r, m = m0 + c;
             if (n < Ne && m < Ne) store_c(Z, (size_t)n * ld + m, tile[c][r]);
         }
     }
@@ -559,10 +633,10 @@ __global__ __launch_bounds__(256) void k_hankel(HankelSets hs, const double *rho
 
 // ---- tables on the uniform grid ------------------------------------------------------------------------------
 // out[row][i] = sum_j S[i][j] y[row][j], S given transposed (nc x nfine) so that a wave's loads of it are whole lines;
-// a lane a fine point, RS rows a thread, a quarter of the nodes a wave whose loads are asked for
-// many at a time. 14 us with S in the caches, 28 without (a point finds it there no more), the rows' coarse values in LDS. pairs: rows 2 t and 2 t + 1 side by side per point
-// (the tables' A and Q). Reading S, 8192 x 260 doubles, bounds it; the library's two real products and the copies into
-// this layout took 60 us more.
+// a lane a fine point, RS rows a thread, a quarter of the nodes a wave, whose loads are asked for many at a time; the
+// rows' coarse values in LDS. pairs: rows 2 t and 2 t + 1 side by side per point (the tables' A and Q). Reading S, 8192
+// x 260 doubles, bounds it: 14 us with S in the caches, 28 without (a point finds it there no more); the library's two
+// real products and the copies into this layout took 60 us more.
 constexpr int RS = 4, RP = 64, RG = 4;       // rows a thread, points and node groups of a workgroup
 constexpr int RN = 512, RU = 22;             // coarse nodes in LDS at a time; loads of S in flight a thread
 __global__ __launch_bounds__(RP * RG) void k_resample(const double *St, int nc, int nfine, const double2 *y, int rows,
@@ -964,9 +1038,9 @@ int m25x_fill_far(void *Z, int zdtype, long ld, const m25x_mesh *g, const m25x_t
     hipStream_t s = (hipStream_t)stream;
     TimedLaunch tl(s, M25X_K_FILL_FAR, zdtype, (zdtype == M25X_C128 ? 16.0 : 8.0) * g->Ne * (double)g->Ne, 0.0);
     if (zdtype == M25X_C128)
-        hipLaunchKernelGGL(k_fill_far<double2>, grid, dim3(256), 0, s, (double2 *)Z, ld, dmesh(g), dtab(tb), w);
+        hipLaunchKernelGGL(k_fill_far<double2>, grid, dim3(FTH), 0, s, (double2 *)Z, ld, dmesh(g), dtab(tb), w);
     else if (zdtype == M25X_C64)
-        hipLaunchKernelGGL(k_fill_far<float2>, grid, dim3(256), 0, s, (float2 *)Z, ld, dmesh(g), dtab(tb), w);
+        hipLaunchKernelGGL(k_fill_far<float2>, grid, dim3(FTH), 0, s, (float2 *)Z, ld, dmesh(g), dtab(tb), w);
     else
         return fail(M25X_EINVAL, "fill_far: zdtype %d", zdtype);
     return check_launch("fill_far");
