@@ -370,6 +370,16 @@ __device__ __forceinline__ int reg_gepp(bool have, const T *src, long lda, int n
     return npiv;
 }
 
+// an int that another workgroup of the launch reads, or wrote
+__device__ __forceinline__ void put_word(int *p, int v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int get_word(const int *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The tournament of panel [j0, j0 + jb) over rows [j0, n). Leaves: blockIdx.x (P of them) of RL rows. A node takes its
 // children's nominees straight from A, which the launch leaves untouched: only their row numbers pass between
 // workgroups. The root writes the panel's L11 \ U11 (top, column-major TW x TW), the interchanges (ipiv[j0 .. j0 + jb),
@@ -406,31 +416,33 @@ __device__ __forceinline__ void tslu_body(const T *A, long lda, long n, long j0,
             nchild = std::min(AR, lsize - parent * AR);
         }
         const int poff = loff + lsize, first = parent * AR;
-        // nominate: this node's pivot rows
+        // Nominate: this node's pivot rows. They pass between workgroups as device-scope words, which go past the caches,
+        // each wave waiting for its own before the workgroup counts itself in: a device-scope fence instead writes
+        // back and drops a whole L2, which waits for whatever else is dirty there (beside a trailing update or a copy
+        // a tournament took 1.5 to 1.8 times as long with three fences a level) and costs the update its tiles.
         TNode<T> *nd = nodes + loff + idx;
-        if (t == 0) nd->count = cnt;
-        if (t < cnt) nd->id[t] = ids[order[t]];
-        __threadfence();
+        if (t == 0) put_word(&nd->count, cnt);
+        if (t < cnt) put_word(&nd->id[t], ids[order[t]]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         if (t == 0) {
-            const int old = __hip_atomic_fetch_add(arrive + poff + parent, 1, __ATOMIC_ACQ_REL,
+            const int old = __hip_atomic_fetch_add(arrive + poff + parent, 1, __ATOMIC_RELAXED,
                                                    __HIP_MEMORY_SCOPE_AGENT);
             go = old == nchild - 1;
             if (go) __hip_atomic_store(arrive + poff + parent, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
         if (!go) return;
-        __threadfence();
         // the last child to arrive factors the node: its children's nominees stacked in child order
         const TNode<T> *c0n = nodes + loff + first;
-        if (t < nchild) counts[t] = c0n[t].count;
+        if (t < nchild) counts[t] = get_word(&c0n[t].count);
         __syncthreads();
         int ch = 0, i = row;
         nr = 0;
         for (int q = 0; q < nchild; ++q) nr += counts[q];
         while (ch < nchild - 1 && i >= counts[ch]) { i -= counts[ch]; ++ch; }
         have = row < nr;
-        const int id = have ? c0n[ch].id[i] : (int)r0;
+        const int id = have ? get_word(&c0n[ch].id[i]) : (int)r0;
         src = A + j0 * lda + id;
         if (have && h == 0) ids[row] = id;
         loff = poff;
