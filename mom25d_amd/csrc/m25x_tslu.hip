@@ -248,9 +248,8 @@ template <int N> __device__ __forceinline__ void fms4(double *xr, double *xi, do
 // The thread's columns J0 .. J1 - 1 (multiples of four) updated by pivot jp of a sub-panel: its multiplier l, the
 // pivot row's values (U12) from LDS.
 template <typename T, int J0, int J1>
-__device__ __forceinline__ void row_update(RowH<T> &x, T l, const T *us)
+__device__ __forceinline__ void row_update(RowH<T> &x, T l, const T *us, int l16)
 {
-    const int l16 = threadIdx.x & 15;
     if constexpr (J0 < J1 && J0 < 16) {
         const T u = us[l16];
         auto upd = [&](auto qc) __attribute__((always_inline)) {
@@ -323,15 +322,19 @@ __device__ __forceinline__ int reg_gepp(bool have, const T *src, long lda, int n
     auto sub = [&](auto sc) __attribute__((always_inline)) {
         constexpr int s = decltype(sc)::value, kb = s * SPW, J = (s + 1) * (SPW / 2), JN = J + SPW / 2;
         if (!more) return;
+        // the thread's places in LDS computed anew for each sub-panel: kept for all of them they go to scratch memory
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int row = (tid >> 6) * 32 + (tid & 31), h = (tid >> 5) & 1, l16 = tid & 15;
         const int nst = npiv - kb < SPW ? npiv - kb : SPW;
 #pragma unroll 1
         for (int jp = 0; jp < nst; ++jp) {      // the panel waves' steps; meanwhile the last sub-panel's pivots
             lds_barrier();
-            if constexpr (s > 0 && J < TH) row_update<T, J, TH>(x, sh.lp[(s & 1) ^ 1][jp][row], sh.us[jp][h]);
+            if constexpr (s > 0 && J < TH) row_update<T, J, TH>(x, sh.lp[(s & 1) ^ 1][jp][row], sh.us[jp][h], l16);
             lds_barrier();
         }
         if constexpr (s > 0 && J < TH)
-            for (int jp = nst; jp < SPW; ++jp) row_update<T, J, TH>(x, sh.lp[(s & 1) ^ 1][jp][row], sh.us[jp][h]);
+            for (int jp = nst; jp < SPW; ++jp) row_update<T, J, TH>(x, sh.lp[(s & 1) ^ 1][jp][row], sh.us[jp][h], l16);
         lds_barrier();                          // A
         if (top) {                              // the rows that become pivots later keep their multipliers
 #pragma unroll
@@ -350,7 +353,7 @@ __device__ __forceinline__ int reg_gepp(bool have, const T *src, long lda, int n
             lds_barrier();                      // B
             lds_barrier();                      // C
 #pragma unroll
-            for (int jp = 0; jp < SPW; ++jp) row_update<T, J, JN>(x, sh.lp[s & 1][jp][row], sh.us[jp][h]);
+            for (int jp = 0; jp < SPW; ++jp) row_update<T, J, JN>(x, sh.lp[s & 1][jp][row], sh.us[jp][h], l16);
 #pragma unroll
             for (int i = 0; i < SPW / 2; ++i) sh.lp[(s & 1) ^ 1][2 * i + h][row] = x.get(J + i);
             lds_barrier();                      // D
