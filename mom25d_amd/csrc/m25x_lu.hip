@@ -753,8 +753,29 @@ template <typename T> __device__ __forceinline__ void rhs_row(const Tri<T> &c, l
     b[1] = csel(c.kc > 1, p[c.kc > 1 ? 1 : 0], CX<T>::make(0, 0));
 }
 
-// sums within groups of lanes by DPP moves: quad_perm [1,0,3,2] (0xB1), quad_perm [2,3,0,1] (0x4E), row_half_mirror
-// (0x141); and over the halves and quarters of a wave by lane swaps
+// right-hand side r of rows g0 and g1
+template <typename T> __device__ __forceinline__ void rhs_pair(const Tri<T> &c, long g0, long g1, int r, T (&b)[2])
+{
+    if (c.wait) {
+        const T *p0 = c.src + g0 * CR + r, *p1 = c.src + g1 * CR + r;
+        auto attempt = [&]() {
+            const bool a0 = take(p0, b[0]), a1 = take(p1, b[1]);
+            return a0 && a1;
+        };
+        const bool ok = attempt();
+        if (!wave_all(ok)) {
+            if ((threadIdx.x & 63) == 0) nap_wait(p0, 64, c.abort);
+            wave_wait<true>(ok, c.abort, attempt);
+        }
+        return;
+    }
+    const int rr = r < c.kc ? r : 0;
+    const T zero = CX<T>::make(0, 0);
+    b[0] = csel(r < c.kc, c.src[(c.sperm ? (long)c.sperm[g0] : g0) * c.lds + rr], zero);
+    b[1] = csel(r < c.kc, c.src[(c.sperm ? (long)c.sperm[g1] : g1) * c.lds + rr], zero);
+}
+
+// sums within groups of lanes by DPP moves: quad_perm [1,0,3,2] (0xB1), quad_perm [2,3,0,1] (0x4E); and over the halves and quarters of a wave by lane swaps
 template <int CTRL> __device__ __forceinline__ float dpp_of(float v)
 {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
@@ -883,12 +904,8 @@ __device__ __forceinline__ int far_sum(typename CX<T>::R (&o)[2 * CR], Tile<T> (
         for (int e = 0; e < 4; ++e) ok &= is_set(yn[e]);
         ok |= !(gk < n);
         if (!wave_all(ok)) {
-            if (q - p > 2) {
-                if (lane == 0 && k0 < n) nap_wait(c.dst + k0 * CR, q - p, c.abort);
-                wave_wait<true>(ok, c.abort, [&]() { return ask(p); });
-            } else {
-                wave_wait<false>(ok, c.abort, [&]() { return ask(p); });
-            }
+            if (q - p > 2 && lane == 0 && k0 < n) nap_wait(c.dst + k0 * CR, q - p, c.abort);
+            wave_wait<true>(ok, c.abort, [&]() { return ask(p); });
         }
         T y[4];
 #pragma unroll
@@ -932,12 +949,13 @@ __device__ __forceinline__ int far_sum(typename CX<T>::R (&o)[2 * CR], Tile<T> (
 // -- complex64 --
 // The block's own triangle is inverted in FP64 when the workgroup starts, and the inverse multiplied into the tile of
 // the block before it (W = inv(Op_qq) Op_q,q-1, FP64 too): a block's step is then y_q = z_q - W y_q-1, one product,
-// with z_q = inv(Op_qq) (b_q - sum over a < q - 1 of Op_qa y_a) formed while y_q-1 is still on its way. Substitution
-// needs 64 dependent steps instead, 1.4 us at 52 cycles (a broadcast and two dependent multiply-adds): the block's step
-// went from 3.0 to 1.5 us (hand-off 0.6, meeting at the barrier 0.15, the product 0.35, its sums over lanes 0.15, and
-// z_q not ready before) and a solve of N = 7799, 4 right-hand sides from 739 to 452 us. The products in FP64 with the
-// inverse in FP64 keep what substitution in FP32 gives and more: an inverse's error, eps64 cond(Op_qq), stays under
-// eps32 up to condition 5e8, and measured against FP64 solves of the same factor the solution's error is
+// with z_q = inv(Op_qq) (b_q - sum over a < q - 1 of Op_qa y_a) formed by the other half of the waves while y_q-1 is
+// still on its way. Substitution needs 64 dependent steps instead, 1.4 us at 52 cycles (a broadcast and two dependent
+// multiply-adds): the block's step went from 3.0 to 1.4 us, of which the way from one workgroup's store to the next one's
+// sight of it is about 1.0 (0.54 with one line and nothing else on the way; it grows with the lines a poll asks for, but
+// passing them on in LDS costs as much), and a solve of N = 7799, 4 right-hand sides from 739 to 425 us. The products in
+// FP64 with the inverse in FP64 keep what substitution in FP32 gives and more: an inverse's error, eps64 cond(Op_qq),
+// stays under eps32 up to condition 5e8, and measured against FP64 solves of the same factor the solution's error is
 // 1.3e-7 against the substitution's 3.9e-7 on a board-like system of N = 3001, 6e-5 against 1e-4 on a random one (an
 // inverse or W rounded to FP32 is not good enough: a factor whose pivots span 1e7 then preconditions poorly).
 // The first blocks of a chain take the tile before theirs as any other one: W is ready 10 us after the inverse, and until
@@ -1016,16 +1034,61 @@ __device__ __forceinline__ void invert_lower(double2 (*S)[S_LD], const double2 *
     invert_level<32>(S, tid);
 }
 
-// (ar, ai)[r] += sum over the lane's columns c8 + 8 v of (wr, wi)[v] x[column][r]
-__device__ __forceinline__ void rows_product(double (&ar)[CR], double (&ai)[CR], const double (&wr)[TE],
-                                             const double (&wi)[TE], const double2 (*x)[CR], int c8)
+// The products of the chain's steps. A wave has 16 rows of the operator, lane (cg, r) = (lane / 16, lane % 16) row r and
+// columns 16 cg + v, and lane (cg, l) the vector's elements pair_col(h, lane) for right-hand side l % 2: the lanes of a
+// column group then find its 16 pairs in their own DPP row, and a multiply-add takes them from there (row_newbcast) with
+// no LDS read, exchange or barrier between a vector's arrival and the product. Written out because the compiler does not fold a 64-bit broadcast into the operation;
+// the s_nop covers the two wait states between a vector write of x and its DPP read.
+__device__ inline int pair_col(int h, int lane) { return (lane & 48) + 8 * h + ((lane & 15) >> 1); }
+template <int N>
+__device__ __forceinline__ void mac4(double (&a)[8], double xr, double xi, const double *wr, const double *wi)
 {
-#pragma unroll
-    for (int v = 0; v < TE; ++v)
-#pragma unroll
-        for (int r = 0; r < CR; ++r) zfma(ar[r], ai[r], make_double2(wr[v], wi[v]), x[c8 + 8 * v][r]);
+    constexpr int n = 2 * (N & 7);
+#define M25X_MAC(A0, A1, A2, A3, R, I, n0, n1, x, s)                                                         \
+    "v_fmac_f64_dpp %" #A0 ", %" #x ", " s "%" #R " row_newbcast:%c" #n0 " row_mask:0xf bank_mask:0xf\n"     \
+    "v_fmac_f64_dpp %" #A1 ", %" #x ", %" #I " row_newbcast:%c" #n0 " row_mask:0xf bank_mask:0xf\n"          \
+    "v_fmac_f64_dpp %" #A2 ", %" #x ", " s "%" #R " row_newbcast:%c" #n1 " row_mask:0xf bank_mask:0xf\n"     \
+    "v_fmac_f64_dpp %" #A3 ", %" #x ", %" #I " row_newbcast:%c" #n1 " row_mask:0xf bank_mask:0xf\n"
+#define M25X_MAC2(R, I, n0, n1, R2, I2, m0, m1)                                                              \
+    M25X_MAC(0, 1, 2, 3, R, I, n0, n1, 8, "") M25X_MAC(4, 5, 6, 7, R2, I2, m0, m1, 8, "")                    \
+    M25X_MAC(0, 1, 2, 3, I, R, n0, n1, 9, "-") M25X_MAC(4, 5, 6, 7, I2, R2, m0, m1, 9, "-")
+    asm("s_nop 1\n" M25X_MAC2(10, 14, 18, 19, 11, 15, 20, 21) M25X_MAC2(12, 16, 22, 23, 13, 17, 24, 25)
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7])
+        : "v"(xr), "v"(xi), "v"(wr[N]), "v"(wr[N + 1]), "v"(wr[N + 2]), "v"(wr[N + 3]), "v"(wi[N]), "v"(wi[N + 1]),
+          "v"(wi[N + 2]), "v"(wi[N + 3]), "n"(n), "n"(n + 1), "n"(n + 2), "n"(n + 3), "n"(n + 4), "n"(n + 5), "n"(n + 6),
+          "n"(n + 7));
+#undef M25X_MAC2
+#undef M25X_MAC
 }
-
+// the sums over v and, by lane exchanges, over the four column groups: lane (cg, r) gets row r's real (cg even) or
+// imaginary part for right-hand side cg / 2. Even and odd columns in sums of their own: eight chains of multiply-adds
+// cover their latency.
+__device__ __forceinline__ double rows_product(const float2 (&x)[2], const double *wr, const double *wi)
+{
+    const double r0 = (double)x[0].x, i0 = (double)x[0].y, r1 = (double)x[1].x, i1 = (double)x[1].y;
+    double a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    mac4<0>(a, r0, i0, wr, wi);
+    mac4<4>(a, r0, i0, wr, wi);
+    mac4<8>(a, r1, i1, wr, wi);
+    mac4<12>(a, r1, i1, wr, wi);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) a[e] += a[4 + e];
+    return swap16_add(swap32_add(a[0], a[2]), swap32_add(a[1], a[3]));
+}
+// (wr, wi)[N + i] -= a x[N + i of the DPP row], i < 4: a row of W gains the multiple a of a row of the tile
+template <int N> __device__ __forceinline__ void row_msub4(double *wr, double *wi, double2 x, double2 a)
+{
+#define M25X_MSUB(R, I, n)                                                                                   \
+    "v_fmac_f64_dpp %" #R ", %8, -%10 row_newbcast:%c" #n " row_mask:0xf bank_mask:0xf\n"                    \
+    "v_fmac_f64_dpp %" #I ", %8, -%11 row_newbcast:%c" #n " row_mask:0xf bank_mask:0xf\n"                    \
+    "v_fmac_f64_dpp %" #R ", %9, %11 row_newbcast:%c" #n " row_mask:0xf bank_mask:0xf\n"                     \
+    "v_fmac_f64_dpp %" #I ", %9, -%10 row_newbcast:%c" #n " row_mask:0xf bank_mask:0xf\n"
+    asm("s_nop 1\n" M25X_MSUB(0, 4, 12) M25X_MSUB(1, 5, 13) M25X_MSUB(2, 6, 14) M25X_MSUB(3, 7, 15)
+        : "+v"(wr[N]), "+v"(wr[N + 1]), "+v"(wr[N + 2]), "+v"(wr[N + 3]), "+v"(wi[N]), "+v"(wi[N + 1]), "+v"(wi[N + 2]),
+          "+v"(wi[N + 3])
+        : "v"(x.x), "v"(x.y), "v"(a.x), "v"(a.y), "n"(N), "n"(N + 1), "n"(N + 2), "n"(N + 3));
+#undef M25X_MSUB
+}
 template <bool RM>
 __device__ __forceinline__ void chain_of(const Tri<float2> &c, int q)
 {
@@ -1055,11 +1118,12 @@ __device__ __forceinline__ void chain_of(const Tri<float2> &c, int q)
         md[u] = RM ? c.LU[gi * c.lda + gk] : c.LU[gk * c.lda + gi];
         mn[u] = RM ? c.LU[gi * c.lda + gn] : c.LU[gn * c.lda + gi];
     }
-    // the lane's row of the products below: waves w and w + 4 share a SIMD, and W's rows take more the later they are
-    const int li = 8 * (wv < 4 ? wv : 11 - wv) + (lane >> 3), c8 = lane & 7, gl = flip(li);
+    // waves 0-3 end with a row of -W each lane and finish the block, waves 4-7 with one of the inverse and form z
+    const bool last = wv < 4;
+    const int wi4 = wv & 3, li = 16 * wi4 + (lane & 15), gl = flip(li);    // the lane's row of the products
     const bool inrow = gl < m;
     const long grow = r0 + std::min(gl, m - 1);
-    const long orow = c.out && c.operm ? c.operm[grow] : grow;
+    const long orow = last && c.out && c.operm ? c.operm[grow] : grow;
     constexpr int D = Depth<float2>::D;
     Tile<float2> t[D];
     far_begin<float2, RM>(t, c, nfar, r0, m, wv, lane, order);
@@ -1077,79 +1141,85 @@ __device__ __forceinline__ void chain_of(const Tri<float2> &c, int q)
     }
     __syncthreads();
     invert_lower(S, rd, tid);
-    double vr[TE], vi[TE], wr[TE], wi[TE];                                 // row li of the inverse, and of -W
+    double wr[16], wi[16];                   // columns 16 (lane / 16) + v of row li
+    const int cg16 = lane & 48;
+    if (last) {
 #pragma unroll
-    for (int v = 0; v < TE; ++v) {
-        const double2 a = S[li][c8 + 8 * v];
-        vr[v] = a.x;
-        vi[v] = a.y;
-        wr[v] = wi[v] = 0.0;
-    }
-    if (near) {
-        const int kend = 8 * (wv < 4 ? wv : 11 - wv) + 8;                  // the inverse is zero past its diagonal
+        for (int v = 0; v < 16; ++v) wr[v] = wi[v] = 0.0;
+        if (near) {
 #pragma unroll 2
-        for (int k = 0; k < kend; ++k) {
-            const double2 a = S[li][k];
-            const double2 na = make_double2(-a.x, -a.y);
+            for (int k = 0; k < 16 * wi4 + 16; ++k) {        // the inverse is zero past its diagonal
+                const double2 a = S[li][k], x = N[k][lane];
+                row_msub4<0>(wr, wi, x, a);
+                row_msub4<4>(wr, wi, x, a);
+                row_msub4<8>(wr, wi, x, a);
+                row_msub4<12>(wr, wi, x, a);
+            }
+        }
+    } else {
 #pragma unroll
-            for (int v = 0; v < TE; ++v) zfma(wr[v], wi[v], na, N[k][c8 + 8 * v]);
+        for (int v = 0; v < 16; ++v) {
+            const double2 a = S[li][cg16 + v];
+            wr[v] = a.x;
+            wi[v] = a.y;
         }
     }
+    float2 bx[2];                            // waves 4-7: the right-hand sides of places pair_col(h, lane)
+    if (!last)
+        rhs_pair(c, r0 + std::min(flip(pair_col(0, lane)), m - 1), r0 + std::min(flip(pair_col(1, lane)), m - 1), lane & 1, bx);
     __syncthreads();
-    float4(*red)[SB] = (float4(*)[SB])lds;                                 // [wave][row]: partial sums of the pair
-    double2(*vb)[CR] = (double2(*)[CR])(red + NWV);                        // the block's right-hand sides
-    double2(*yb)[CR] = vb + SB;                                            // y of the block before
-    float2 bx[CR];
-    rhs_row(c, grow, bx);
+    float4(*red)[SB] = (float4(*)[SB])lds;                                 // [wave][place]: partial sums of the pair
+    u64(*zs)[64] = (u64(*)[64])(red + NWV);                                // z, as rows_sum leaves it; set when written
+    if (last) zs[wv][lane] = UNSET;
     {
         float o[2 * CR];
         const int i = far_sum<float2, RM>(o, t, c, q, nfar, r0, m, wv, lane, order);
         red[wv][flip(i)] = make_float4(o[0], o[1], o[2], o[3]);
     }
     __syncthreads();
-    {                                    // the 8 waves' sums of row li meet in its 8 lanes
-        const float4 g = red[c8][li];
-        float h[2 * CR] = {g.x, g.y, g.z, g.w};
+    float2 y[2];
+    if (!last) {                             // z = inv(Op_qq) (b - the far sum): the 8 waves' parts meet in every wave
 #pragma unroll
-        for (int e = 0; e < 2 * CR; ++e) {
-            h[e] += dpp_of<0xB1>(h[e]);
-            h[e] += dpp_of<0x4E>(h[e]);
-            h[e] += dpp_of<0x141>(h[e]);
+        for (int h = 0; h < 2; ++h) {
+            const int k = pair_col(h, lane);
+            float2 g[NWV];
+#pragma unroll
+            for (int w = 0; w < NWV; ++w) g[w] = ((const float2 *)&red[w][k])[lane & 1];
+#pragma unroll
+            for (int st = 1; st < NWV; st *= 2)
+#pragma unroll
+                for (int w = 0; w + st < NWV; w += 2 * st) g[w] = tadd(g[w], g[w + st]);
+            y[h] = csel(flip(k) < m, tadd(bx[h], g[0]), make_float2(0.f, 0.f));
         }
-        if (c8 < CR)
-            vb[li][c8] = make_double2(inrow ? (double)((c8 ? bx[1].x : bx[0].x) + (c8 ? h[2] : h[0])) : 0.0,
-                                      inrow ? (double)((c8 ? bx[1].y : bx[0].y) + (c8 ? h[3] : h[1])) : 0.0);
+        __builtin_amdgcn_s_setprio(2);
+        const double z = rows_product(y, wr, wi);
+        __hip_atomic_store(&zs[wi4][lane], mark_safe((u64)__double_as_longlong(z), 0x7ff8000000000000ull),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);       // lane's word of z, marked as y's are
+        return;
     }
-    __syncthreads();
-    // the block before: lanes 0-15 of wave wv poll its rows 8 wv .. 8 wv + 7, first while z is formed
-    const long gk = kn + 8 * wv + lane / CR;
-    const bool need = near && lane < 8 * CR && gk < n;
-    float2 y = make_float2(0.f, 0.f);
-    auto attempt = [&]() { return take(c.dst + gk * CR + lane % CR, y); };
     __builtin_amdgcn_s_setprio(3);
-    if (need) y = fetch(c.dst + gk * CR + lane % CR);
-    __builtin_amdgcn_sched_barrier(0);
-    double ar[CR] = {0.0, 0.0}, ai[CR] = {0.0, 0.0};
-    rows_product(ar, ai, vr, vi, vb, c8);
-    __builtin_amdgcn_sched_barrier(0);       // y is looked at after the product
-    if (near) {
-        wave_wait<false>(is_set(y), c.abort, attempt);
-        if (lane < 8 * CR)
-            yb[8 * wv + lane / CR][lane % CR] = make_double2(need ? (double)y.x : 0.0, need ? (double)y.y : 0.0);
-        __syncthreads();
-        rows_product(ar, ai, wr, wi, yb, c8);
+    double x = 0.0;
+    if (near) {                              // y = z - W y of the block before
+        const long g0 = kn + pair_col(0, lane), g1 = kn + pair_col(1, lane);
+        const float2 *p0 = c.dst + std::min(g0, n - 1) * CR + (lane & 1), *p1 = c.dst + std::min(g1, n - 1) * CR + (lane & 1);
+        auto attempt = [&]() {
+            const bool a0 = take(p0, y[0]), a1 = take(p1, y[1]);
+            return a0 && a1;
+        };
+        wave_wait<true>(attempt(), c.abort, attempt);
+        y[0] = csel(g0 < n, y[0], make_float2(0.f, 0.f));
+        y[1] = csel(g1 < n, y[1], make_float2(0.f, 0.f));
+        x = rows_product(y, wr, wi);
     }
-    // the sums over the row's 8 lanes: each keeps one right-hand side (its lowest bit)
-    const bool b0 = c8 & 1;
-    double xr = (b0 ? ar[1] : ar[0]) + dpp_of<0xB1>(b0 ? ar[0] : ar[1]);
-    double xi = (b0 ? ai[1] : ai[0]) + dpp_of<0xB1>(b0 ? ai[0] : ai[1]);
-    xr += dpp_of<0x4E>(xr);
-    xi += dpp_of<0x4E>(xi);
-    // the two quads of a row: the half mirror pairs lane c8 with 7 - c8, the other right-hand side; a quad swap
-    // within it puts that right
-    xr += dpp_of<0x141>(dpp_of<0xB1>(xr));
-    xi += dpp_of<0x141>(dpp_of<0xB1>(xi));
-    if (inrow && c8 < CR) to_out(c, grow, orow, c8, make_float2((float)xr, (float)xi));
+    u64 z = UNSET;
+    auto got_z = [&]() {
+        z = __hip_atomic_load(&zs[wi4][lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return z != UNSET;
+    };
+    wave_wait<false>(got_z(), c.abort, got_z);
+    const unsigned f = __float_as_uint((float)(x + __longlong_as_double((long long)z)));
+    const auto both = __builtin_amdgcn_permlane16_swap(f, f, false, false);    // even column groups: (re, im)
+    if (inrow && !(lane & 16)) to_out(c, grow, orow, lane >> 5, make_float2(__uint_as_float(both[0]), __uint_as_float(both[1])));
 }
 
 // -- complex128 --
