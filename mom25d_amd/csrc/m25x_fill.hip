@@ -7,6 +7,8 @@
 // the tables, read through L2 (a table is 8192 x 32 B).
 #include "m25x_common.h"
 
+#include <type_traits>
+
 using namespace m25x;
 
 namespace {
@@ -275,73 +277,118 @@ struct DQuad {
     const double *P3, *W3, *P6, *W6;
 };
 
+// The separations of the parts extracted from table t, at most two, and their coefficients
+__device__ __forceinline__ int extracted(const DTab &T, int t, double (&d)[2], double2 (&cA)[2], double2 (&cq)[2])
+{
+    d[0] = d[1] = 0;
+    const int kd = T.kind[t];
+    if (kd == 0) {
+        cA[0] = T.cA[t]; cq[0] = T.cq[t];
+        if (!(T.dimg[t] > 0)) return 1;
+        d[1] = T.dimg[t]; cA[1] = T.cAi[t]; cq[1] = T.cqi[t];
+        return 2;
+    }
+    if (kd != 1) return 0;
+    d[0] = T.d[t]; cA[0] = T.cA[t]; cq[0] = T.cq[t];
+    return 1;
+}
+// the six moments of an extracted part at separation d of the pair (p, q)
+__device__ void static_part(const DMesh &g, const DQuad &qd, int p, int q, double d, double (&m)[6])
+{
+    const bool keep = rule_over_p(g.area[p], g.area[q], p, q);
+    const int po = keep ? p : q, qi = keep ? q : p;
+    double V[6];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const int nd = qd.tris[3 * qi + j];
+        V[2 * j] = qd.nodes[2 * nd]; V[2 * j + 1] = qd.nodes[2 * nd + 1];
+    }
+    double mo[2], ms[2];
+    offplane_one(V, qd.P6 + 12 * (size_t)po, qd.W6 + 6 * (size_t)po, d, m[0], mo, ms, m[5]);
+    m[1] = keep ? mo[0] : ms[0]; m[2] = keep ? mo[1] : ms[1];
+    m[3] = keep ? ms[0] : mo[0]; m[4] = keep ? ms[1] : mo[1];
+}
+// stat: the extracted parts' moments of every pair (geometry and separations only), 2 x 6 doubles
+__global__ __launch_bounds__(256) void k_near_static(DMesh g, DTab T, DQuad qd, const int *P, const int *Q, long n,
+                                                     double *stat)
+{
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int p = P[i], q = Q[i];
+    double d[2], m[6];
+    double2 cA[2], cq[2];
+    const int next = extracted(T, T.tab[g.lt[p] * T.L + g.lt[q]], d, cA, cq);
+    for (int k = 0; k < next; ++k) {
+        static_part(g, qd, p, q, d[k], m);
+#pragma unroll
+        for (int j = 0; j < 6; ++j) stat[12 * (size_t)i + 6 * k + j] = m[j];
+    }
+}
+
 // One thread a near pair: the smooth rest by 3 x 3 (same interface) or 6 x 6 (cross) quadrature, the extracted
-// parts analytically (kept in stat across frequencies), less the centroid value the far fill put there
-// (mom25d_core.cpp:417-476). M: n x 7 complex128 (M0, Mox, Moy, Msx, Msy, Mrr, Mq).
-__global__ __launch_bounds__(256) void k_near_moments(DMesh g, DTab T, DQuad qd, const int *P, const int *Q, long n,
-                                                      double *stat, int stat_ready, double2 *M, double2 *qcorr)
+// parts analytically (KEPT: from stat, k_near_static's, kept across frequencies), less the centroid value the far fill
+// put there (mom25d_core.cpp:417-476). M: n x 7 complex128 (M0, Mox, Moy, Msx, Msy, Mrr, Mq). The lookups' latency
+// bounds it: with the analytic parts in this kernel a thread had 194 registers, two waves a SIMD, and its lookups
+// came one at a time. 1.5 million pairs (7799 unknowns): 345 -> 259 us with the
+// caches warm.
+template <bool KEPT>
+__global__ __launch_bounds__(256, KEPT ? 4 : 2) void k_near_moments(DMesh g, DTab T, DQuad qd, const int *P, const int *Q, long n,
+                                                      const double *stat, double2 *M, double2 *qcorr)
 {
     const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int p = P[i], q = Q[i];
     const int la = g.lt[p], lb = g.lt[q];
     const int t = T.tab[la * T.L + lb];
-    const bool same = la == lb;
-    const int np = same ? 3 : 6;
-    const double *Pa = same ? qd.P3 + 6 * (size_t)p : qd.P6 + 12 * (size_t)p;
-    const double *Pb = same ? qd.P3 + 6 * (size_t)q : qd.P6 + 12 * (size_t)q;
-    const double *Wa = same ? qd.W3 + 3 * (size_t)p : qd.W6 + 6 * (size_t)p;
-    const double *Wb = same ? qd.W3 + 3 * (size_t)q : qd.W6 + 6 * (size_t)q;
     double2 M0 = {0, 0}, Mox = {0, 0}, Moy = {0, 0}, Msx = {0, 0}, Msy = {0, 0}, Mrr = {0, 0}, Mq = {0, 0};
-    for (int a = 0; a < np; ++a) {
-        const double pax = Pa[2 * a], pay = Pa[2 * a + 1], wa = Wa[a];
+    auto smooth = [&](auto npc, const double *Pp, const double *Wp) __attribute__((always_inline)) {
+        constexpr int np = decltype(npc)::value;
+        double qx[np], qy[np], qw[np];
+#pragma unroll
         for (int b = 0; b < np; ++b) {
-            const double pbx = Pb[2 * b], pby = Pb[2 * b + 1];
-            const double dx = pax - pbx, dy = pay - pby;
-            double2 ga, gq;
-            tab_rest(T, t, sqrt(dx * dx + dy * dy), ga, gq);
-            const double wt = wa * Wb[b];
-            ga = cscale(ga, wt); gq = cscale(gq, wt);
-            M0 = cadd(M0, ga);
-            Mox = cadd(Mox, cscale(ga, pax)); Moy = cadd(Moy, cscale(ga, pay));
-            Msx = cadd(Msx, cscale(ga, pbx)); Msy = cadd(Msy, cscale(ga, pby));
-            Mrr = cadd(Mrr, cscale(ga, pax * pbx + pay * pby));
-            Mq = cadd(Mq, gq);
+            qx[b] = Pp[2 * np * (size_t)q + 2 * b];
+            qy[b] = Pp[2 * np * (size_t)q + 2 * b + 1];
+            qw[b] = Wp[np * (size_t)q + b];
         }
-    }
-    const bool keep = rule_over_p(g.area[p], g.area[q], p, q);
-    const int po = keep ? p : q, qi = keep ? q : p;
-    const int kd = T.kind[t];
-    int next = 0;
-    double dd[2] = {0, 0};
+#pragma unroll 1
+        for (int a = 0; a < np; ++a) {
+            const double pax = Pp[2 * np * (size_t)p + 2 * a], pay = Pp[2 * np * (size_t)p + 2 * a + 1];
+            const double wa = Wp[np * (size_t)p + a];
+#pragma unroll
+            for (int b0 = 0; b0 < np; b0 += 3) {
+                double2 ga[3], gq[3];                // three lookups in flight before the first is used
+#pragma unroll
+                for (int b = 0; b < 3; ++b) {
+                    const double dx = pax - qx[b0 + b], dy = pay - qy[b0 + b];
+                    tab_rest(T, t, sqrt(dx * dx + dy * dy), ga[b], gq[b]);
+                }
+#pragma unroll
+                for (int b = 0; b < 3; ++b) {
+                    const double wt = wa * qw[b0 + b], x = qx[b0 + b], y = qy[b0 + b];
+                    const double2 A = cscale(ga[b], wt);
+                    M0 = cadd(M0, A);
+                    Mox = cadd(Mox, cscale(A, pax)); Moy = cadd(Moy, cscale(A, pay));
+                    Msx = cadd(Msx, cscale(A, x)); Msy = cadd(Msy, cscale(A, y));
+                    Mrr = cadd(Mrr, cscale(A, pax * x + pay * y));
+                    Mq = cadd(Mq, cscale(gq[b], wt));
+                }
+            }
+        }
+    };
+    if (la == lb) smooth(std::integral_constant<int, 3>{}, qd.P3, qd.W3);
+    else smooth(std::integral_constant<int, 6>{}, qd.P6, qd.W6);
+    double dd[2];
     double2 cAs[2], cqs[2];
-    if (kd == 0) {
-        dd[0] = 0.0; cAs[0] = T.cA[t]; cqs[0] = T.cq[t]; next = 1;
-        if (T.dimg[t] > 0) { dd[1] = T.dimg[t]; cAs[1] = T.cAi[t]; cqs[1] = T.cqi[t]; next = 2; }
-    } else if (kd == 1) {
-        dd[0] = T.d[t]; cAs[0] = T.cA[t]; cqs[0] = T.cq[t]; next = 1;
-    }
-    for (int k = 0; k < next; ++k) {
+    const int next = extracted(T, t, dd, cAs, cqs);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        if (k >= next) break;
         double m[6];
-        double *sp = stat ? stat + 12 * (size_t)i + 6 * k : nullptr;
-        if (sp && stat_ready) {
+        if constexpr (KEPT) {
 #pragma unroll
-            for (int j = 0; j < 6; ++j) m[j] = sp[j];
+            for (int j = 0; j < 6; ++j) m[j] = stat[12 * (size_t)i + 6 * k + j];
         } else {
-            double V[6];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int nd = qd.tris[3 * qi + j];
-                V[2 * j] = qd.nodes[2 * nd]; V[2 * j + 1] = qd.nodes[2 * nd + 1];
-            }
-            double mro[2], mrs[2];
-            offplane_one(V, qd.P6 + 12 * (size_t)po, qd.W6 + 6 * (size_t)po, dd[k], m[0], keep ? mro : mrs,
-                         keep ? mrs : mro, m[5]);
-            m[1] = mro[0]; m[2] = mro[1]; m[3] = mrs[0]; m[4] = mrs[1];
-            if (sp) {
-#pragma unroll
-                for (int j = 0; j < 6; ++j) sp[j] = m[j];
-            }
+            static_part(g, qd, p, q, dd[k], m);
         }
         const double2 cA = cAs[k], cq = cqs[k];
         M0 = cadd(M0, cscale(cA, m[0])); Mox = cadd(Mox, cscale(cA, m[1])); Moy = cadd(Moy, cscale(cA, m[2]));
@@ -1063,8 +1110,16 @@ int m25x_near_moments(const m25x_mesh *g, const m25x_tables *tb, const m25x_quad
     if (n == 0) return M25X_OK;
     DQuad d{q->nodes, q->tris, q->P3, q->W3, q->P6, q->W6};
     TimedLaunch tl((hipStream_t)stream, M25X_K_NEAR_MOMENTS, M25X_C128, 7.0 * 16 * n, 0.0);
-    hipLaunchKernelGGL(k_near_moments, dim3(blocks(n, 256)), dim3(256), 0, (hipStream_t)stream, dmesh(g), dtab(tb),
-                       d, P, Q, n, stat, stat_ready, (double2 *)M, (double2 *)qcorr);
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 grid(blocks(n, 256));
+    if (stat) {
+        if (!stat_ready) hipLaunchKernelGGL(k_near_static, grid, dim3(256), 0, s, dmesh(g), dtab(tb), d, P, Q, n, stat);
+        hipLaunchKernelGGL(k_near_moments<true>, grid, dim3(256), 0, s, dmesh(g), dtab(tb), d, P, Q, n, (const double *)stat,
+                           (double2 *)M, (double2 *)qcorr);
+    } else {
+        hipLaunchKernelGGL(k_near_moments<false>, grid, dim3(256), 0, s, dmesh(g), dtab(tb), d, P, Q, n,
+                           (const double *)nullptr, (double2 *)M, (double2 *)qcorr);
+    }
     return check_launch("near_moments");
 }
 

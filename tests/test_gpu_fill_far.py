@@ -32,3 +32,25 @@ def test_fill_far_is_far_block(gpu, order, dt):
         m, n = torch.triu_indices(Ne, Ne, device=Z.device)
         assert torch.equal(Z[m, n], want[m, n]), Ne
         assert torch.equal(Z, Z.T), Ne
+
+
+def test_near_moments_with_kept_parts(gpu):
+    """The pairs' moments with the extracted parts kept (computed at the first call, read at the next) and without a
+    store for them: the same bits, whichever way the parts come; and a store is filled again when they change."""
+    from mom25d_amd import boards
+    from mom25d_amd.sim import Simulation
+    dv, w = gpu, 2 * np.pi * 2.3e9
+    for board in (boards.microstrip, boards.seeded_board):
+        st, shapes, ports, vias, kw = board(dmax=3e-3, ncross=2)
+        sim = Simulation(st, shapes, ports, vias, verbose=False, **kw)
+        fo = sim.fast
+        fo.setup(2.3e9)
+        want = dv.near_moments(fo.mesh, fo.tabs, fo.plan, w, stat=False)
+        for kept in (False, True, True):
+            assert fo.plan.stat_ready == kept
+            for a, b in zip(dv.near_moments(fo.mesh, fo.tabs, fo.plan, w), want):
+                assert torch.equal(torch.view_as_real(a), torch.view_as_real(b)), (board.__name__, kept)
+        fo.plan.stat.fill_(float('nan'))
+        fo.plan.stat_kind = None
+        for a, b in zip(dv.near_moments(fo.mesh, fo.tabs, fo.plan, w), want):
+            assert torch.equal(torch.view_as_real(a), torch.view_as_real(b)), board.__name__
