@@ -156,140 +156,215 @@ extern "C" int m25x_zgemm_nk_batched(int nitems, const m25x_mv_item *h, const m2
 // ---- classical Gram-Schmidt, twice, for the batched GMRES ------------------------------------------------------
 // V: (j + 1) basis vectors, each n x k complex128 row-major (vector i at V + i n k); w: n x k. Per column c:
 // h1 = V^H w, w1 = w - V h1, h2 = V^H w1, w2 = w1 - V h2, h = h1 + h2, nrm = |w2|, V[j + 1] = w2 / nrm (nrm = 0: w2).
-// Sums over rows in fixed blocks, then over blocks in order: the result does not depend on timing.
+// Sums over rows in fixed blocks, then over blocks in a fixed order: the result does not depend on timing.
+//
+// Four launches, each waiting for the sums of the one before; the basis (3 MB at n = 7799, k = 4, six vectors) stays in
+// the caches, so what counts is each launch's chain of memory round trips. Rows are spread so that a thread has one
+// up to n k = 32 768 elements (column = the thread's low bits, so reads are consecutive), the basis is read
+// GS_CH vectors at a time with the loads in flight together, a wave's GS_CH sums are folded by halving (each exchange
+// sends the half that the partner keeps: 8 exchanges for 8 sums over 16 lanes, not 32), and every block of the next
+// launch adds the blocks' partial sums itself instead of a launch of one workgroup between them. Seven launches with
+// one vector a round trip took 38.5 us at n = 7799, k = 4 on six vectors and 94 on 30, these take 18.1 and 34.2;
+// at n = 905 27.9 and 16.6 on six, at n = 20 000 348 and 59 on 30.
 namespace {
 
-constexpr int GS_B = 64;                 // row blocks
-constexpr int GS_T = 256;                // threads a block: 8 columns x 32 row lanes
+constexpr int GS_B = 128;                // row blocks at most
+constexpr int GS_T = 256;                // threads a block: KP columns x GS_T / KP row lanes
 constexpr int GS_MAXV = 64;              // basis vectors at most
+constexpr int GS_CH = 8;                 // basis vectors read at a time
 
-// partial dots of the rows of block blockIdx.x: P[b][i][c] = sum_r conj(V[i][r][c]) x[r][c], for i < nv; with
-// upd: first x -= sum_i V[i] h[i] (h from H), stored back. The dots run over the basis in chunks of GS_CH vectors.
-constexpr int GS_CH = 32;
-template <bool UPD>
-__global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V, long n, int k, int nv,
-                                                 double2 *__restrict__ x, const double2 *__restrict__ H,
-                                                 double2 *__restrict__ P)
+// h[i k + c] = sum over the blocks' partial sums P[b][i k + c]: m = nv k entries, up to GS_T / m threads an entry.
+__device__ inline void gs_sum(const double2 *__restrict__ P, int nb, int m, double2 *h, double2 *part)
 {
-    __shared__ double2 red[GS_T / 64][GS_CH][8];
-    const int c = threadIdx.x & 7, rl = threadIdx.x >> 3, wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const long rows = (n + GS_B - 1) / GS_B, r0 = blockIdx.x * rows, r1 = r0 + rows < n ? r0 + rows : n;
-    if (UPD && c < k)                              // each thread updates the rows it reads below
-        for (long r = r0 + rl; r < r1; r += GS_T / 8) {
-            double2 xv = x[r * k + c];
-            for (int i = 0; i < nv; ++i) {
-                const double2 v = V[(long)i * n * k + r * k + c], h = H[i * k + c];
-                xv.x -= v.x * h.x - v.y * h.y;
-                xv.y -= v.x * h.y + v.y * h.x;
+    const int t = threadIdx.x, S = m < GS_T ? GS_T / m : 1;
+    for (int e0 = 0; e0 < m; e0 += GS_T) {
+        const int e = S > 1 ? t % m : e0 + t, sl = S > 1 ? t / m : 0;
+        double2 s = make_double2(0, 0);
+        if (e < m && sl < S) {
+#pragma unroll 8
+            for (int b = sl; b < nb; b += S) {
+                const double2 p = P[(long)b * m + e];
+                s.x += p.x; s.y += p.y;
             }
-            x[r * k + c] = xv;
+            if (S > 1) part[t] = s;
+            else h[e] = s;
         }
+    }
+    __syncthreads();
+    if (S > 1) {
+        if (t < m) {
+            double2 s = part[t];
+            for (int l = 1; l < S; ++l) { s.x += part[l * m + t].x; s.y += part[l * m + t].y; }
+            h[t] = s;
+        }
+        __syncthreads();
+    }
+}
+
+// The vectors i0 .. i0 + GS_CH - 1 at element e, the last one repeated past nv (its uses are then dropped or zero).
+__device__ inline void gs_load(double2 (&v)[GS_CH], const double2 *__restrict__ V, long nk, long e, int i0, int nv)
+{
+#pragma unroll
+    for (int u = 0; u < GS_CH; ++u) v[u] = V[(long)(i0 + u < nv ? i0 + u : nv - 1) * nk + e];
+}
+
+// x - sum_i V[i] h[i] at element e of column c
+__device__ inline double2 gs_minus(double2 x, const double2 *__restrict__ V, long nk, long e, int c, int k, int nv,
+                                   const double2 *h)
+{
     for (int i0 = 0; i0 < nv; i0 += GS_CH) {
-        double2 acc[GS_CH];
+        double2 v[GS_CH];
+        gs_load(v, V, nk, e, i0, nv);
 #pragma unroll
-        for (int i = 0; i < GS_CH; ++i) acc[i] = make_double2(0, 0);
+        for (int u = 0; u < GS_CH; ++u)
+            if (i0 + u < nv) {
+                const double2 hv = h[(i0 + u) * k + c];
+                x.x -= v[u].x * hv.x - v[u].y * hv.y;
+                x.y -= v[u].x * hv.y + v[u].y * hv.x;
+            }
+    }
+    return x;
+}
+
+// Partial dots of block blockIdx.x's rows: P[b][i k + c] = sum_r conj(V[i][r][c]) x[r][c]. UPD: x -= V h first, h the
+// sum of the last pass's partial sums Pin; block 0 stores h to H.
+template <int KP, bool UPD>
+__global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V, long n, int k, int nv,
+                                                 double2 *__restrict__ x, const double2 *__restrict__ Pin,
+                                                 double2 *__restrict__ H, double2 *__restrict__ P)
+{
+    __shared__ double2 red[GS_MAXV][GS_T / 64][KP];
+    __shared__ double2 h[UPD ? GS_MAXV * KP : 1], part[UPD ? GS_T : 1];
+    constexpr int RL = GS_T / KP;
+    const int t = threadIdx.x, c = t % KP, rl = t / KP, wv = t >> 6, lane = t & 63;
+    const long nk = n * k, step = (long)gridDim.x * RL;
+    if (UPD) {
+        gs_sum(Pin, gridDim.x, nv * k, h, part);
+        if (blockIdx.x == 0)
+            for (int e = t; e < nv * k; e += GS_T) H[e] = h[e];
+        if (c < k)                               // each thread updates the elements it reads below
+            for (long r = (long)blockIdx.x * RL + rl; r < n; r += step)
+                x[r * k + c] = gs_minus(x[r * k + c], V, nk, r * k + c, c, k, nv, h);
+    }
+    for (int i0 = 0; i0 < nv; i0 += GS_CH) {
+        double2 a[GS_CH];
+#pragma unroll
+        for (int u = 0; u < GS_CH; ++u) a[u] = make_double2(0, 0);
         if (c < k)
-            for (long r = r0 + rl; r < r1; r += GS_T / 8) {
+            for (long r = (long)blockIdx.x * RL + rl; r < n; r += step) {
                 const double2 xv = x[r * k + c];
+                double2 v[GS_CH];
+                gs_load(v, V, nk, r * k + c, i0, nv);
 #pragma unroll
-                for (int i = 0; i < GS_CH; ++i)
-                    if (i0 + i < nv) {
-                        const double2 v = V[(long)(i0 + i) * n * k + r * k + c];
-                        acc[i].x += v.x * xv.x + v.y * xv.y;
-                        acc[i].y += v.x * xv.y - v.y * xv.x;
-                    }
+                for (int u = 0; u < GS_CH; ++u) {
+                    a[u].x += v[u].x * xv.x + v[u].y * xv.y;
+                    a[u].y += v[u].x * xv.y - v[u].y * xv.x;
+                }
             }
-        // the eight row lanes of a wave (lane bits 3-5), then the four waves
+        // the wave's row lanes: three halvings leave one sum a lane, vector 4 b0 + 2 b1 + b2 of its row lane's low bits
 #pragma unroll
-        for (int i = 0; i < GS_CH; ++i)
-            if (i0 + i < nv) {
-                double sx = acc[i].x, sy = acc[i].y;
+        for (int s = 0; s < 3; ++s) {
+            const int half = 4 >> s, o = KP << s;
+            const bool up = lane & o;
 #pragma unroll
-                for (int o = 8; o < 64; o <<= 1) { sx += __shfl_xor(sx, o); sy += __shfl_xor(sy, o); }
-                if (lane < 8) red[wv][i][c] = make_double2(sx, sy);
+            for (int u = 0; u < half; ++u) {
+                const double2 keep = up ? a[u + half] : a[u], send = up ? a[u] : a[u + half];
+                a[u].x = keep.x + __shfl_xor(send.x, o);
+                a[u].y = keep.y + __shfl_xor(send.y, o);
             }
-        __syncthreads();
-        const int m = nv - i0 < GS_CH ? nv - i0 : GS_CH;
-        for (int idx = threadIdx.x; idx < m * k; idx += GS_T) {
-            const int i = idx / k, cc = idx % k;
-            double2 s = make_double2(0, 0);
-            for (int l = 0; l < GS_T / 64; ++l) { s.x += red[l][i][cc].x; s.y += red[l][i][cc].y; }
-            P[((long)blockIdx.x * GS_MAXV + i0 + i) * 8 + cc] = s;
         }
-        __syncthreads();
+#pragma unroll
+        for (int o = KP << 3; o < 64; o <<= 1) { a[0].x += __shfl_xor(a[0].x, o); a[0].y += __shfl_xor(a[0].y, o); }
+        const int b = lane / KP, i = i0 + ((b & 1) << 2 | (b & 2) | (b >> 2 & 1));
+        if (lane < 8 * KP && i < nv) red[i][wv][c] = a[0];
+    }
+    __syncthreads();
+    for (int e = t; e < nv * k; e += GS_T) {
+        const double2 *q = &red[e / k][0][e % k];
+        double2 s = q[0];
+#pragma unroll
+        for (int w = 1; w < GS_T / 64; ++w) { s.x += q[w * KP].x; s.y += q[w * KP].y; }
+        P[(long)blockIdx.x * nv * k + e] = s;
     }
 }
 
-// H[i][c] = sum_b P[b][i][c] (in block order); with acc: Hs[i][c] += H[i][c] as well
-__global__ void k_gs_sum(const double2 *__restrict__ P, int k, int nv, double2 *__restrict__ H, double2 *Hs, int first)
-{
-    const int idx = threadIdx.x;
-    if (idx >= nv * k) return;
-    const int i = idx / k, c = idx % k;
-    double2 s = make_double2(0, 0);
-    for (int b = 0; b < GS_B; ++b) {
-        const double2 p = P[((long)b * GS_MAXV + i) * 8 + c];
-        s.x += p.x; s.y += p.y;
-    }
-    H[i * k + c] = s;
-    if (first) Hs[i * k + c] = s;
-    else { Hs[i * k + c].x += s.x; Hs[i * k + c].y += s.y; }
-}
-
-// x -= V h (h from H), stored back; Q[b][c] = partial |x|^2
+// x -= V h2, h2 the sum of the partial sums Pin; Q[b][c] = partial |x|^2; block 0 adds h2 to H.
+template <int KP>
 __global__ __launch_bounds__(GS_T) void k_gs_final(const double2 *__restrict__ V, long n, int k, int nv,
-                                                  double2 *__restrict__ x, const double2 *__restrict__ H,
-                                                  double *__restrict__ Q)
+                                                  double2 *__restrict__ x, const double2 *__restrict__ Pin,
+                                                  double2 *__restrict__ H, double *__restrict__ Q)
 {
-    __shared__ double red[GS_T / 8][8];
-    const int c = threadIdx.x & 7, rl = threadIdx.x >> 3;
-    const long rows = (n + GS_B - 1) / GS_B, r0 = blockIdx.x * rows, r1 = r0 + rows < n ? r0 + rows : n;
+    __shared__ double2 h[GS_MAXV * KP], part[GS_T];
+    __shared__ double red[GS_T / 64][KP];
+    constexpr int RL = GS_T / KP;
+    const int t = threadIdx.x, c = t % KP, rl = t / KP;
+    gs_sum(Pin, gridDim.x, nv * k, h, part);
+    if (blockIdx.x == 0)
+        for (int e = t; e < nv * k; e += GS_T) { H[e].x += h[e].x; H[e].y += h[e].y; }
     double q = 0;
     if (c < k)
-        for (long r = r0 + rl; r < r1; r += GS_T / 8) {
-            double2 xv = x[r * k + c];
-            for (int i = 0; i < nv; ++i) {
-                const double2 v = V[(long)i * n * k + r * k + c], h = H[i * k + c];
-                xv.x -= v.x * h.x - v.y * h.y;
-                xv.y -= v.x * h.y + v.y * h.x;
-            }
+        for (long r = (long)blockIdx.x * RL + rl; r < n; r += (long)gridDim.x * RL) {
+            const double2 xv = gs_minus(x[r * k + c], V, n * k, r * k + c, c, k, nv, h);
             x[r * k + c] = xv;
             q += xv.x * xv.x + xv.y * xv.y;
         }
-    red[rl][c] = q;
+#pragma unroll
+    for (int o = KP; o < 64; o <<= 1) q += __shfl_xor(q, o);
+    if ((t & 63) < KP) red[t >> 6][c] = q;
     __syncthreads();
-    if (threadIdx.x < k) {
-        double s = 0;
-        for (int l = 0; l < GS_T / 8; ++l) s += red[l][threadIdx.x];
-        Q[blockIdx.x * 8 + threadIdx.x] = s;
+    if (t < k) {
+        double s = red[0][t];
+        for (int w = 1; w < GS_T / 64; ++w) s += red[w][t];
+        Q[blockIdx.x * KP + t] = s;
     }
 }
 
-// hcol[nv][c] = |x| (real); V[nv] = x / |x|
-__global__ void k_gs_norm(const double *__restrict__ Q, int k, int nv, double2 *__restrict__ hcol)
+// H[nv][c] = |x| (real, block 0), out = x / |x|; Q: nb blocks' partial |x|^2.
+template <int KP>
+__global__ __launch_bounds__(GS_T) void k_gs_scale(const double2 *__restrict__ x, long n, int k, int nv, int nb,
+                                                  const double *__restrict__ Q, double2 *__restrict__ H,
+                                                  double2 *__restrict__ out)
 {
-    const int c = threadIdx.x;
-    if (c >= k) return;
-    double s = 0;
-    for (int b = 0; b < GS_B; ++b) s += Q[b * 8 + c];
-    hcol[nv * k + c] = make_double2(sqrt(s), 0);
+    __shared__ double red[GS_T / 64][KP];
+    constexpr int RL = GS_T / KP;
+    const int t = threadIdx.x, c = t % KP, rl = t / KP;
+    const long r = (long)blockIdx.x * RL + rl;
+    const bool in = c < k && r < n;
+    const double2 xv = in ? x[r * k + c] : make_double2(0, 0);
+    double q = 0;
+    if (c < k)
+        for (int b = rl; b < nb; b += RL) q += Q[b * KP + c];
+#pragma unroll
+    for (int o = KP; o < 64; o <<= 1) q += __shfl_xor(q, o);
+    if ((t & 63) < KP) red[t >> 6][c] = q;
+    __syncthreads();
+    double s = red[0][c];
+    for (int w = 1; w < GS_T / 64; ++w) s += red[w][c];
+    const double nr = sqrt(s), sc = nr > 0 ? 1.0 / nr : 1.0;
+    if (blockIdx.x == 0 && t < k) H[nv * k + t] = make_double2(nr, 0);
+    if (in) out[r * k + c] = make_double2(xv.x * sc, xv.y * sc);
 }
 
-__global__ void k_gs_scale(const double2 *__restrict__ x, long nk, int k, int nv, const double2 *__restrict__ hcol,
-                           double2 *__restrict__ out)
+template <int KP>
+void cgs2(const double2 *V, long n, int k, int nv, double2 *x, double2 *H, double2 *out, double2 *P, hipStream_t s)
 {
-    const long idx = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (idx >= nk) return;
-    const double nr = hcol[nv * k + (int)(idx % k)].x;
-    const double sc = nr > 0 ? 1.0 / nr : 1.0;
-    out[idx] = make_double2(x[idx].x * sc, x[idx].y * sc);
+    const long full = (n + GS_T / KP - 1) / (GS_T / KP);
+    const int nb = (int)std::min<long>(full, GS_B);
+    double2 *P2 = P + (size_t)GS_B * GS_MAXV * 8;
+    double *Q = (double *)(P2 + (size_t)GS_B * GS_MAXV * 8);
+    hipLaunchKernelGGL((k_gs_dots<KP, false>), dim3(nb), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)nullptr,
+                       (double2 *)nullptr, P);
+    hipLaunchKernelGGL((k_gs_dots<KP, true>), dim3(nb), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)P, H, P2);
+    hipLaunchKernelGGL(k_gs_final<KP>, dim3(nb), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)P2, H, Q);
+    hipLaunchKernelGGL(k_gs_scale<KP>, dim3((unsigned)full), dim3(GS_T), 0, s, (const double2 *)x, n, k, nv, nb,
+                       (const double *)Q, H, out);
 }
 
 }  // namespace
 
 extern "C" size_t m25x_cgs2_work_bytes(void)
 {
-    return (size_t)GS_B * GS_MAXV * 8 * sizeof(double2) + GS_MAXV * 8 * sizeof(double2) + GS_B * 8 * sizeof(double);
+    return 2 * (size_t)GS_B * GS_MAXV * 8 * sizeof(double2) + GS_B * 8 * sizeof(double);
 }
 
 extern "C" int m25x_cgs2(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
@@ -299,18 +374,8 @@ extern "C" int m25x_cgs2(const double *V, long n, int k, int nv, double *w, doub
         return fail(M25X_EINVAL, "cgs2: bad arguments (1 <= k <= 8, 1 <= nv <= %d)", GS_MAXV - 1);
     if (work_bytes < m25x_cgs2_work_bytes()) return fail(M25X_EINVAL, "cgs2: workspace too small");
     hipStream_t s = (hipStream_t)stream;
-    const double2 *Vc = (const double2 *)V;
-    double2 *x = (double2 *)w, *H = (double2 *)hcol;
-    double2 *P = (double2 *)work, *h = P + (size_t)GS_B * GS_MAXV * 8;
-    double *Q = (double *)(h + GS_MAXV * 8);
     TimedLaunch tl(s, M25X_K_CGS2, M25X_C128, 16.0 * n * k * (2.0 * nv + 3), 16.0 * n * k * nv);
-    hipLaunchKernelGGL(k_gs_dots<false>, dim3(GS_B), dim3(GS_T), 0, s, Vc, n, k, nv, x, (const double2 *)nullptr, P);
-    hipLaunchKernelGGL(k_gs_sum, dim3(1), dim3(GS_MAXV * 8), 0, s, (const double2 *)P, k, nv, h, H, 1);
-    hipLaunchKernelGGL(k_gs_dots<true>, dim3(GS_B), dim3(GS_T), 0, s, Vc, n, k, nv, x, (const double2 *)h, P);
-    hipLaunchKernelGGL(k_gs_sum, dim3(1), dim3(GS_MAXV * 8), 0, s, (const double2 *)P, k, nv, h, H, 0);
-    hipLaunchKernelGGL(k_gs_final, dim3(GS_B), dim3(GS_T), 0, s, Vc, n, k, nv, x, (const double2 *)h, Q);
-    hipLaunchKernelGGL(k_gs_norm, dim3(1), dim3(64), 0, s, (const double *)Q, k, nv, H);
-    hipLaunchKernelGGL(k_gs_scale, dim3((unsigned)((n * k + 255) / 256)), dim3(256), 0, s, (const double2 *)x, n * k,
-                       k, nv, (const double2 *)H, (double2 *)vnext);
+    const auto run = k == 1 ? cgs2<1> : k == 2 ? cgs2<2> : k <= 4 ? cgs2<4> : cgs2<8>;
+    run((const double2 *)V, n, k, nv, (double2 *)w, (double2 *)hcol, (double2 *)vnext, (double2 *)work, s);
     return check_launch("cgs2");
 }
