@@ -344,8 +344,8 @@ typedef struct m25x_lu_item {
 int m25x_getrf_batched(int dtype, int nitems, const m25x_lu_item *items_host, const m25x_lu_item *items_dev,
                        void *stream);
 
-/* One solve of the batch: as m25x_getrs's arguments (perm required: m25x_getrf's), nrhs <= 4 (complex128) or 8
- * (complex64), work: m25x_getrs_work_bytes(dtype, n, nrhs) bytes of its own. */
+/* One solve of the batch: as m25x_getrs's arguments (perm required: m25x_getrf's, 1 <= nrhs <= 8), work:
+ * m25x_getrs_work_bytes(dtype, n, ldb) bytes of its own. */
 typedef struct m25x_rs_item {
     const void *LU;
     long n, lda;
@@ -418,6 +418,14 @@ size_t m25x_cgs2_work_bytes(void);
  * gmres_batched (src/mom25d/fast.py:1437-1500, modified Gram-Schmidt: the same basis to rounding). */
 int m25x_cgs2(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
               size_t work_bytes, void *stream);
+
+/* dst[i][c] = r[i] src[i][c] (r: n doubles, NULL for 1) for n x k complex arrays of the given dtypes (M25X_C64,
+ * M25X_C128; leading dimensions lds, ldd >= k in elements; not overlapping): the product in FP64, rounded once to
+ * dst's type. The solves' right-hand sides and answers between the refinement's FP64 and a complex64 factor, with
+ * the row scaling of a reused factor (src/mom25d/fast.py:996-1084). No entry is read when n or k
+ * is zero. */
+int m25x_cast_rows(int src_dtype, const void *src, long lds, int dst_dtype, void *dst, long ldd, long n, long k,
+                   const double *r, void *stream);
 
 #ifdef __cplusplus
 }

@@ -478,9 +478,27 @@ def getrf(Z, pivot='tournament'):
     return Factor(Z, ipiv, perm, info)
 
 
-def getrs(F, B, trans=1):
+def cast_rows(src, dtype, scale=None, out=None):
+    """scale[:, None] * src (scale real float64 (n,) or None) as a contiguous tensor of dtype, or into out (columns of
+    a row-major tensor): the product in FP64, one rounding. src: (n, k) complex, any strides; never src itself."""
+    src = src.resolve_conj().resolve_neg()
+    if src.dtype not in (c64, c128):
+        src = src.to(c128)
+    if src.stride(1) != 1 or src.stride(0) < src.shape[1]:
+        src = src.contiguous()
+    if out is None:
+        out = torch.empty(src.shape, dtype=dtype, device=src.device)
+    n, k = src.shape
+    code = lambda t: L.C128 if t.dtype == c128 else L.C64
+    L.call('m25x_cast_rows', code(src), ptr(src), max(src.stride(0), k), code(out), ptr(out), max(out.stride(0), k), n, k,
+           ptr(scale), stream())
+    return out
+
+
+def getrs(F, B, trans=1, scale=None):
     """X with Z X = B (trans 1) or Z^T X = B (trans 0), B (n,) or (n, k) complex (any dtype); the solve in the
-    factor's precision, complex128 out. Columns are solved 8 at a time."""
+    factor's precision, complex128 out. Columns are solved 8 at a time. scale (n,) float64: diag(scale) times the
+    solve of diag(scale) B, the products in FP64."""
     one = B.dim() == 1
     B = B.reshape(B.shape[0], -1)
     n, k = B.shape
@@ -488,13 +506,13 @@ def getrs(F, B, trans=1):
     dt = L.C128 if F.dtype == c128 else L.C64
     for c0 in range(0, k, 8):
         kc = min(8, k - c0)
-        X = B[:, c0:c0 + kc].to(F.dtype, copy=True).contiguous()      # solved in place: never the caller's B
+        X = cast_rows(B[:, c0:c0 + kc], F.dtype, scale)               # solved in place: never the caller's B
         wb = L.lib().m25x_getrs_work_bytes(dt, n, kc)
         work = torch.empty(wb, dtype=torch.uint8, device=B.device)
         L.call('m25x_getrs', dt, ptr(F.LU), n, F.LU.stride(0), ptr(F.ipiv), ptr(F.perm), ptr(X), kc, kc,
                int(trans), ptr(work), wb, stream())
         _solve_fault(B.device).bitwise_or_(work[wb - 256:wb - 252].view(torch.int32))   # the call's abort word
-        out[:, c0:c0 + kc] = X.to(c128)
+        cast_rows(X, c128, scale, out[:, c0:c0 + kc])
     return out[:, 0] if one else out
 
 
@@ -583,7 +601,7 @@ class BatchSolve:
         each item the (first column, columns) in R instead of self.cols (columns 0 skip the item)."""
         cols = subset or self.cols
         nmax, k = R.shape
-        X = R.to(self.dtype, copy=True).contiguous()            # solved in place: never the caller's R
+        X = cast_rows(R, self.dtype)                            # solved in place: never the caller's R
         items = []
         for F, w, (c0, kc) in zip(self.factors, self.work, cols):
             for p in range(0, kc, 8):
@@ -596,7 +614,7 @@ class BatchSolve:
             L.call('m25x_getrs_batched', self.code, len(items), host, ptr(dev_tab), int(trans), ptr(self.status),
                    stream())
             _solve_fault(X.device).bitwise_or_(self.status)
-        return X.to(c128)
+        return cast_rows(X, c128)
 
 
 def zgemm_nk_batched(Zs, V, cols, out=None):

@@ -281,11 +281,11 @@ class FastOperator:
         k = self._reusable(f)
         if k is not None:
             f0, F0, d0, tf0 = k
-            r = (d0 / dsc)[:, None]
+            r = d0 / dsc
             cap = int(np.clip(0.8 * tf0 / max(self._t_iter or 1e-3, 1e-6), *REUSE_ITER))
             with sim.log.timer('refinement (GMRES, reused factorisation)', f"the one of {f0 / 1e9:.4g} GHz, at most {cap}"):
                 t = time.time()
-                Y, ok, rel = self._refine(A, B, lambda R: r * dv.getrs(F0, r * R, trans=1), cap, 1,
+                Y, ok, rel = self._refine(A, B, lambda R: dv.getrs(F0, R, trans=1, scale=r), cap, 1,
                                           x0=self._guess(dsc, B))
                 self._t_iter = (time.time() - t) / max(1, max(self.iters, default=1))
             self._reach_learn(abs(np.log(f / f0)), ok, self.iters, cap)

@@ -40,3 +40,50 @@ def test_step_against_numpy(gpu, n, k, nv):
     assert np.abs(hg - h).max() <= tol and np.abs(Wg - w).max() <= tol
     assert np.abs(Vg[nv] * h[nv].real - w).max() <= 2 * tol
     assert np.array_equal(Vg[:nv], V[:nv])
+
+
+@pytest.mark.parametrize("dst", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("form", ["c128", "c64", "columns", "transposed", "conj", "real", "repeated", "one row"])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_cast_rows_is_product_and_conversion(gpu, form, dst, scaled):
+    """Bit for bit the product and the conversion that it stands for, whatever the source's type and strides."""
+    dv = gpu
+    torch.manual_seed(3)
+    dev = dv.device()
+    full = torch.randn(333, 9, dtype=torch.complex128, device=dev)
+    src = dict(c128=full, c64=full.to(torch.complex64), columns=full[:, 2:5], transposed=full.t(), conj=full.conj()[:, 1:],
+               real=full.real, repeated=full[5:6].expand(40, 9))
+    src['one row'] = full[7:8, 3:]
+    src = src[form]
+    r = torch.rand(src.shape[0], dtype=torch.float64, device=dev) + 0.5 if scaled else None
+    want = ((src.to(torch.complex128) if r is None else r[:, None] * src.to(torch.complex128)).to(dst)).contiguous()
+    keep = src.clone()
+    wide = torch.zeros((src.shape[0], src.shape[1] + 3), dtype=dst, device=dev)
+    got = dv.cast_rows(src, dst, r)
+    dv.cast_rows(src, dst, r, wide[:, 2:2 + src.shape[1]])
+    assert got.dtype == dst and torch.equal(got, want) and torch.equal(wide[:, 2:-1], want)
+    assert not wide[:, :2].any() and not wide[:, -1:].any() and torch.equal(src, keep)
+
+
+@pytest.mark.parametrize("k", [1, 4, 11])
+@pytest.mark.parametrize("dtype", [torch.complex64, torch.complex128])
+def test_scaled_solve(gpu, k, dtype):
+    """diag(r) solve(diag(r) B) in one call: the same bits as the two products around the solve."""
+    dv = gpu
+    torch.manual_seed(4)
+    n = 200
+    Z = (torch.randn(n, n, dtype=torch.complex128, device=dv.device()) + 30 * torch.eye(n, device=dv.device())).to(dtype)
+    F = dv.getrf(Z)
+    B = torch.randn(n, k, dtype=torch.complex128, device=dv.device())
+    r = torch.rand(n, dtype=torch.float64, device=dv.device()) + 0.5
+    assert torch.equal(dv.getrs(F, B, scale=r), r[:, None] * dv.getrs(F, r[:, None] * B))
+    assert not dv.solve_faults()
+
+
+def test_cast_rows_refuses(gpu):
+    from mom25d_amd import _lib as L
+    t = gpu.ptr(torch.zeros(8, dtype=torch.complex128, device=gpu.device()))
+    for bad in [(7, t, 2, 1, t, 2, 2, 2), (L.C128, t, 1, L.C64, t, 2, 2, 2), (L.C128, t, 2, L.C64, t, 1, 2, 2),
+                (L.C128, None, 2, L.C64, t, 2, 2, 2), (L.C128, t, 2, L.C64, t, 2, -1, 2)]:
+        with pytest.raises(Exception):
+            L.call('m25x_cast_rows', *bad, None, gpu.stream())
