@@ -419,6 +419,13 @@ size_t m25x_cgs2_work_bytes(void);
 int m25x_cgs2(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
               size_t work_bytes, void *stream);
 
+/* The same for 1 <= k <= M25X_CGS2_COLS columns (many points' systems side by side), each column by itself, with
+ * m25x_cgs2_cols_work_bytes(k) bytes of workspace. */
+#define M25X_CGS2_COLS 65536
+size_t m25x_cgs2_cols_work_bytes(int k);
+int m25x_cgs2_cols(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
+                   size_t work_bytes, void *stream);
+
 /* dst[i][c] = r[i] src[i][c] (r: n doubles, NULL for 1) for n x k complex arrays of the given dtypes (M25X_C64,
  * M25X_C128; leading dimensions lds, ldd >= k in elements; not overlapping): the product in FP64, rounded once to
  * dst's type. The solves' right-hand sides and answers between the refinement's FP64 and a complex64 factor, with

@@ -165,15 +165,33 @@ extern "C" int m25x_zgemm_nk_batched(int nitems, const m25x_mv_item *h, const m2
 // sends the half that the partner keeps: 8 exchanges for 8 sums over 16 lanes, not 32), and every block of the next
 // launch adds the blocks' partial sums itself instead of a launch of one workgroup between them. Seven launches with
 // one vector a round trip took 38.5 us at n = 7799, k = 4 on six vectors and 94 on 30, these take 18.1 and 34.2;
-// at n = 905 27.9 and 16.6 on six, at n = 20 000 348 and 59 on 30.
+// at n = 905 27.9 and 16.6 on six, at n = 20 000 348 and 59 on 30. More than eight columns (many points side by side)
+// go in groups of eight, a grid row each, with fewer row blocks as the groups fill the chip by themselves.
 namespace {
 
-constexpr int GS_B = 128;                // row blocks at most
+constexpr int GS_B = 128;                // row blocks at most, and over all groups of columns where each has GS_BMIN
+constexpr int GS_BMIN = 16;
+constexpr int GS_C = 8;                  // columns a group
 constexpr int GS_T = 256;                // threads a block: KP columns x GS_T / KP row lanes
 constexpr int GS_MAXV = 64;              // basis vectors at most
 constexpr int GS_CH = 8;                 // basis vectors read at a time
 
-// h[i k + c] = sum over the blocks' partial sums P[b][i k + c]: m = nv k entries, up to GS_T / m threads an entry.
+constexpr int gs_groups(int k) { return (k + GS_C - 1) / GS_C; }
+constexpr int gs_blocks(int k) { return GS_B / gs_groups(k) > GS_BMIN ? GS_B / gs_groups(k) : GS_BMIN; }
+
+// A grid row's columns c0 .. c0 + kc - 1, and its own partial sums (two passes' and the norms').
+struct GsGroup {
+    int c0, kc;
+    long p, q;
+};
+template <int KP>
+__device__ inline GsGroup gs_group(int k)
+{
+    const int g = blockIdx.y, c0 = g * GS_C;
+    return {c0, k - c0 < KP ? k - c0 : KP, (long)g * gridDim.x * GS_MAXV * GS_C, (long)g * gridDim.x * GS_C};
+}
+
+// h[i kc + c] = sum over the blocks' partial sums P[b][i kc + c]: m = nv kc entries, up to GS_T / m threads an entry.
 __device__ inline void gs_sum(const double2 *__restrict__ P, int nb, int m, double2 *h, double2 *part)
 {
     const int t = threadIdx.x, S = m < GS_T ? GS_T / m : 1;
@@ -208,8 +226,8 @@ __device__ inline void gs_load(double2 (&v)[GS_CH], const double2 *__restrict__ 
     for (int u = 0; u < GS_CH; ++u) v[u] = V[(long)(i0 + u < nv ? i0 + u : nv - 1) * nk + e];
 }
 
-// x - sum_i V[i] h[i] at element e of column c
-__device__ inline double2 gs_minus(double2 x, const double2 *__restrict__ V, long nk, long e, int c, int k, int nv,
+// x - sum_i V[i] h[i] at element e of column c of kc
+__device__ inline double2 gs_minus(double2 x, const double2 *__restrict__ V, long nk, long e, int c, int kc, int nv,
                                    const double2 *h)
 {
     for (int i0 = 0; i0 < nv; i0 += GS_CH) {
@@ -218,7 +236,7 @@ __device__ inline double2 gs_minus(double2 x, const double2 *__restrict__ V, lon
 #pragma unroll
         for (int u = 0; u < GS_CH; ++u)
             if (i0 + u < nv) {
-                const double2 hv = h[(i0 + u) * k + c];
+                const double2 hv = h[(i0 + u) * kc + c];
                 x.x -= v[u].x * hv.x - v[u].y * hv.y;
                 x.y -= v[u].x * hv.y + v[u].y * hv.x;
             }
@@ -226,7 +244,7 @@ __device__ inline double2 gs_minus(double2 x, const double2 *__restrict__ V, lon
     return x;
 }
 
-// Partial dots of block blockIdx.x's rows: P[b][i k + c] = sum_r conj(V[i][r][c]) x[r][c]. UPD: x -= V h first, h the
+// Partial dots of block blockIdx.x's rows: P[b][i kc + c] = sum_r conj(V[i][r][c]) x[r][c]. UPD: x -= V h first, h the
 // sum of the last pass's partial sums Pin; block 0 stores h to H.
 template <int KP, bool UPD>
 __global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V, long n, int k, int nv,
@@ -237,20 +255,24 @@ __global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V,
     __shared__ double2 h[UPD ? GS_MAXV * KP : 1], part[UPD ? GS_T : 1];
     constexpr int RL = GS_T / KP;
     const int t = threadIdx.x, c = t % KP, rl = t / KP, wv = t >> 6, lane = t & 63;
+    const GsGroup g = gs_group<KP>(k);
+    const int kc = g.kc, m = nv * kc;
     const long nk = n * k, step = (long)gridDim.x * RL;
+    V += g.c0;
+    x += g.c0;
     if (UPD) {
-        gs_sum(Pin, gridDim.x, nv * k, h, part);
+        gs_sum(Pin + g.p, gridDim.x, m, h, part);
         if (blockIdx.x == 0)
-            for (int e = t; e < nv * k; e += GS_T) H[e] = h[e];
-        if (c < k)                               // each thread updates the elements it reads below
+            for (int e = t; e < m; e += GS_T) H[e / kc * k + g.c0 + e % kc] = h[e];
+        if (c < kc)                              // each thread updates the elements it reads below
             for (long r = (long)blockIdx.x * RL + rl; r < n; r += step)
-                x[r * k + c] = gs_minus(x[r * k + c], V, nk, r * k + c, c, k, nv, h);
+                x[r * k + c] = gs_minus(x[r * k + c], V, nk, r * k + c, c, kc, nv, h);
     }
     for (int i0 = 0; i0 < nv; i0 += GS_CH) {
         double2 a[GS_CH];
 #pragma unroll
         for (int u = 0; u < GS_CH; ++u) a[u] = make_double2(0, 0);
-        if (c < k)
+        if (c < kc)
             for (long r = (long)blockIdx.x * RL + rl; r < n; r += step) {
                 const double2 xv = x[r * k + c];
                 double2 v[GS_CH];
@@ -279,12 +301,12 @@ __global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V,
         if (lane < 8 * KP && i < nv) red[i][wv][c] = a[0];
     }
     __syncthreads();
-    for (int e = t; e < nv * k; e += GS_T) {
-        const double2 *q = &red[e / k][0][e % k];
+    for (int e = t; e < m; e += GS_T) {
+        const double2 *q = &red[e / kc][0][e % kc];
         double2 s = q[0];
 #pragma unroll
         for (int w = 1; w < GS_T / 64; ++w) { s.x += q[w * KP].x; s.y += q[w * KP].y; }
-        P[(long)blockIdx.x * nv * k + e] = s;
+        P[g.p + (long)blockIdx.x * m + e] = s;
     }
 }
 
@@ -298,13 +320,20 @@ __global__ __launch_bounds__(GS_T) void k_gs_final(const double2 *__restrict__ V
     __shared__ double red[GS_T / 64][KP];
     constexpr int RL = GS_T / KP;
     const int t = threadIdx.x, c = t % KP, rl = t / KP;
-    gs_sum(Pin, gridDim.x, nv * k, h, part);
+    const GsGroup g = gs_group<KP>(k);
+    const int kc = g.kc, m = nv * kc;
+    V += g.c0;
+    x += g.c0;
+    gs_sum(Pin + g.p, gridDim.x, m, h, part);
     if (blockIdx.x == 0)
-        for (int e = t; e < nv * k; e += GS_T) { H[e].x += h[e].x; H[e].y += h[e].y; }
+        for (int e = t; e < m; e += GS_T) {
+            double2 &to = H[e / kc * k + g.c0 + e % kc];
+            to.x += h[e].x; to.y += h[e].y;
+        }
     double q = 0;
-    if (c < k)
+    if (c < kc)
         for (long r = (long)blockIdx.x * RL + rl; r < n; r += (long)gridDim.x * RL) {
-            const double2 xv = gs_minus(x[r * k + c], V, n * k, r * k + c, c, k, nv, h);
+            const double2 xv = gs_minus(x[r * k + c], V, n * k, r * k + c, c, kc, nv, h);
             x[r * k + c] = xv;
             q += xv.x * xv.x + xv.y * xv.y;
         }
@@ -312,10 +341,10 @@ __global__ __launch_bounds__(GS_T) void k_gs_final(const double2 *__restrict__ V
     for (int o = KP; o < 64; o <<= 1) q += __shfl_xor(q, o);
     if ((t & 63) < KP) red[t >> 6][c] = q;
     __syncthreads();
-    if (t < k) {
+    if (t < kc) {
         double s = red[0][t];
         for (int w = 1; w < GS_T / 64; ++w) s += red[w][t];
-        Q[blockIdx.x * KP + t] = s;
+        Q[g.q + blockIdx.x * KP + t] = s;
     }
 }
 
@@ -329,11 +358,12 @@ __global__ __launch_bounds__(GS_T) void k_gs_scale(const double2 *__restrict__ x
     constexpr int RL = GS_T / KP;
     const int t = threadIdx.x, c = t % KP, rl = t / KP;
     const long r = (long)blockIdx.x * RL + rl;
-    const bool in = c < k && r < n;
-    const double2 xv = in ? x[r * k + c] : make_double2(0, 0);
+    const int c0 = blockIdx.y * GS_C, kc = k - c0 < KP ? k - c0 : KP;
+    const bool in = c < kc && r < n;
+    const double2 xv = in ? x[r * k + c0 + c] : make_double2(0, 0);
     double q = 0;
-    if (c < k)
-        for (int b = rl; b < nb; b += RL) q += Q[b * KP + c];
+    if (c < kc)
+        for (int b = rl; b < nb; b += RL) q += Q[(long)blockIdx.y * nb * GS_C + b * KP + c];
 #pragma unroll
     for (int o = KP; o < 64; o <<= 1) q += __shfl_xor(q, o);
     if ((t & 63) < KP) red[t >> 6][c] = q;
@@ -341,43 +371,60 @@ __global__ __launch_bounds__(GS_T) void k_gs_scale(const double2 *__restrict__ x
     double s = red[0][c];
     for (int w = 1; w < GS_T / 64; ++w) s += red[w][c];
     const double nr = sqrt(s), sc = nr > 0 ? 1.0 / nr : 1.0;
-    if (blockIdx.x == 0 && t < k) H[nv * k + t] = make_double2(nr, 0);
-    if (in) out[r * k + c] = make_double2(xv.x * sc, xv.y * sc);
+    if (blockIdx.x == 0 && t < kc) H[nv * k + c0 + t] = make_double2(nr, 0);
+    if (in) out[r * k + c0 + c] = make_double2(xv.x * sc, xv.y * sc);
 }
 
 template <int KP>
 void cgs2(const double2 *V, long n, int k, int nv, double2 *x, double2 *H, double2 *out, double2 *P, hipStream_t s)
 {
+    const int ng = gs_groups(k);
     const long full = (n + GS_T / KP - 1) / (GS_T / KP);
-    const int nb = (int)std::min<long>(full, GS_B);
-    double2 *P2 = P + (size_t)GS_B * GS_MAXV * 8;
-    double *Q = (double *)(P2 + (size_t)GS_B * GS_MAXV * 8);
-    hipLaunchKernelGGL((k_gs_dots<KP, false>), dim3(nb), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)nullptr,
+    const int nb = (int)std::min<long>(full, gs_blocks(k));
+    double2 *P2 = P + (size_t)ng * nb * GS_MAXV * GS_C;
+    double *Q = (double *)(P2 + (size_t)ng * nb * GS_MAXV * GS_C);
+    hipLaunchKernelGGL((k_gs_dots<KP, false>), dim3(nb, ng), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)nullptr,
                        (double2 *)nullptr, P);
-    hipLaunchKernelGGL((k_gs_dots<KP, true>), dim3(nb), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)P, H, P2);
-    hipLaunchKernelGGL(k_gs_final<KP>, dim3(nb), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)P2, H, Q);
-    hipLaunchKernelGGL(k_gs_scale<KP>, dim3((unsigned)full), dim3(GS_T), 0, s, (const double2 *)x, n, k, nv, nb,
+    hipLaunchKernelGGL((k_gs_dots<KP, true>), dim3(nb, ng), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)P, H, P2);
+    hipLaunchKernelGGL(k_gs_final<KP>, dim3(nb, ng), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)P2, H, Q);
+    hipLaunchKernelGGL(k_gs_scale<KP>, dim3((unsigned)full, ng), dim3(GS_T), 0, s, (const double2 *)x, n, k, nv, nb,
                        (const double *)Q, H, out);
+}
+
+int cgs2_any(const char *who, int kmax, const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext,
+             void *work, size_t work_bytes, size_t need, hipStream_t s)
+{
+    if (!V || !w || !hcol || !vnext || !work || n < 1 || k < 1 || k > kmax || nv < 1 || nv > GS_MAXV - 1)
+        return fail(M25X_EINVAL, "%s: bad arguments (1 <= k <= %d, 1 <= nv <= %d)", who, kmax, GS_MAXV - 1);
+    if (work_bytes < need) return fail(M25X_EINVAL, "%s: workspace too small", who);
+    TimedLaunch tl(s, M25X_K_CGS2, M25X_C128, 16.0 * n * k * (2.0 * nv + 3), 16.0 * n * k * nv);
+    const auto run = k == 1 ? cgs2<1> : k == 2 ? cgs2<2> : k <= 4 ? cgs2<4> : cgs2<8>;
+    run((const double2 *)V, n, k, nv, (double2 *)w, (double2 *)hcol, (double2 *)vnext, (double2 *)work, s);
+    return check_launch(who);
 }
 
 }  // namespace
 
-extern "C" size_t m25x_cgs2_work_bytes(void)
+extern "C" size_t m25x_cgs2_cols_work_bytes(int k)
 {
-    return 2 * (size_t)GS_B * GS_MAXV * 8 * sizeof(double2) + GS_B * 8 * sizeof(double);
+    if (k < 1 || k > M25X_CGS2_COLS) return 0;
+    return (size_t)gs_groups(k) * gs_blocks(k) * GS_C * (2 * GS_MAXV * sizeof(double2) + sizeof(double));
 }
+
+extern "C" size_t m25x_cgs2_work_bytes(void) { return m25x_cgs2_cols_work_bytes(GS_C); }
 
 extern "C" int m25x_cgs2(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
                          size_t work_bytes, void *stream)
 {
-    if (!V || !w || !hcol || !vnext || !work || n < 1 || k < 1 || k > 8 || nv < 1 || nv > GS_MAXV - 1)
-        return fail(M25X_EINVAL, "cgs2: bad arguments (1 <= k <= 8, 1 <= nv <= %d)", GS_MAXV - 1);
-    if (work_bytes < m25x_cgs2_work_bytes()) return fail(M25X_EINVAL, "cgs2: workspace too small");
-    hipStream_t s = (hipStream_t)stream;
-    TimedLaunch tl(s, M25X_K_CGS2, M25X_C128, 16.0 * n * k * (2.0 * nv + 3), 16.0 * n * k * nv);
-    const auto run = k == 1 ? cgs2<1> : k == 2 ? cgs2<2> : k <= 4 ? cgs2<4> : cgs2<8>;
-    run((const double2 *)V, n, k, nv, (double2 *)w, (double2 *)hcol, (double2 *)vnext, (double2 *)work, s);
-    return check_launch("cgs2");
+    return cgs2_any("cgs2", GS_C, V, n, k, nv, w, hcol, vnext, work, work_bytes, m25x_cgs2_work_bytes(),
+                    (hipStream_t)stream);
+}
+
+extern "C" int m25x_cgs2_cols(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
+                              size_t work_bytes, void *stream)
+{
+    return cgs2_any("cgs2_cols", M25X_CGS2_COLS, V, n, k, nv, w, hcol, vnext, work, work_bytes,
+                    m25x_cgs2_cols_work_bytes(k), (hipStream_t)stream);
 }
 
 // ---- the solves' right-hand sides between precisions ----------------------------------------------------------

@@ -539,6 +539,12 @@ def _item_table(cls, items):
     return arr, raw.to(device(), non_blocking=False)
 
 
+def _call_table(cls, items):
+    """_item_table for one call on the current stream, which the host does not wait for."""
+    arr = (cls * len(items))(*items)
+    return arr, upload(np.frombuffer(arr, np.int64))[0]
+
+
 class BatchFactors:
     """The LU factors of a batch of matrices (m25x_getrf_batched): factors[i] is a Factor of Zs[i], in place."""
 
@@ -610,7 +616,7 @@ class BatchSolve:
                                       X.data_ptr() + (c0 + p) * X.element_size(), k, q, 0, w.data_ptr(),
                                       w.numel()))
         if items:
-            host, dev_tab = _item_table(L.RsItem, items)
+            host, dev_tab = _call_table(L.RsItem, items)
             L.call('m25x_getrs_batched', self.code, len(items), host, ptr(dev_tab), int(trans), ptr(self.status),
                    stream())
             _solve_fault(X.device).bitwise_or_(self.status)
@@ -629,7 +635,7 @@ def zgemm_nk_batched(Zs, V, cols, out=None):
             items.append(L.MvItem(Z.data_ptr(), Z.shape[0], Z.stride(0), V.data_ptr() + (c0 + p) * 16,
                                   Y.data_ptr() + (c0 + p) * 16, V.shape[1], Y.shape[1], q, 0))
     if items:
-        host, dev_tab = _item_table(L.MvItem, items)
+        host, dev_tab = _call_table(L.MvItem, items)
         L.call('m25x_zgemm_nk_batched', len(items), host, ptr(dev_tab), stream())
     return Y
 
@@ -703,19 +709,16 @@ def zgemm_nk(Z, X):
     return Y[:, 0] if one else Y
 
 
-_CGS2_WORK = {}
+CGS2_COLS = 65536             # columns of one cgs2 call at most
 
 
 def cgs2(V, nv, W, hcol):
     """One Arnoldi step on the device: W (n x k complex128, overwritten) orthogonalised against V[:nv] by classical
     Gram-Schmidt applied twice; hcol[:nv + 1] (nv + 1, k) receives the coefficients and |W| (real); V[nv] = W / |W|.
-    V: (m, n, k) complex128 contiguous, k <= 8. Calls on one device share a workspace: one stream at a time."""
+    V: (m, n, k) complex128 contiguous. Each call has its own workspace."""
     m, n, k = V.shape
     if not (V.is_contiguous() and W.is_contiguous() and hcol.is_contiguous()) or W.shape != (n, k) or nv >= m:
         raise ValueError("cgs2: V (m, n, k), W (n, k) contiguous, nv < m")
-    dev = V.device
-    work = _CGS2_WORK.get(dev)
-    if work is None:
-        work = _CGS2_WORK[dev] = torch.empty(L.lib().m25x_cgs2_work_bytes(), dtype=torch.uint8, device=dev)
-    L.call('m25x_cgs2', ptr(V), n, k, nv, ptr(W), ptr(hcol), ptr(V[nv]), ptr(work), work.numel(), stream())
+    work = torch.empty(L.lib().m25x_cgs2_cols_work_bytes(k), dtype=torch.uint8, device=V.device)
+    L.call('m25x_cgs2_cols', ptr(V), n, k, nv, ptr(W), ptr(hcol), ptr(V[nv]), ptr(work), work.numel(), stream())
 

@@ -3,7 +3,7 @@
 Right-preconditioned, k systems in lockstep: every operator / preconditioner call is one (N x k_active) product on
 the GPU (the FP64 Z product of m25x_zgemm_nk, the complex64 factor's solves of m25x_getrs). The Krylov basis stays
 on the device and is orthogonalised by classical Gram-Schmidt applied twice (the reference uses modified
-Gram-Schmidt: the same basis to rounding), fused in one call (m25x_cgs2) for up to 8 systems; the small Hessenberg
+Gram-Schmidt: the same basis to rounding), fused in one call (m25x_cgs2, m25x_cgs2_cols); the small Hessenberg
 columns come to the host once per iteration for the conjugated Givens rotations, the convergence test and the
 stall cut-off, as the reference computes them. The next iteration's device work (preconditioner, product,
 orthogonalisation) does not depend on those, so it is queued before the host waits for the current column
@@ -88,8 +88,8 @@ def gmres_batched(A, B, M=None, x0=None, rtol=1e-6, restart=30, maxiter=10, stal
         rn = np.zeros((restart + 1, ka))                             # residual estimates, for the prediction
         rn[0] = beta
         hbuf = torch.empty((restart + 1, ka), dtype=torch.complex128, device=dev)
-        # classical Gram-Schmidt twice (as stable as modified Gram-Schmidt): one fused device call for up to 8
-        # systems and 63 basis vectors (then pipelined one iteration ahead), batched tensor products beyond
+        # classical Gram-Schmidt twice (as stable as modified Gram-Schmidt): one fused device call for up to 63 basis
+        # vectors, batched tensor products beyond; up to 8 systems are pipelined one iteration ahead
         fused = ka <= 8 and restart < 64
         if fused:
             pin, evs, queued = _pinned((restart + 1, ka)), [torch.cuda.Event(), torch.cuda.Event()], -1
@@ -115,14 +115,18 @@ def gmres_batched(A, B, M=None, x0=None, rtol=1e-6, restart=30, maxiter=10, stal
             else:
                 Zs[j] = M(V[j])
                 Wv = A(Zs[j]).contiguous()
-                Vj = V[:j + 1]
-                h1 = (Vj.conj() * Wv[None]).sum(1)
-                Wv = Wv - (Vj * h1[:, None, :]).sum(0)
-                h2 = (Vj.conj() * Wv[None]).sum(1)
-                Wv = Wv - (Vj * h2[:, None, :]).sum(0)
-                hn = torch.linalg.vector_norm(Wv, dim=0)
-                V[j + 1] = Wv / torch.where(hn > 0, hn, torch.ones_like(hn))
-                hc = torch.cat([h1 + h2, hn[None].to(torch.complex128)], 0).cpu().numpy()
+                if restart < 64 and ka <= dv.CGS2_COLS:
+                    dv.cgs2(V, j + 1, Wv, hbuf)
+                    hc = hbuf[:j + 2].cpu().numpy()
+                else:
+                    Vj = V[:j + 1]
+                    h1 = (Vj.conj() * Wv[None]).sum(1)
+                    Wv = Wv - (Vj * h1[:, None, :]).sum(0)
+                    h2 = (Vj.conj() * Wv[None]).sum(1)
+                    Wv = Wv - (Vj * h2[:, None, :]).sum(0)
+                    hn = torch.linalg.vector_norm(Wv, dim=0)
+                    V[j + 1] = Wv / torch.where(hn > 0, hn, torch.ones_like(hn))
+                    hc = torch.cat([h1 + h2, hn[None].to(torch.complex128)], 0).cpu().numpy()
             H[:j + 2, j] = hc
             for i in range(j):                                       # previous Givens rotations
                 H[i, j], H[i + 1, j] = (cs[i] * H[i, j] + sn[i] * H[i + 1, j],
@@ -168,6 +172,7 @@ def gmres_batched(A, B, M=None, x0=None, rtol=1e-6, restart=30, maxiter=10, stal
                 kn = np.flatnonzero(live)
                 kt = torch.from_numpy(kn).to(dev)
                 V, Zs = V[:, :, kt].contiguous(), Zs[:, :, kt].contiguous()
+                hbuf = hbuf[:, kt].contiguous()
                 H, g, cs, sn, rn = H[:, :, kn], g[:, kn], cs[:, kn], sn[:, kn], rn[:, kn]
                 last, live, act, ka = last[kn], live[kn], act[kn], len(kn)
                 if track is not None:

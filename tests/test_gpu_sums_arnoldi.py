@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,k,nv", [(1, 8, 1), (31, 7, 8), (33, 6, 9), (129, 2, 7), (300, 1, 63), (905, 5, 51), (905, 4, 63),
-                                    (16385, 2, 16), (8193, 4, 17), (20000, 3, 2), (4097, 8, 32)])
+                                    (16385, 2, 16), (8193, 4, 17), (20000, 3, 2), (4097, 8, 32),
+                                    (700, 9, 3), (1100, 16, 8), (905, 24, 33), (300, 67, 6), (513, 130, 2), (5, 1025, 4)])
 def test_step_against_numpy(gpu, n, k, nv):
     dv = gpu
     rng = np.random.default_rng(17 * n + k + nv)
