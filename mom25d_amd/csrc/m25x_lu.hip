@@ -8,17 +8,18 @@
 //           between, the next column's candidates published before the barrier); pivots by LAPACK's rule
 //           (largest |Re| + |Im|, the first on ties)
 //   laswp   the panel's interchanges on the columns left and right of it
-//   trsm    U12 = L11^-1 A12 (unit lower, forward substitution, one workgroup per 16 columns)
+//   trsm    U12 = L11^-1 A12 (unit lower, forward substitution, one workgroup per 16 columns: k_trsm, these panels
+//           only)
 //   gemm    A22 -= A21 U12 on the matrix cores: complex products as real ones through the real embedding
 //           (Re C = [Re A, Im A] [Re B; -Im B], Im C = [Re A, Im A] [Im B; Re B]), v_mfma_f64_16x16x4 for
 //           complex128 and v_mfma_f32_16x16x4 for complex64 (FP32 accumulation)
 // Tournament pivoting (CALU), panels of TW = 64 columns: the panel's pivots by a tree of GEPPs in one launch with no
 // grid barrier (k_tslu), its row moves on every column (k_apply_moves), then L21 = A21 U11^-1 and U12 = L11^-1 A12 by
-// substitution (k_tri) and A22 -= L21 U12 on the matrix cores (complex64 with FP64 accumulation: one
-// rounding per update).
-// The solves (getrs): one launch per triangle, one workgroup per 64-row diagonal block; each accumulates the
-// products of its rows with the earlier blocks as their values appear, then solves its own block and hands its
-// values on as self-marking words.
+// substitution (k_tri) and A22 -= L21 U12 on the matrix cores (complex64 in FP32, or with FP64 accumulation where
+// asked for); the next panel's tournament runs beside the larger updates.
+// The solves (getrs): both triangles in one launch, one workgroup per 64-row diagonal block, triangle and two
+// right-hand sides; each accumulates the products of its rows with the earlier blocks as their values appear, then
+// solves its own block and hands its values on as self-marking words.
 #include <atomic>
 #include <mutex>
 #include <vector>

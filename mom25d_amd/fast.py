@@ -6,9 +6,8 @@ Per frequency, everything on the device:
   fill     Z (N x N complex128): far field, near-field correction (pairs and their analytic moments resident
            across frequencies), via rows / columns and block, lumped elements
   solve    'double': Z equilibrated (D Z D, d = 1/sqrt|Z_ii|), complex128 LU, solves
-           'mixed' : the complex64 copy of the equilibrated Z factored (trailing updates on the FP64 matrix
-                     cores, one rounding to FP32 an entry), GMRES refinement
-                     against the FP64 Z (restart 30, stall (4, 0.1) for a fresh factor, converged at 100 x 1e-6);
+           'mixed' : the complex64 copy of the equilibrated Z factored (trailing updates on the FP32 matrix
+                     cores), GMRES refinement against the FP64 Z (restart 30, stall (4, 0.1) for a fresh factor, converged at 100 x 1e-6);
                      a kept factor of a nearby frequency tried first (its reach learnt); where the complex64
                      factor does not converge, complex128 LU, and double precision up to MIXED_RETRY x f
 The currents come back to the host (N x ports); everything else stays on the GPU.

@@ -6,7 +6,8 @@
   sommerfeld_contour       the integration path of the Sommerfeld integrals (src/mom25d/via.py:36-53)
   green_tables             every interface pair's GreenTableML of a frequency (src/mom25d/multilayer.py:253-318,
                            src/mom25d/sim.py:736-745) in one batch: one launch of m25x_spectra for all spectra, one
-                           Hankel transform (m25x_hankel) and one spline product for all tables
+                           Hankel transform (m25x_hankel_sets) and one spline product (m25x_resample) for all
+                           tables
   RunLog                   stage timings and notes (src/mom25d/multilayer.py:30-53)
 
 The spectral network itself (layer admittances, the voltages of a shunt source, the spectra) is the HIP kernel
