@@ -426,6 +426,11 @@ size_t m25x_cgs2_cols_work_bytes(int k);
 int m25x_cgs2_cols(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
                    size_t work_bytes, void *stream);
 
+/* m25x_cgs2_cols without changing w (the vector between its passes is in vnext): for a w that is an operator's
+ * result, which may be the operator's argument or kept by its owner. The same hcol and vnext bit for bit. */
+int m25x_cgs2_keep(const double *V, long n, int k, int nv, const double *w, double *hcol, double *vnext, void *work,
+                   size_t work_bytes, void *stream);
+
 /* dst[i][c] = r[i] src[i][c] (r: n doubles, NULL for 1) for n x k complex arrays of the given dtypes (M25X_C64,
  * M25X_C128; leading dimensions lds, ldd >= k in elements; not overlapping): the product in FP64, rounded once to
  * dst's type. The solves' right-hand sides and answers between the refinement's FP64 and a complex64 factor, with

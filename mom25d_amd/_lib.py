@@ -122,6 +122,7 @@ _SIGS = {
     'm25x_cgs2': ([P, L, I, I, P, P, P, P, S, P], I),
     'm25x_cgs2_cols_work_bytes': ([I], S),
     'm25x_cgs2_cols': ([P, L, I, I, P, P, P, P, S, P], I),
+    'm25x_cgs2_keep': ([P, L, I, I, P, P, P, P, S, P], I),
     'm25x_cast_rows': ([I, P, L, I, P, L, L, L, P, P], I),
 }
 

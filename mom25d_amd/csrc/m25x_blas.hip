@@ -156,6 +156,7 @@ extern "C" int m25x_zgemm_nk_batched(int nitems, const m25x_mv_item *h, const m2
 // ---- classical Gram-Schmidt, twice, for the batched GMRES ------------------------------------------------------
 // V: (j + 1) basis vectors, each n x k complex128 row-major (vector i at V + i n k); w: n x k. Per column c:
 // h1 = V^H w, w1 = w - V h1, h2 = V^H w1, w2 = w1 - V h2, h = h1 + h2, nrm = |w2|, V[j + 1] = w2 / nrm (nrm = 0: w2).
+// w1 and w2 go over w, or into V[j + 1] where the caller keeps w (the same reads and writes either way).
 // Sums over rows in fixed blocks, then over blocks in a fixed order: the result does not depend on timing.
 //
 // Four launches, each waiting for the sums of the one before; the basis (3 MB at n = 7799, k = 4, six vectors) stays in
@@ -244,11 +245,11 @@ __device__ inline double2 gs_minus(double2 x, const double2 *__restrict__ V, lon
     return x;
 }
 
-// Partial dots of block blockIdx.x's rows: P[b][i kc + c] = sum_r conj(V[i][r][c]) x[r][c]. UPD: x -= V h first, h the
-// sum of the last pass's partial sums Pin; block 0 stores h to H.
+// Partial dots of block blockIdx.x's rows: P[b][i kc + c] = sum_r conj(V[i][r][c]) w[r][c]. UPD: of x = w - V h, h the
+// sum of the last pass's partial sums Pin, x stored (it may be w); block 0 stores h to H.
 template <int KP, bool UPD>
-__global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V, long n, int k, int nv,
-                                                 double2 *__restrict__ x, const double2 *__restrict__ Pin,
+__global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V, long n, int k, int nv, const double2 *w,
+                                                 double2 *x, const double2 *__restrict__ Pin,
                                                  double2 *__restrict__ H, double2 *__restrict__ P)
 {
     __shared__ double2 red[GS_MAXV][GS_T / 64][KP];
@@ -259,6 +260,7 @@ __global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V,
     const int kc = g.kc, m = nv * kc;
     const long nk = n * k, step = (long)gridDim.x * RL;
     V += g.c0;
+    w += g.c0;
     x += g.c0;
     if (UPD) {
         gs_sum(Pin + g.p, gridDim.x, m, h, part);
@@ -266,7 +268,7 @@ __global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V,
             for (int e = t; e < m; e += GS_T) H[e / kc * k + g.c0 + e % kc] = h[e];
         if (c < kc)                              // each thread updates the elements it reads below
             for (long r = (long)blockIdx.x * RL + rl; r < n; r += step)
-                x[r * k + c] = gs_minus(x[r * k + c], V, nk, r * k + c, c, kc, nv, h);
+                x[r * k + c] = gs_minus(w[r * k + c], V, nk, r * k + c, c, kc, nv, h);
     }
     for (int i0 = 0; i0 < nv; i0 += GS_CH) {
         double2 a[GS_CH];
@@ -274,7 +276,7 @@ __global__ __launch_bounds__(GS_T) void k_gs_dots(const double2 *__restrict__ V,
         for (int u = 0; u < GS_CH; ++u) a[u] = make_double2(0, 0);
         if (c < kc)
             for (long r = (long)blockIdx.x * RL + rl; r < n; r += step) {
-                const double2 xv = x[r * k + c];
+                const double2 xv = UPD ? x[r * k + c] : w[r * k + c];
                 double2 v[GS_CH];
                 gs_load(v, V, nk, r * k + c, i0, nv);
 #pragma unroll
@@ -348,11 +350,10 @@ __global__ __launch_bounds__(GS_T) void k_gs_final(const double2 *__restrict__ V
     }
 }
 
-// H[nv][c] = |x| (real, block 0), out = x / |x|; Q: nb blocks' partial |x|^2.
+// H[nv][c] = |x| (real, block 0), out = x / |x| (out may be x); Q: nb blocks' partial |x|^2.
 template <int KP>
-__global__ __launch_bounds__(GS_T) void k_gs_scale(const double2 *__restrict__ x, long n, int k, int nv, int nb,
-                                                  const double *__restrict__ Q, double2 *__restrict__ H,
-                                                  double2 *__restrict__ out)
+__global__ __launch_bounds__(GS_T) void k_gs_scale(const double2 *x, long n, int k, int nv, int nb,
+                                                  const double *__restrict__ Q, double2 *__restrict__ H, double2 *out)
 {
     __shared__ double red[GS_T / 64][KP];
     constexpr int RL = GS_T / KP;
@@ -376,30 +377,32 @@ __global__ __launch_bounds__(GS_T) void k_gs_scale(const double2 *__restrict__ x
 }
 
 template <int KP>
-void cgs2(const double2 *V, long n, int k, int nv, double2 *x, double2 *H, double2 *out, double2 *P, hipStream_t s)
+void cgs2(const double2 *V, long n, int k, int nv, const double2 *w, double2 *x, double2 *H, double2 *out, double2 *P,
+          hipStream_t s)
 {
     const int ng = gs_groups(k);
     const long full = (n + GS_T / KP - 1) / (GS_T / KP);
     const int nb = (int)std::min<long>(full, gs_blocks(k));
     double2 *P2 = P + (size_t)ng * nb * GS_MAXV * GS_C;
     double *Q = (double *)(P2 + (size_t)ng * nb * GS_MAXV * GS_C);
-    hipLaunchKernelGGL((k_gs_dots<KP, false>), dim3(nb, ng), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)nullptr,
+    hipLaunchKernelGGL((k_gs_dots<KP, false>), dim3(nb, ng), dim3(GS_T), 0, s, V, n, k, nv, w, x, (const double2 *)nullptr,
                        (double2 *)nullptr, P);
-    hipLaunchKernelGGL((k_gs_dots<KP, true>), dim3(nb, ng), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)P, H, P2);
+    hipLaunchKernelGGL((k_gs_dots<KP, true>), dim3(nb, ng), dim3(GS_T), 0, s, V, n, k, nv, w, x, (const double2 *)P, H, P2);
     hipLaunchKernelGGL(k_gs_final<KP>, dim3(nb, ng), dim3(GS_T), 0, s, V, n, k, nv, x, (const double2 *)P2, H, Q);
     hipLaunchKernelGGL(k_gs_scale<KP>, dim3((unsigned)full, ng), dim3(GS_T), 0, s, (const double2 *)x, n, k, nv, nb,
                        (const double *)Q, H, out);
 }
 
-int cgs2_any(const char *who, int kmax, const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext,
-             void *work, size_t work_bytes, size_t need, hipStream_t s)
+// x: where w1 and w2 go, w or vnext
+int cgs2_any(const char *who, int kmax, const double *V, long n, int k, int nv, const double *w, double *x, double *hcol,
+             double *vnext, void *work, size_t work_bytes, size_t need, hipStream_t s)
 {
     if (!V || !w || !hcol || !vnext || !work || n < 1 || k < 1 || k > kmax || nv < 1 || nv > GS_MAXV - 1)
         return fail(M25X_EINVAL, "%s: bad arguments (1 <= k <= %d, 1 <= nv <= %d)", who, kmax, GS_MAXV - 1);
     if (work_bytes < need) return fail(M25X_EINVAL, "%s: workspace too small", who);
     TimedLaunch tl(s, M25X_K_CGS2, M25X_C128, 16.0 * n * k * (2.0 * nv + 3), 16.0 * n * k * nv);
     const auto run = k == 1 ? cgs2<1> : k == 2 ? cgs2<2> : k <= 4 ? cgs2<4> : cgs2<8>;
-    run((const double2 *)V, n, k, nv, (double2 *)w, (double2 *)hcol, (double2 *)vnext, (double2 *)work, s);
+    run((const double2 *)V, n, k, nv, (const double2 *)w, (double2 *)x, (double2 *)hcol, (double2 *)vnext, (double2 *)work, s);
     return check_launch(who);
 }
 
@@ -416,14 +419,21 @@ extern "C" size_t m25x_cgs2_work_bytes(void) { return m25x_cgs2_cols_work_bytes(
 extern "C" int m25x_cgs2(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
                          size_t work_bytes, void *stream)
 {
-    return cgs2_any("cgs2", GS_C, V, n, k, nv, w, hcol, vnext, work, work_bytes, m25x_cgs2_work_bytes(),
+    return cgs2_any("cgs2", GS_C, V, n, k, nv, w, w, hcol, vnext, work, work_bytes, m25x_cgs2_work_bytes(),
                     (hipStream_t)stream);
 }
 
 extern "C" int m25x_cgs2_cols(const double *V, long n, int k, int nv, double *w, double *hcol, double *vnext, void *work,
                               size_t work_bytes, void *stream)
 {
-    return cgs2_any("cgs2_cols", M25X_CGS2_COLS, V, n, k, nv, w, hcol, vnext, work, work_bytes,
+    return cgs2_any("cgs2_cols", M25X_CGS2_COLS, V, n, k, nv, w, w, hcol, vnext, work, work_bytes,
+                    m25x_cgs2_cols_work_bytes(k), (hipStream_t)stream);
+}
+
+extern "C" int m25x_cgs2_keep(const double *V, long n, int k, int nv, const double *w, double *hcol, double *vnext,
+                              void *work, size_t work_bytes, void *stream)
+{
+    return cgs2_any("cgs2_keep", M25X_CGS2_COLS, V, n, k, nv, w, vnext, hcol, vnext, work, work_bytes,
                     m25x_cgs2_cols_work_bytes(k), (hipStream_t)stream);
 }
 

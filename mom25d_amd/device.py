@@ -712,13 +712,16 @@ def zgemm_nk(Z, X):
 CGS2_COLS = 65536             # columns of one cgs2 call at most
 
 
-def cgs2(V, nv, W, hcol):
-    """One Arnoldi step on the device: W (n x k complex128, overwritten) orthogonalised against V[:nv] by classical
-    Gram-Schmidt applied twice; hcol[:nv + 1] (nv + 1, k) receives the coefficients and |W| (real); V[nv] = W / |W|.
-    V: (m, n, k) complex128 contiguous. Each call has its own workspace."""
+def cgs2(V, nv, W, hcol, keep=False):
+    """One Arnoldi step on the device: W (n x k complex128, overwritten unless keep) orthogonalised against V[:nv] by
+    classical Gram-Schmidt applied twice; hcol[:nv + 1] (nv + 1, k) receives the coefficients and |W| (real);
+    V[nv] = W / |W|. V: (m, n, k). All complex128, contiguous and on one device. Each call has its own workspace."""
     m, n, k = V.shape
-    if not (V.is_contiguous() and W.is_contiguous() and hcol.is_contiguous()) or W.shape != (n, k) or nv >= m:
-        raise ValueError("cgs2: V (m, n, k), W (n, k) contiguous, nv < m")
+    if any(t.dtype != c128 or not t.is_contiguous() or t.is_conj() or t.is_neg() or t.device != V.device
+           for t in (V, W, hcol)) or W.shape != (n, k) or hcol.dim() != 2 or hcol.shape[1] != k or \
+            hcol.shape[0] <= nv or nv >= m:
+        raise ValueError("cgs2: V (m, n, k), W (n, k), hcol (nv + 1, k) complex128, contiguous, on one device; nv < m")
     work = torch.empty(L.lib().m25x_cgs2_cols_work_bytes(k), dtype=torch.uint8, device=V.device)
-    L.call('m25x_cgs2_cols', ptr(V), n, k, nv, ptr(W), ptr(hcol), ptr(V[nv]), ptr(work), work.numel(), stream())
+    L.call('m25x_cgs2_keep' if keep else 'm25x_cgs2_cols', ptr(V), n, k, nv, ptr(W), ptr(hcol), ptr(V[nv]), ptr(work),
+           work.numel(), stream())
 
