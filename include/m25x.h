@@ -279,7 +279,8 @@ size_t m25x_getrs_work_bytes(int dtype, long n, long ldb);
  * pivots is kept: complex128 diagonal blocks by substitution, as LAPACK's, complex64 ones as FP64 products. Every wait between the solve's workgroups is
  * bounded: the int at work + (work_bytes - 256, rounded down to a multiple of 4), with the work_bytes passed, is
  * nonzero after a call in which one ran out (X is then not the solution), zero otherwise; it is zeroed once per
- * call, so it covers every right-hand side of the call. Replaces the backend's solve (src/mom25d/gpu.py:76-80; src/mom25d/gpu_vk.py:650-678)
+ * call, so it covers every right-hand side of the call. No wait depends on how many workgroups are resident, so solves
+ * may overlap on a device (streams, threads, processes), each with a workspace of its own. Replaces the backend's solve (src/mom25d/gpu.py:76-80; src/mom25d/gpu_vk.py:650-678)
  * and zgetrs / cgetrs (src/mom25d/fast.py:356-358). */
 int m25x_getrs(int dtype, const void *LU, long n, long lda, const int *ipiv, const int *perm, void *B, long ldb,
                int nrhs, int trans, void *work, size_t work_bytes, void *stream);

@@ -657,8 +657,15 @@ __device__ inline bool wave_all(bool c) { return __builtin_amdgcn_ballot_w64(!c)
 // take the first one's solution as their right-hand side. The chains of a call run side by side (a solve is bound by the
 // latency from block to block, not by the chip), the workgroups of one block in one XCD so that its L2 serves the
 // block's rows to all of them, and the second pass's workgroups prepare their blocks while the first pass runs.
-// Workgroup q waits only on workgroups before it, which start no later, so the launch makes progress with any number
-// of them resident.
+//
+// A workgroup waits only for blocks of its chain before its own, and it begins to wait for them only once workgroups that
+// have started answer for all of those (gate); where one stays away it does that one's block first. So as soon as any
+// workgroup of a chain runs, the chain's first unfinished block is being worked on by one that waits for nothing, and
+// every launch makes progress with any number of its workgroups resident and whatever else is on the device. The order
+// of the numbers alone does not give that: each XCD starts its own workgroups in order, but nothing holds the XCDs in
+// step, and of two solves at once on two streams (a complex64 workgroup has a CU to itself) each could fill one XCD with
+// workgroups that wait for a block the other one keeps out. (Numbers drawn from a counter at the start give it too, but
+// an XCD's workgroups start in a burst and draw neighbouring blocks: complex128 solves took 5 to 9 % longer.)
 //
 // y travels as self-marking values (put / take) in dst, chain after chain, the pair of a row side by side: a reader
 // spins on the values themselves, every lane on its own when the block is one of the two before its own (the chain
@@ -684,8 +691,7 @@ template <typename T> struct Tri {       // one chain's solve of one triangle
     int *abort;                          // raised if a wait exceeds its bound (the result is then garbage, not a hang)
 };
 
-// workgroup -> (pass, block in solve order, chain): the chains of block q are 8 apart, in q's XCD, and every block
-// before q, and the pass before, has lower numbers
+// workgroup -> (pass, block in solve order, chain): the chains of block q are 8 apart, in q's XCD
 struct ChainPos {
     int pass, q, chain;
 };
@@ -695,6 +701,82 @@ __device__ inline ChainPos chain_pos(int wg, int nb, int nchain)
     const int per = chain_wgs(nb, nchain), pass = wg / per, w = wg - pass * per, t = w / 8;
     return ChainPos{pass, t / nchain * 8 + w % 8, t % nchain};
 }
+
+// The blocks of a chain, both passes in order, a bit each: those whose workgroup has started, or that another workgroup
+// does for it, and those that a workgroup has taken to do, which only one can.
+__host__ __device__ inline int held_words(int nb) { return (2 * nb + 63) / 64; }
+struct Held {
+    u64 *started, *taken;
+};
+__device__ inline Held held_of(u64 *held, int chain, int nb)
+{
+    const int w = held_words(nb);
+    return Held{held + 2 * chain * w, held + (2 * chain + 1) * w};
+}
+__device__ inline void start_block(const Held &h, int i)
+{
+    __hip_atomic_fetch_or(h.started + (i >> 6), 1ull << (i & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline bool take_block(const Held &h, int i)
+{
+    const u64 bit = 1ull << (i & 63);
+    return !(__hip_atomic_fetch_or(h.taken + (i >> 6), bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit);
+}
+// the first block before `end` that has not started, or -1 (a whole wave calls)
+__device__ inline int first_missing(const Held &h, int end)
+{
+    for (int b0 = 0; b0 * 64 < end; b0 += 64) {
+        const int b = b0 + (threadIdx.x & 63), left = end - b * 64;
+        const u64 need = left <= 0 ? 0 : left >= 64 ? ~0ull : (1ull << left) - 1;
+        u64 miss = 0;
+        if (need) miss = need & ~__hip_atomic_load(h.started + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const u64 any = __builtin_amdgcn_ballot_w64(miss != 0);
+        if (any) {
+            const int l = __builtin_ctzll(any);
+            const u64 m = (u64)(unsigned)__builtin_amdgcn_readlane((int)(miss >> 32), l) << 32 |
+                          (unsigned)__builtin_amdgcn_readlane((int)miss, l);
+            return (b0 + l) * 64 + __builtin_ctzll(m);
+        }
+    }
+    return -1;
+}
+// The block that the workgroup with block `own` goes on with: its own once all before it have started, the first missing
+// one where it has waited for that long enough, -1 where another workgroup has taken its own. All threads call. The
+// workgroups of an empty chip start within a third of a us of each other and ask when their blocks are prepared; later
+// ones start as an XCD's slots come free, up to 40 us apart (8 blocks of 3.3 us and more). The patience is ten times
+// that: a block that another workgroup does delays the chain.
+constexpr int GATE_POLLS = 400;          // about a us each
+__device__ __forceinline__ int gate(const Held &h, int own)
+{
+    __shared__ int next;
+    if (threadIdx.x < 64) {
+        int got = 0, i = first_missing(h, own);
+        for (int polls = 0; i >= 0; ++polls) {
+            if (polls >= GATE_POLLS) {
+                if (threadIdx.x == 0 && (got = take_block(h, i))) start_block(h, i);
+                if (__builtin_amdgcn_readfirstlane(got)) break;
+            }
+            __builtin_amdgcn_s_sleep(8);
+            i = first_missing(h, own);
+        }
+        if (threadIdx.x == 0) next = i >= 0 ? i : take_block(h, own) ? own : -1;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(next);
+}
+
+// A workgroup's turn at block i of its chain (both passes in order; `own` is its own)
+struct Turn {
+    Held h;
+    int own, i, next;
+    // Once before the first wait for another block: whether to go on with block i. (A block taken to be done for another
+    // workgroup has none missing before it.)
+    __device__ __forceinline__ bool go()
+    {
+        next = i == own ? gate(h, own) : i;
+        return next == i;
+    }
+};
 
 template <typename T> __device__ inline void to_out(const Tri<T> &c, long gi, long go, int r, T v)
 {
@@ -1091,7 +1173,7 @@ template <int N> __device__ __forceinline__ void row_msub4(double *wr, double *w
 #undef M25X_MSUB
 }
 template <bool RM>
-__device__ __forceinline__ void chain_of(const Tri<float2> &c, int q)
+__device__ __forceinline__ void chain_of(const Tri<float2> &c, int q, Turn &turn)
 {
     __shared__ __align__(16) unsigned char lds[C64_LDS];
     double2(*S)[S_LD] = (double2(*)[S_LD])lds;               // the triangle, then its inverse (solve order, lower)
@@ -1099,9 +1181,10 @@ __device__ __forceinline__ void chain_of(const Tri<float2> &c, int q)
     double2 *rd = (double2 *)(N + SB);
     const long n = c.n;
     const int nb = (int)((n + SB - 1) / SB);
-    if (q >= nb) return;
     const bool fwd = c.fwd, unit = c.unit;
-    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));            // (places worked out for each block: kept from block to block they are spilled)
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     auto order = [&](int p) { return fwd ? p : nb - 1 - p; };
     auto flip = [&](int i) { return fwd ? i : SB - 1 - i; };               // local row <-> its place in solve order
     const long r0 = (long)order(q) * SB;
@@ -1166,8 +1249,10 @@ __device__ __forceinline__ void chain_of(const Tri<float2> &c, int q)
         }
     }
     float2 bx[2];                            // waves 4-7: the right-hand sides of places pair_col(h, lane)
-    if (!last)
-        rhs_pair(c, r0 + std::min(flip(pair_col(0, lane)), m - 1), r0 + std::min(flip(pair_col(1, lane)), m - 1), lane & 1, bx);
+    const long b0 = r0 + std::min(flip(pair_col(0, lane)), m - 1), b1 = r0 + std::min(flip(pair_col(1, lane)), m - 1);
+    if (!last && !c.wait) rhs_pair(c, b0, b1, lane & 1, bx);
+    if (!turn.go()) return;
+    if (!last && c.wait) rhs_pair(c, b0, b1, lane & 1, bx);
     __syncthreads();
     float4(*red)[SB] = (float4(*)[SB])lds;                                 // [wave][place]: partial sums of the pair
     u64(*zs)[64] = (u64(*)[64])(red + NWV);                                // z, as rows_sum leaves it; set when written
@@ -1260,7 +1345,7 @@ __device__ __attribute__((always_inline)) void subst(double2 &t, const double2 (
 // took 0.25 us more of a block's step than those of 2. N = 3001, 7 right-hand sides: 650 -> 333 us, 3.3 us
 // a block, of which the substitution is 1.8.
 template <bool RM>
-__device__ __forceinline__ void chain_of(const Tri<double2> &c, int q)
+__device__ __forceinline__ void chain_of(const Tri<double2> &c, int q, Turn &turn)
 {
     typedef double2 T;
     __shared__ T Ms[SB][SB + 1];             // the diagonal block's operator
@@ -1272,9 +1357,10 @@ __device__ __forceinline__ void chain_of(const Tri<double2> &c, int q)
     const T *LU = c.LU;
     const long n = c.n, lda = c.lda;
     const int nb = (int)((n + SB - 1) / SB);
-    if (q >= nb) return;
     const bool fwd = c.fwd, unit = c.unit;
-    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));            // (places worked out for each block: kept from block to block they are spilled)
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const T zero = make_double2(0, 0), one = make_double2(1, 0);
     auto order = [&](int p) { return fwd ? p : nb - 1 - p; };
     auto opp = [&](long gi, long gk) { return RM ? LU + gi * lda + gk : LU + gk * lda + gi; };
@@ -1302,6 +1388,7 @@ __device__ __forceinline__ void chain_of(const Tri<double2> &c, int q)
         const bool in = i < m && k < m && (fwd ? k < i : k > i);
         Ms[i][k] = csel(in, csel(unit, md[u], tmul(md[u], rds[i])), zero);
     }
+    if (!turn.go()) return;
     if (wv == 0) {
         T b[CR];
         rhs_row(c, grow, b);
@@ -1333,44 +1420,92 @@ __device__ __forceinline__ void chain_of(const Tri<double2> &c, int q)
     if (inrow && c.out && wv < c.kc) c.out[(c.operm ? (long)c.operm[grow] : grow) * c.ldo + wv] = y;
 }
 
-// the chain's part of one call: pass 0 reads B, pass 1 the solution of pass 0 and also writes B (every workgroup that
-// reads a row of B has done so before the second pass has a solution for it: that needs the first pass's last block)
-template <typename T>
-__device__ __forceinline__ Tri<T> chain_args(const T *LU, long lda, long n, T *B, long ldb, const int *perm, T *W1, T *W2,
-                                             int nrhs, int trans, const ChainPos &at, int *abort)
+template <typename T> struct Solve {     // a call's arguments and a workgroup's place in it
+    const T *LU;
+    long lda, n;
+    T *B;
+    long ldb;
+    const int *perm;
+    T *W1, *W2;
+    int *abort;
+    Held h;
+    int nrhs, chain, own, pad;
+};
+// block i (both passes in order) of the chain: pass 0 reads B, pass 1 the solution of pass 0 and also writes B (every
+// workgroup that reads a row of B has done so before the second pass has a solution for it: that needs the first pass's
+// last block)
+template <typename T> __device__ __forceinline__ Tri<T> chain_args(const Solve<T> &v, int pass, int trans)
 {
     Tri<T> c;
-    const int pass = at.pass;
-    T *Bc = B + at.chain * CR;
-    c.LU = LU; c.lda = lda; c.n = n;
-    c.kc = std::min(CR, nrhs - at.chain * CR);
+    T *Bc = v.B + v.chain * CR;
+    c.LU = v.LU; c.lda = v.lda; c.n = v.n;
+    c.kc = std::min(CR, v.nrhs - v.chain * CR);
     c.fwd = pass == 0;                       // U^T, then L^T (row-major: RM); or L, then U
     c.unit = pass == trans;
-    c.abort = abort;
+    c.abort = v.abort;
     c.wait = pass;
-    c.src = pass ? W1 + at.chain * CR * n : Bc;
-    c.lds = ldb;
-    c.sperm = pass || trans ? nullptr : perm;
-    c.dst = (pass ? W2 : W1) + at.chain * CR * n;
+    c.src = pass ? v.W1 + v.chain * CR * v.n : Bc;
+    c.lds = v.ldb;
+    c.sperm = pass || trans ? nullptr : v.perm;
+    c.dst = (pass ? v.W2 : v.W1) + v.chain * CR * v.n;
     c.out = pass ? Bc : nullptr;
-    c.ldo = ldb;
-    c.operm = pass && trans ? perm : nullptr;
+    c.ldo = v.ldb;
+    c.operm = pass && trans ? v.perm : nullptr;
     return c;
 }
 
-// RM: the operator's rows are contiguous (trans = 1: U^T then L^T in the factor's row-major buffer)
-template <typename T, bool RM>
-__global__ __launch_bounds__(TB) void k_trsv(const T *LU, long lda, long n, T *B, long ldb, const int *perm, T *W1, T *W2,
-                                             int nrhs, int *abort)
+// p, which came through LDS, known to the compiler to be in global memory (else its loads become flat ones)
+template <typename P> __device__ __forceinline__ P *in_global(P *p)
 {
-    const ChainPos at = chain_pos(blockIdx.x, (int)((n + SB - 1) / SB), (nrhs + CR - 1) / CR);
-    chain_of<RM>(chain_args(LU, lda, n, B, ldb, perm, W1, W2, nrhs, (int)RM, at, abort), at.q);
+    return (P *)(__attribute__((address_space(1))) P *)(u64)p;
 }
 
-// UNSET words to the first n words of each of gridDim.y buffers
-__global__ void k_fill_unset(u64 *p, long pitch, long n)
+// RM: the operator's rows are contiguous (trans = 1: U^T then L^T in the factor's row-major buffer). The workgroup's own
+// block, where another one stays away that one's first. The arguments come back from LDS before a further block: held in
+// scalar registers over a block they are spilled (20 of them, and a complex64 solve takes 2 to 4 % longer).
+template <typename T, bool RM>
+__device__ __forceinline__ void trsv_body(Solve<T> v, const ChainPos &at, u64 *held)
+{
+    __shared__ Solve<T> kept;
+    const int nb = (int)((v.n + SB - 1) / SB);
+    if (at.q >= nb) return;
+    v.chain = at.chain;
+    v.own = at.pass * nb + at.q;
+    v.h = held_of(held, at.chain, nb);
+    if (threadIdx.x == 0) {
+        start_block(v.h, v.own);
+        kept = v;
+    }
+    for (int i = v.own;;) {
+        const int nbv = (int)((v.n + SB - 1) / SB), pass = i >= nbv;
+        Turn turn{v.h, v.own, i, i};
+        chain_of<RM>(chain_args(v, pass, (int)RM), i - pass * nbv, turn);
+        if (turn.next < 0 || (turn.next == i && i == turn.own)) return;
+        __builtin_amdgcn_s_setprio(0);
+        __syncthreads();                     // every wave is done with the block's LDS
+        constexpr int NW = sizeof(Solve<T>) / 4;
+        int w[NW];
+#pragma unroll
+        for (int u = 0; u < NW; ++u) w[u] = __builtin_amdgcn_readfirstlane(((const int *)&kept)[u]);
+        __builtin_memcpy(&v, w, sizeof v);
+        v.LU = in_global(v.LU); v.B = in_global(v.B); v.perm = in_global(v.perm); v.W1 = in_global(v.W1);
+        v.W2 = in_global(v.W2); v.abort = in_global(v.abort);
+        v.h = Held{in_global(v.h.started), in_global(v.h.taken)};
+        i = turn.next == i ? v.own : turn.next;
+    }
+}
+
+template <typename T, bool RM>
+__global__ __launch_bounds__(TB) void k_trsv(Solve<T> v, u64 *held)
+{
+    trsv_body<T, RM>(v, chain_pos(blockIdx.x, (int)((v.n + SB - 1) / SB), (v.nrhs + CR - 1) / CR), held);
+}
+
+// UNSET words to the first n words of each of gridDim.y buffers; the nheld words of the chains' blocks 0
+__global__ void k_fill_unset(u64 *p, long pitch, long n, u64 *held, int nheld)
 {
     const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i < nheld && blockIdx.y == 0) held[i] = 0;
     if (i < n) p[blockIdx.y * pitch + i] = UNSET;
 }
 
@@ -1615,23 +1750,24 @@ int getrf_tp(T *A, long n, long lda, int *ipiv, int *perm, int *info, void *work
     return M25X_OK;
 }
 
-// Solve workspace: y of the two solves (W1, W2: n x MAXRHS each), written as self-marking values over UNSET words;
-// a third such buffer and n values that the solves no longer use (the size is part of the interface); the
-// permutation, the abort word (at the passed work_bytes - 256, rounded down to an int: callers read it there) and 63
-// spare ints.
+// Solve workspace: y of the two solves (W1, W2: n x MAXRHS each), written as self-marking values over UNSET words; the
+// words of the chains' blocks, in room for a third such buffer and n values (with that room the size is what it has been:
+// the largest n that m25x_getrs_noalloc takes follows from it); the permutation, the abort word (at the passed
+// work_bytes - 256, rounded down to an int: callers read it there) and 63 spare ints.
 template <typename T> size_t getrs_work(long n, long)
 {
     return sizeof(T) * (3 * (size_t)n * MAXRHS + (size_t)n) + sizeof(int) * ((size_t)n + 64);
 }
 template <typename T> struct RsWork {
     T *W1, *W2;
+    u64 *held;
     int *perm;
 };
 template <typename T> __host__ __device__ inline RsWork<T> rs_carve(void *work, long n)
 {
     const size_t wn = (size_t)n * MAXRHS;
     T *w = (T *)work;
-    return RsWork<T>{w, w + wn, (int *)(w + 3 * wn + n)};
+    return RsWork<T>{w, w + wn, (u64 *)(w + 2 * wn), (int *)(w + 3 * wn + n)};
 }
 
 // The solve with the buffers at buf (getrs_work(n) - 256 bytes) and the abort word given (not reset here).
@@ -1648,14 +1784,13 @@ int getrs_noreset(const T *LU, long n, long lda, const int *ipiv, const int *per
     }
     const long words = (long)(nchain * CR * sizeof(T) / 8) * n;
     hipLaunchKernelGGL(k_fill_unset, dim3(blocks(words, 256), 2), dim3(256), 0, s, (u64 *)w.W1,
-                       (long)((w.W2 - w.W1) * sizeof(T) / 8), words);
+                       (long)((w.W2 - w.W1) * sizeof(T) / 8), words, w.held, 2 * nchain * held_words(nb));
     if (int rc = check_launch("getrs")) return rc;
     TimedLaunch tl(s, M25X_K_TRSV, dtype_of<T>(), ((double)n * n + 4.0 * n * nrhs) * sizeof(T), 8.0 * n * n * nrhs);
     const dim3 grid(2 * chain_wgs(nb, nchain));
-    if (trans)
-        hipLaunchKernelGGL((k_trsv<T, true>), grid, dim3(TB), 0, s, LU, lda, n, B, ldb, perm, w.W1, w.W2, nrhs, abort);
-    else
-        hipLaunchKernelGGL((k_trsv<T, false>), grid, dim3(TB), 0, s, LU, lda, n, B, ldb, perm, w.W1, w.W2, nrhs, abort);
+    const Solve<T> v{LU, lda, n, B, ldb, perm, w.W1, w.W2, abort, {}, nrhs};
+    if (trans) hipLaunchKernelGGL((k_trsv<T, true>), grid, dim3(TB), 0, s, v, w.held);
+    else hipLaunchKernelGGL((k_trsv<T, false>), grid, dim3(TB), 0, s, v, w.held);
     return check_launch("getrs/trsv");
 }
 
@@ -1794,7 +1929,7 @@ int getrf_batched_t(int nitems, const m25x_lu_item *h, const m25x_lu_item *d, hi
     return M25X_OK;
 }
 
-// W1, W2 of every item filled with UNSET words
+// W1, W2 of every item filled with UNSET words, the words of its chains' blocks 0
 template <typename T>
 __global__ void k_rs_prep_b(const m25x_rs_item *items)
 {
@@ -1803,11 +1938,11 @@ __global__ void k_rs_prep_b(const m25x_rs_item *items)
     const long words = (long)((it.nrhs + CR - 1) / CR * CR * sizeof(T) / 8) * it.n;
     const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (i < words) ((u64 *)w.W1)[i] = ((u64 *)w.W2)[i] = UNSET;
+    if (i < 2 * ((it.nrhs + CR - 1) / CR) * held_words((int)((it.n + SB - 1) / SB))) w.held[i] = 0;
 }
 
-// Both triangles of every item: workgroup g is workgroup g / nitems of item g % nitems (the chains side by side; a
-// workgroup waits only on workgroups of its own item before it, which have smaller g). nb, nchain: the most blocks and
-// chains of an item.
+// Both triangles of every item: workgroup g is workgroup g / nitems of item g % nitems (the chains side by side). nb,
+// nchain: the most blocks and chains of an item.
 template <typename T, bool RM>
 __global__ __launch_bounds__(TB) void k_trsv_b(const m25x_rs_item *items, int nitems, int nb, int nchain, int *abort)
 {
@@ -1815,8 +1950,8 @@ __global__ __launch_bounds__(TB) void k_trsv_b(const m25x_rs_item *items, int ni
     const ChainPos at = chain_pos(blockIdx.x / nitems, nb, nchain);
     if (at.chain * CR >= it.nrhs) return;
     const RsWork<T> w = rs_carve<T>(it.work, it.n);
-    chain_of<RM>(chain_args((const T *)it.LU, it.lda, it.n, (T *)it.B, it.ldb, it.perm, w.W1, w.W2, it.nrhs, (int)RM, at,
-                            abort), at.q);
+    trsv_body<T, RM>(Solve<T>{(const T *)it.LU, it.lda, it.n, (T *)it.B, it.ldb, it.perm, w.W1, w.W2, abort, {}, it.nrhs},
+                     at, w.held);
 }
 
 template <typename T>
