@@ -49,8 +49,8 @@ def on_dev(a, dtype):
 
 def upload(*arrays):
     """Device copies of small NumPy arrays for kernels on the current stream, in one transfer that the host does not
-    wait for (through a pinned buffer, which is not used again before the transfer is done). For data of one call:
-    what is kept and read on other streams later goes through on_dev, which waits."""
+    wait for (through a pinned buffer, which is not used again before the transfer is done). For data of one call: what
+    is kept and may be read on another stream later goes through on_dev, which waits, or is held by a Kept."""
     arrays = [np.ascontiguousarray(a) for a in arrays]
     at, n = [], 0
     for a in arrays:
@@ -66,6 +66,42 @@ def upload(*arrays):
 
 _TORCH_DTYPE = {np.dtype(a).char: b for a, b in ((np.float64, f64), (np.int32, i32), (np.complex128, c128),
                                                  (np.int64, torch.int64))}
+
+
+def _current():
+    """The current stream as (id, device, type): what torch.cuda.current_stream() wraps in 2.7 us."""
+    return torch._C._cuda_getCurrentStream(torch.cuda.current_device())
+
+
+class Kept:
+    """Device tensors queued on the current stream that later calls read, on whatever stream those run: read() before
+    each use makes the current stream wait for them where it is another one, and the allocator for that stream before
+    their memory is used again. The wait is recorded when it is needed (two events a point, recorded beforehand, took
+    1.6 % of a small lean fill and 4 % of a batch of small boards); a stream that is not torch's own may be gone by
+    then, so there it is recorded at once. A call that is being captured waits for nothing outside, and nothing waits
+    for a stream that is: a capture begins with the device idle."""
+
+    def __init__(self, *tensors):
+        self.tensors, self.on, self.event = tensors, _current(), None
+        own = self.on[0] == 0 or self.on[0] & 1                  # the default stream or one of torch's pool
+        if not own and not torch.cuda.is_current_stream_capturing():
+            self.event = torch.cuda.current_stream().record_event()
+
+    def read(self):
+        if _current() == self.on or torch.cuda.is_current_stream_capturing():
+            return
+        s = torch.cuda.current_stream()
+        if self.event is not None:
+            s.wait_event(self.event)
+        else:
+            i, d, t = self.on
+            made = torch.cuda.Stream(stream_id=i, device_index=d, device_type=t)
+            with torch.cuda.stream(made):
+                captured = torch.cuda.is_current_stream_capturing()
+            if not captured:
+                s.wait_stream(made)
+        for t in self.tensors:
+            t.record_stream(s)
 
 
 def _cx_pairs(z):
@@ -121,7 +157,14 @@ class DevTables:
         s.dr, s.d, s.dimg = self.dr.data_ptr(), self.d.data_ptr(), self.dimg.data_ptr()
         s.cA, s.cq, s.cAi, s.cqi = (x.data_ptr() for x in (self.cA, self.cq, self.cAi, self.cqi))
         s.tab, s.kind = self.tab.data_ptr(), self.kind.data_ptr()
-        self.struct = s
+        self._arg = s
+        self._kept = Kept(self.AQ, self.dr, self.d, self.dimg, self.cA, self.cq, self.cAi, self.cqi, self.tab, self.kind)
+
+    @property
+    def struct(self):
+        """The library's view of the tables, for a call on the current stream (the tables are kept from call to call)."""
+        self._kept.read()
+        return self._arg
 
     @classmethod
     def from_dict(cls, tb):
@@ -211,7 +254,7 @@ class NearPlan:
                                          right=False).to(i32).contiguous()
         self.stat = torch.zeros((n, 12), dtype=f64, device=dv) if keep_stat else None
         self.stat_ready = False
-        self.stat_kind = None
+        self.stat_kind = self.stat_made = None          # the tables' parts it holds; its Kept
 
 
 def near_moments(mesh, tabs, plan, w, stat=True):
@@ -221,12 +264,16 @@ def near_moments(mesh, tabs, plan, w, stat=True):
     qc = torch.empty(plan.n, dtype=c128, device=device())
     use = stat and plan.stat is not None
     if use and plan.stat_kind != tabs.sig:
-        plan.stat_ready, plan.stat_kind = False, tabs.sig
+        if plan.stat_made is not None:                 # calls on other streams may still read the old ones
+            plan.stat = torch.zeros_like(plan.stat)
+        plan.stat_ready, plan.stat_kind, plan.stat_made = False, tabs.sig, None
+    ready = use and plan.stat_ready
+    if ready and plan.stat_made is not None:
+        plan.stat_made.read()
     L.call('m25x_near_moments', C.byref(mesh.struct), C.byref(tabs.struct), C.byref(mesh.quad), ptr(plan.P),
-           ptr(plan.Q), plan.n, float(w), ptr(plan.stat) if use else None, int(use and plan.stat_ready), ptr(M),
-           ptr(qc), stream())
-    if use:
-        plan.stat_ready = True
+           ptr(plan.Q), plan.n, float(w), ptr(plan.stat) if use else None, int(ready), ptr(M), ptr(qc), stream())
+    if use and not ready and not torch.cuda.is_current_stream_capturing():      # (a captured call has filled nothing yet)
+        plan.stat_made, plan.stat_ready = Kept(plan.stat), True
     return M, qc
 
 

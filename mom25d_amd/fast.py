@@ -122,6 +122,7 @@ class FastOperator:
             dv.near_scatter(Z, self.mesh, self.plan, st['M'], w)
         self._op = dict(f=st['f'], w=w, vals=dv.near_values(self.mesh, self.plan, st['M'], w) if dtype == dv.c64 else None,
                         B=st['B'], C=st['C'], lumped=st['lumped'], M=st['M'])
+        self._keep_op()
         if Nv:
             B, C = st['B'], st['C']
             Z[:Ne, Ne:] = B
@@ -131,6 +132,10 @@ class FastOperator:
             r, c, v = st['lumped']
             Z.index_put_((r, c), v.to(dtype), accumulate=True)
         return Z
+
+    def _keep_op(self):
+        op = self._op
+        op['kept'] = dv.Kept(*(t for t in (op['vals'], op['B'], op['C'], op['M'], *(op['lumped'] or ())) if t is not None))
 
     def fill(self, f, dtype=dv.c128):
         """Z (device, N x N, not equilibrated) at f: prepare(f) then assemble (see both)."""
@@ -143,8 +148,10 @@ class FastOperator:
         op, Ne = self._op, self.sim.Ne
         one = X.dim() == 1
         X = X.reshape(X.shape[0], -1).to(dv.c128).contiguous()
-        if op.get('vals') is None:
+        op['kept'].read()
+        if op['vals'] is None:
             op['vals'] = dv.near_values(self.mesh, self.plan, op['M'], op['w'])
+            self._keep_op()
         Y = torch.empty_like(X)
         dv.matvec_far(X[:Ne], self.mesh, self.tabs, op['w'], out=Y[:Ne])
         dv.csr_matvec(self.plan, op['vals'], X[:Ne], Y[:Ne])
