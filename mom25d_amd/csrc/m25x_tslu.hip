@@ -1,5 +1,6 @@
 // m25x_tslu.hip - the tournament of a tournament-pivoting LU panel (k_tslu), built once per element type
 // (M25X_TSLU_C64 set: complex64, else complex128) so the two unrolled instantiations compile in parallel.
+#include <cstddef>
 #include "m25x_lu_dev.h"
 
 namespace m25x {
@@ -30,9 +31,16 @@ template <typename T> struct GeppLds {
     T prow[SPW][SPW];                     // its pivot rows of L \ U within it
     T rcp[SPW];                           // the reciprocals of its pivots
     int4 key[2][PWV];                     // the panel waves' best: magnitude words, position (two steps, alternating)
-    T spare[PWV][SPW + 1];                // where the rows that are not the best write
+    T spare[PWV][SPW + 16 / sizeof(T)];   // where the rows that are not the best write: a key, or a row and its reciprocal
     int step_of[Tour<T>::RL];             // a pivot row's step, -1 before
 };
+// a key goes to the start of a spare row as one int4, whose place the compiler takes to be a multiple of 16 bytes
+template <typename T> constexpr bool spare_aligned()
+{
+    return alignof(GeppLds<T>) >= sizeof(int4) && offsetof(GeppLds<T>, spare) % sizeof(int4) == 0 &&
+           sizeof(GeppLds<T>::spare[0]) % sizeof(int4) == 0;
+}
+static_assert(spare_aligned<float2>() && spare_aligned<double2>(), "a spare row starts at 16 bytes");
 
 // LDS traffic done, then the barrier: stores to global memory stay in flight across it
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
