@@ -644,10 +644,12 @@ class BatchSolve:
         self.factors, self.cols = factors, cols
         self.dtype = factors[0].dtype
         self.code = L.C128 if self.dtype == c128 else L.C64
-        dv = device()
-        self.work = [torch.empty(L.lib().m25x_getrs_work_bytes(self.code, F.n, 8), dtype=torch.uint8, device=dv)
-                     for F in factors]
-        self.status = torch.zeros(1, dtype=i32, device=dv)
+        # a workspace for each eight columns of an item: its parts run side by side
+        self.work = [[self._part(F) for _ in range(0, max(kc, 1), 8)] for F, (_, kc) in zip(factors, cols)]
+        self.status = torch.zeros(1, dtype=i32, device=device())
+
+    def _part(self, F):
+        return torch.empty(L.lib().m25x_getrs_work_bytes(self.code, F.n, 8), dtype=torch.uint8, device=device())
 
     def __call__(self, R, trans=1, subset=None):
         """X (n_max, k) complex128 with F_i X_i = R_i for each item's column block of R (n_max, k); subset: for
@@ -656,9 +658,12 @@ class BatchSolve:
         nmax, k = R.shape
         X = cast_rows(R, self.dtype)                            # solved in place: never the caller's R
         items = []
-        for F, w, (c0, kc) in zip(self.factors, self.work, cols):
+        for F, parts, (c0, kc) in zip(self.factors, self.work, cols):
             for p in range(0, kc, 8):
                 q = min(8, kc - p)
+                if p // 8 == len(parts):
+                    parts.append(self._part(F))
+                w = parts[p // 8]
                 items.append(L.RsItem(F.LU.data_ptr(), F.n, F.LU.stride(0), F.perm.data_ptr(),
                                       X.data_ptr() + (c0 + p) * X.element_size(), k, q, 0, w.data_ptr(),
                                       w.numel()))
