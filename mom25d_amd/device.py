@@ -51,6 +51,9 @@ def upload(*arrays):
     """Device copies of small NumPy arrays for kernels on the current stream, in one transfer that the host does not
     wait for (through a pinned buffer, which is not used again before the transfer is done). For data of one call: what
     is kept and may be read on another stream later goes through on_dev, which waits, or is held by a Kept."""
+    if torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("mom25d_amd: a call that uploads data of its own cannot be captured (a replay would copy what "
+                           "its host buffer holds by then)")
     arrays = [np.ascontiguousarray(a) for a in arrays]
     at, n = [], 0
     for a in arrays:
