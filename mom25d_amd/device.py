@@ -38,6 +38,12 @@ def ptr(t):
     return C.c_void_p(t.data_ptr()) if t is not None else None
 
 
+def plain(X):
+    """The complex128 values of X as the kernels read them through a pointer: contiguous, and conjugated where torch has
+    put that off. X itself where it is so."""
+    return X.to(c128).resolve_conj().resolve_neg().contiguous()
+
+
 def on_dev(a, dtype):
     """A contiguous device tensor of dtype from a NumPy array (or tensor)."""
     if isinstance(a, torch.Tensor):
@@ -301,7 +307,7 @@ def csr_matvec(plan, vals, X, Y=None):
     """Y (+)= dZ X with dZ the near correction (plan's rows and columns, vals from near_values); X (Ne, k) or
     (Ne,). Adds into Y when given."""
     one = X.dim() == 1
-    X = X.reshape(X.shape[0], -1).to(c128).contiguous()
+    X = plain(X.reshape(X.shape[0], -1))
     n, k = X.shape[0], X.shape[1]
     if n < len(plan.rowptr) - 1:
         raise ValueError("csr_matvec: X has fewer rows than the edge block")
@@ -318,7 +324,7 @@ def matvec_far(X, mesh, tabs, w, out=None):
     """Y = Z_far X (device complex128 (Ne,) or (Ne, k)) without forming Z; columns 8 at a time. out: a contiguous
     (Ne, k) complex128 tensor to write (a new one when None)."""
     one = X.dim() == 1
-    X = X.reshape(X.shape[0], -1).to(c128).contiguous()
+    X = plain(X.reshape(X.shape[0], -1))
     if X.shape[0] != mesh.Ne:
         raise ValueError("matvec_far: X must have Ne rows")
     k = X.shape[1]
@@ -341,7 +347,7 @@ def via_matvec(B, Cv, X, Y):
     if X.shape != Y.shape or X.shape[0] != ne + nv or Cv.shape != (nv, nv) or not (
             X.is_contiguous() and Y.is_contiguous() and X.dtype == Y.dtype == B.dtype == Cv.dtype == c128):
         raise ValueError("via_matvec: X, Y contiguous complex128 (Ne + Nv, k), B (Ne, Nv), C (Nv, Nv) complex128")
-    B, Cv, k = B.contiguous(), Cv.contiguous(), X.shape[1]
+    B, Cv, X, k = plain(B), plain(Cv), plain(X), X.shape[1]
     wb = L.lib().m25x_via_matvec_work_bytes(nv, k)
     work = torch.empty(wb, dtype=torch.uint8, device=X.device)
     L.call('m25x_via_matvec', ptr(B), ptr(Cv), ne, nv, ptr(X), k, k, ptr(Y), k, ptr(work), wb, stream())
@@ -681,7 +687,7 @@ class BatchSolve:
 def zgemm_nk_batched(Zs, V, cols, out=None):
     """Y with Y_i = Z_i V_i for each item's column block (first column, columns) of V (n_max, k) complex128: one
     launch for all items (rows past an item's n are zero in Y)."""
-    V = V.to(c128).contiguous()
+    V = plain(V)
     Y = torch.zeros_like(V) if out is None else out
     items = []
     for Z, (c0, kc) in zip(Zs, cols):
@@ -757,7 +763,7 @@ def zgemm_nk(Z, X):
     Y = torch.empty((n, k), dtype=c128, device=X.device)
     for c0 in range(0, k, 8):
         kc = min(8, k - c0)
-        Xc = X[:, c0:c0 + kc].contiguous()
+        Xc = plain(X[:, c0:c0 + kc])
         Yc = torch.empty((n, kc), dtype=c128, device=X.device)
         L.call('m25x_zgemm_nk', ptr(Z), n, Z.stride(0), ptr(Xc), kc, ptr(Yc), stream())
         Y[:, c0:c0 + kc] = Yc

@@ -147,7 +147,7 @@ class FastOperator:
         and columns and the lumped elements. X: device (N,) or (N, k)."""
         op, Ne = self._op, self.sim.Ne
         one = X.dim() == 1
-        X = X.reshape(X.shape[0], -1).to(dv.c128).contiguous()
+        X = dv.plain(X.reshape(X.shape[0], -1))
         op['kept'].read()
         if op['vals'] is None:
             op['vals'] = dv.near_values(self.mesh, self.plan, op['M'], op['w'])

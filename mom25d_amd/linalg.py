@@ -34,12 +34,6 @@ def _cnorm(X):
     return torch.linalg.vector_norm(X, dim=0).cpu().numpy()
 
 
-def _values(W):
-    """An operator's result as the fused step reads it (which leaves it as it is: it may be the operator's argument, or
-    kept by its owner): complex128, contiguous, conjugated where that was put off. The same tensor where it is so."""
-    return W.to(torch.complex128).resolve_conj().resolve_neg().contiguous()
-
-
 def gmres_batched(A, B, M=None, x0=None, rtol=1e-6, restart=30, maxiter=10, stall=None, track=None,
                   stall_each=False, guess=False):
     """(X, iterations per column) for A X = B; A, M: callables on device (N x k) complex128 tensors; B device.
@@ -102,7 +96,7 @@ def gmres_batched(A, B, M=None, x0=None, rtol=1e-6, restart=30, maxiter=10, stal
 
             def enqueue(i):
                 Zs[i] = M(V[i])
-                dv.cgs2(V, i + 1, _values(A(Zs[i])), hbuf, keep=True)
+                dv.cgs2(V, i + 1, dv.plain(A(Zs[i])), hbuf, keep=True)
                 pin[i % 2][:i + 2].copy_(hbuf[:i + 2], non_blocking=True)
                 evs[i % 2].record()
         for j in range(restart):
@@ -120,7 +114,8 @@ def gmres_batched(A, B, M=None, x0=None, rtol=1e-6, restart=30, maxiter=10, stal
                 hc = pin[j % 2][:j + 2].numpy().copy()
             else:
                 Zs[j] = M(V[j])
-                Wv = _values(A(Zs[j]))
+                # (kept as it is: it may be the operator's argument, or its owner's)
+                Wv = dv.plain(A(Zs[j]))
                 if restart < 64 and ka <= dv.CGS2_COLS:
                     dv.cgs2(V, j + 1, Wv, hbuf, keep=True)
                     hc = hbuf[:j + 2].cpu().numpy()
