@@ -1668,6 +1668,25 @@ private:
     int index = 0;
 };
 
+// What a call has on its side stream: the caller's stream waits for it before the matrix is read again, and where the call
+// ends early (a launch that fails), so that the matrix' memory is free to its owner in the caller's stream's order.
+struct Beside {
+    hipStream_t s;
+    const Side *side;
+    bool open = false;
+    int join()
+    {
+        if (open && hipStreamWaitEvent(s, side->done, 0) != hipSuccess) return fail(M25X_EHIP, "getrf: wait");
+        open = false;
+        return M25X_OK;
+    }
+    ~Beside()
+    {
+        if (open && (hipEventRecord(side->done, side->s) != hipSuccess || hipStreamWaitEvent(s, side->done, 0) != hipSuccess))
+            (void)hipStreamSynchronize(side->s);
+    }
+};
+
 // From this many trailing rows on a step's update is split: below it the update is hardly longer than what the split
 // costs (the extra launch and two events, about 25 us; at 2500 rows 7.48 ms without and 7.38 with it).
 constexpr long LOOK_ROWS = 2048;
@@ -1719,10 +1738,10 @@ int getrf_tp(T *A, long n, long lda, int *ipiv, int *perm, int *info, void *work
                          lda, M, N, (long)jb);
     };
     if (int rc = tournament(0)) return rc;
-    bool beside = false;                     // the last update's rest runs on the side stream
+    Beside beside{s, side};                  // the last update's rest, where it runs on the side stream
     for (long j0 = 0; j0 < n; j0 += TW) {
         const int jb = (int)std::min((long)TW, n - j0);
-        if (beside && hipStreamWaitEvent(s, side->done, 0) != hipSuccess) return fail(M25X_EHIP, "getrf: wait");
+        if (int rc = beside.join()) return rc;
         {
             TimedLaunch tl(s, M25X_K_APPLY_MOVES, dt, 2.0 * es * 2 * jb * n, 0.0);
             hipLaunchKernelGGL(k_apply_moves<T>, dim3(blocks(n, 8) + (perm ? 1 : 0)), dim3(256), 0, s, A, lda, 0L, n,
@@ -1732,13 +1751,13 @@ int getrf_tp(T *A, long n, long lda, int *ipiv, int *perm, int *info, void *work
         const long c0 = j0 + jb;
         if (c0 >= n) break;
         launch_tri(s, A, lda, j0, n - c0, (const T *)top);   // L21 = A21 U11^-1 and U12 = L11^-1 A12
-        beside = side && n - c0 >= LOOK_ROWS;
-        if (beside) {
+        if (side && n - c0 >= LOOK_ROWS) {
             const long c1 = c0 + TW;
             update(s, j0, jb, c0, c1);                       // the next panel's columns
             if (hipEventRecord(side->next, s) != hipSuccess || hipStreamWaitEvent(side->s, side->next, 0) != hipSuccess)
                 return fail(M25X_EHIP, "getrf: look-ahead");
             if (int rc = tournament(c0)) return rc;          // in place before the rest is let go
+            beside.open = true;
             update(side->s, j0, jb, c1, n);
             if (hipEventRecord(side->done, side->s) != hipSuccess) return fail(M25X_EHIP, "getrf: look-ahead");
         } else {
