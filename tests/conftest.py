@@ -21,3 +21,10 @@ def gpu():
     from mom25d_amd import device as dv
     dv.device()
     return dv
+
+
+def pytest_collection_modifyitems(items):
+    """The serving loop's tests first. One asserts that a tight budget gives more batches than a free one, where requests
+    arrive 5 ms apart: that holds while the process's first calls are slow, so that the free server's first batch leaves
+    the rest to gather. Tests that warm the same calls before it, whatever their files are called, would undo it."""
+    items.sort(key=lambda it: it.path.name != 'test_gpu_serve.py')
