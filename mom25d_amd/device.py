@@ -85,30 +85,29 @@ def _current():
 class Kept:
     """Device tensors queued on the current stream that later calls read, on whatever stream those run: read() before
     each use makes the current stream wait for them where it is another one, and the allocator for that stream before
-    their memory is used again. The wait is recorded when it is needed (two events a point, recorded beforehand, took
-    1.6 % of a small lean fill and 4 % of a batch of small boards); a stream that is not torch's own may be gone by
-    then, so there it is recorded at once. A call that is being captured waits for nothing outside, and nothing waits
-    for a stream that is: a capture begins with the device idle."""
+    their memory is used again. The event to wait for is recorded at the first such use, and the wait is then for all
+    that the first stream has in its queue (two events a point, recorded beforehand, took 1.6 % of a small lean fill and
+    4 % of a batch of small boards); at once for what is kept for long, or where the stream is not torch's own and may be
+    gone by then. A call that is being captured waits for nothing outside, and nothing waits for a stream that is: a
+    capture begins with the device idle."""
 
-    def __init__(self, *tensors):
+    def __init__(self, *tensors, at_once=False):
         self.tensors, self.on, self.event = tensors, _current(), None
         own = self.on[0] == 0 or self.on[0] & 1                  # the default stream or one of torch's pool
-        if not own and not torch.cuda.is_current_stream_capturing():
+        if (at_once or not own) and not torch.cuda.is_current_stream_capturing():
             self.event = torch.cuda.current_stream().record_event()
 
     def read(self):
         if _current() == self.on or torch.cuda.is_current_stream_capturing():
             return
+        if self.event is None:
+            i, d, t = self.on
+            with torch.cuda.stream(torch.cuda.Stream(stream_id=i, device_index=d, device_type=t)):
+                if not torch.cuda.is_current_stream_capturing():
+                    self.event = torch.cuda.current_stream().record_event()
         s = torch.cuda.current_stream()
         if self.event is not None:
             s.wait_event(self.event)
-        else:
-            i, d, t = self.on
-            made = torch.cuda.Stream(stream_id=i, device_index=d, device_type=t)
-            with torch.cuda.stream(made):
-                captured = torch.cuda.is_current_stream_capturing()
-            if not captured:
-                s.wait_stream(made)
         for t in self.tensors:
             t.record_stream(s)
 
@@ -282,7 +281,7 @@ def near_moments(mesh, tabs, plan, w, stat=True):
     L.call('m25x_near_moments', C.byref(mesh.struct), C.byref(tabs.struct), C.byref(mesh.quad), ptr(plan.P),
            ptr(plan.Q), plan.n, float(w), ptr(plan.stat) if use else None, int(ready), ptr(M), ptr(qc), stream())
     if use and not ready and not torch.cuda.is_current_stream_capturing():      # (a captured call has filled nothing yet)
-        plan.stat_made, plan.stat_ready = Kept(plan.stat), True
+        plan.stat_made, plan.stat_ready = Kept(plan.stat, at_once=True), True
     return M, qc
 
 

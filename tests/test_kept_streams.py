@@ -20,16 +20,15 @@ class Stream:
     def __init__(self, stream_id):
         self.made[stream_id] = self
         self.waits, self.cuda_stream, self.stream_id, self.capturing, self.gone = [], id(self), stream_id, False, False
+        self.events = 0
 
     def record_event(self, event=None):
-        assert not self.gone
+        assert not self.gone and not self.capturing
+        self.events += 1
         return ('queued on', self)
 
     def wait_event(self, e):
         self.waits.append(e)
-
-    def wait_stream(self, s):
-        self.wait_event(s.record_event())
 
 
 @pytest.fixture
@@ -84,10 +83,13 @@ def test_tables(cuda):
     cuda.now = cuda.b
     assert t.struct.ntab == 1 and cuda.b.waits == [('queued on', cuda.a)]
     assert {(x.data_ptr(), cuda.b) for x in (t.AQ, t.dr, t.cA, t.tab)} <= set(cuda.recorded)
+    assert t.struct.ntab == 1 and cuda.a.events == 1 and len(cuda.b.waits) == 2   # what came later is not waited for
     cuda.b.capturing = True
-    assert t.struct.ntab == 1 and len(cuda.b.waits) == 1
-    cuda.b.capturing, cuda.a.capturing = False, True
-    assert t.struct.ntab == 1 and len(cuda.b.waits) == 1
+    assert t.struct.ntab == 1 and len(cuda.b.waits) == 2
+    cuda.now, cuda.b.capturing = cuda.a, False
+    t = _tables()
+    cuda.now, cuda.a.capturing = cuda.b, True
+    assert t.struct.ntab == 1 and len(cuda.b.waits) == 2 and cuda.a.events == 1
 
 
 def test_stream_of_another_library(cuda):
@@ -103,8 +105,10 @@ def test_moments(cuda):
     first = _ready(cuda)
     dv.near_moments(MESH, t, p, 1.0)
     assert first == (p.stat.data_ptr(), 0) and _ready(cuda) == (p.stat.data_ptr(), 1) and not cuda.a.waits
+    made = cuda.a.events                                                          # once a mesh: recorded at once
     cuda.now = cuda.b
     dv.near_moments(MESH, _tables(), p, 1.0)                                      # tables of its own, the moments kept
+    assert made == 1 and cuda.a.events == 1
     assert cuda.b.waits == [('queued on', cuda.a)] and (p.stat.data_ptr(), cuda.b) in cuda.recorded
     assert _ready(cuda) == (p.stat.data_ptr(), 1)
     old = p.stat                                                                  # other parts extracted: filled again,
