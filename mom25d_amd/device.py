@@ -541,9 +541,15 @@ def cast_rows(src, dtype, scale=None, out=None):
         src = src.to(c128)
     if src.stride(1) != 1 or src.stride(0) < src.shape[1]:
         src = src.contiguous()
+    n, k = src.shape
+    if scale is not None and (scale.dtype != f64 or scale.shape != (n,) or not scale.is_contiguous() or
+                              scale.device != src.device):
+        raise ValueError("cast_rows: scale must be a contiguous float64 tensor of one value a row, on src's device")
     if out is None:
         out = torch.empty(src.shape, dtype=dtype, device=src.device)
-    n, k = src.shape
+    elif out.shape != src.shape or out.dtype != dtype or out.device != src.device or (k > 1 and out.stride(1) != 1) or \
+            (n > 1 and out.stride(0) < k):
+        raise ValueError("cast_rows: out must be columns of a row-major tensor of dtype, of src's shape, on its device")
     code = lambda t: L.C128 if t.dtype == c128 else L.C64
     L.call('m25x_cast_rows', code(src), ptr(src), max(src.stride(0), k), code(out), ptr(out), max(out.stride(0), k), n, k,
            ptr(scale), stream())
@@ -778,8 +784,8 @@ def cgs2(V, nv, W, hcol, keep=False):
     V[nv] = W / |W|. V: (m, n, k). All complex128, contiguous and on one device. Each call has its own workspace."""
     m, n, k = V.shape
     if any(t.dtype != c128 or not t.is_contiguous() or t.is_conj() or t.is_neg() or t.device != V.device
-           for t in (V, W, hcol)) or W.shape != (n, k) or hcol.dim() != 2 or hcol.shape[1] != k or \
-            hcol.shape[0] <= nv or nv >= m:
+           for t in (V, W, hcol)) or W.shape != (n, k) or nv >= m or \
+            hcol.numel() < (nv + 1) * k:
         raise ValueError("cgs2: V (m, n, k), W (n, k), hcol (nv + 1, k) complex128, contiguous, on one device; nv < m")
     work = torch.empty(L.lib().m25x_cgs2_cols_work_bytes(k), dtype=torch.uint8, device=V.device)
     L.call('m25x_cgs2_keep' if keep else 'm25x_cgs2_cols', ptr(V), n, k, nv, ptr(W), ptr(hcol), ptr(V[nv]), ptr(work),
