@@ -38,10 +38,14 @@ def ptr(t):
     return C.c_void_p(t.data_ptr()) if t is not None else None
 
 
+def _as_is(X):
+    return X.dtype is c128 and X.is_contiguous() and not (X.is_conj() or X.is_neg())
+
+
 def plain(X):
     """The complex128 values of X as the kernels read them through a pointer: contiguous, and conjugated where torch has
     put that off. X itself where it is so."""
-    return X.to(c128).resolve_conj().resolve_neg().contiguous()
+    return X if _as_is(X) else X.to(c128).resolve_conj().resolve_neg().contiguous()
 
 
 def on_dev(a, dtype):
@@ -783,9 +787,8 @@ def cgs2(V, nv, W, hcol, keep=False):
     classical Gram-Schmidt applied twice; hcol[:nv + 1] (nv + 1, k) receives the coefficients and |W| (real);
     V[nv] = W / |W|. V: (m, n, k). All complex128, contiguous and on one device. Each call has its own workspace."""
     m, n, k = V.shape
-    if any(t.dtype != c128 or not t.is_contiguous() or t.is_conj() or t.is_neg() or t.device != V.device
-           for t in (V, W, hcol)) or W.shape != (n, k) or nv >= m or \
-            hcol.numel() < (nv + 1) * k:
+    if not (_as_is(V) and _as_is(W) and _as_is(hcol)) or W.shape != (n, k) or nv >= m or \
+            hcol.numel() < (nv + 1) * k or W.device != V.device or hcol.device != V.device:
         raise ValueError("cgs2: V (m, n, k), W (n, k), hcol (nv + 1, k) complex128, contiguous, on one device; nv < m")
     work = torch.empty(L.lib().m25x_cgs2_cols_work_bytes(k), dtype=torch.uint8, device=V.device)
     L.call('m25x_cgs2_keep' if keep else 'm25x_cgs2_cols', ptr(V), n, k, nv, ptr(W), ptr(hcol), ptr(V[nv]), ptr(work),
