@@ -256,9 +256,8 @@ size_t m25x_getrf_work_bytes(int dtype, long n);
 
 /* LU of the column-major n x n matrix A (leading dimension lda; the row-major Z seen as Z^T), in place: L unit
  * lower, U upper, ipiv 0-based LAPACK-style interchanges (int32, device), the layout of
- * scipy.linalg.lu_factor(Z.T). complex128: trailing updates on the FP64 matrix cores. complex64: with partial
- * pivoting on the FP32 matrix cores (FP32 accumulation); with tournament pivoting on the FP64 matrix cores (one
- * rounding to FP32 an entry). pivot: M25X_PIVOT_PARTIAL or M25X_PIVOT_TOURNAMENT. perm (device int[n], may be
+ * scipy.linalg.lu_factor(Z.T). complex128: trailing updates on the FP64 matrix cores. complex64: on the FP32 matrix
+ * cores with FP32 accumulation (tournament pivoting: or on the FP64 ones, m25x_lu_set_update_precision). pivot: M25X_PIVOT_PARTIAL or M25X_PIVOT_TOURNAMENT. perm (device int[n], may be
  * NULL): the interchanges as one permutation, m25x_ipiv_perm's. info (device int, may be NULL): 0, 1 + the first
  * zero pivot, or -1 when a bounded wait between the workgroups of a partial-pivoting panel ran out (the factor is
  * then not valid; the tournament has no such wait). Replaces the GPU backend's factor (src/mom25d/gpu.py:69-74;
@@ -358,8 +357,8 @@ typedef struct m25x_rs_item {
     size_t work_bytes;
 } m25x_rs_item;
 
-/* The solves of nitems factors (trans as m25x_getrs), each triangle one launch for all items: the chains of the
- * items' diagonal blocks side by side in one grid. status (device int): zeroed, then nonzero if a wait between
+/* The solves of nitems factors (trans as m25x_getrs), both triangles of all items in one launch: the chains of the
+ * items' diagonal blocks side by side in one grid. The items' workspaces must not overlap. status (device int): zeroed, then nonzero if a wait between
  * workgroups ran out in any item. */
 int m25x_getrs_batched(int dtype, int nitems, const m25x_rs_item *items_host, const m25x_rs_item *items_dev, int trans,
                        int *status, void *stream);

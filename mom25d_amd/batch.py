@@ -11,7 +11,7 @@ Simulation.sparams per frequency; src/mom25d/fast.py:704-850 fills and factors o
   refine    one GMRES over the ports of every point of similar size (groups within GROUP_SPREAD), side by side as
             the columns of one (n_max, k_total) block, zero-padded:
             the operator is block-diagonal - the FP64 products of all points in one launch (m25x_zgemm_nk_batched),
-            the preconditioner all points' triangular solves in one launch per triangle (m25x_getrs_batched) - and
+            the preconditioner all points' triangular solves in one launch (m25x_getrs_batched) - and
             a point whose refinement stalls stops alone
   S         per point; a point whose complex64 factor does not converge is solved again by its own board's
             single-point path (complex128 LU)

@@ -1255,7 +1255,7 @@ __device__ __forceinline__ void chain_of(const Tri<float2> &c, int q, Turn &turn
     if (!last && c.wait) rhs_pair(c, b0, b1, lane & 1, bx);
     __syncthreads();
     float4(*red)[SB] = (float4(*)[SB])lds;                                 // [wave][place]: partial sums of the pair
-    u64(*zs)[64] = (u64(*)[64])(red + NWV);                                // z, as rows_sum leaves it; set when written
+    u64(*zs)[64] = (u64(*)[64])(red + NWV);                                // z, as rows_product leaves it; set when written
     if (last) zs[wv][lane] = UNSET;
     {
         float o[2 * CR];

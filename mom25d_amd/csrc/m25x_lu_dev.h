@@ -83,7 +83,7 @@ template <typename T> __device__ inline double cabs1(T a) { return fabs((double)
 // ---- tournament pivoting (communication-avoiding LU panels) -----------------------------------------------
 // A panel's TW pivot rows are chosen by a tree of GEPPs (Grigori, Demmel and Xiang, "CALU: a communication
 // optimal LU factorization algorithm", SIAM J. Matrix Anal. Appl. 32 (2011)): each leaf workgroup factors RL rows
-// of the panel in LDS and nominates its pivot rows; a tree node factors its children's nominees (their original
+// of the panel (in registers) and nominates its pivot rows; a tree node factors its children's nominees (their original
 // rows, stacked in child order) and nominates its own; the root's pivot rows are the panel's, and the root's
 // factors of them are the panel's L11 \ U11. One launch a panel: a node is factored by whichever of its children
 // arrives last (an atomic count per node), so no workgroup ever waits on another. The rows below take
