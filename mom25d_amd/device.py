@@ -710,24 +710,29 @@ def zgemm_nk_batched(Zs, V, cols, out=None):
     return Y
 
 
-_FAULTS = {}
+_FAULTS = {}                             # (device, stream id) -> the flag of the solves on that stream
 
 
 def _solve_fault(dev):
-    f = _FAULTS.get(dev)
+    key = dev, _current()[0]
+    f = _FAULTS.get(key)
+    if f is None and torch.cuda.is_current_stream_capturing():      # a flag made in a capture is cleared by each replay
+        f = next((g for (d, _), g in list(_FAULTS.items()) if d == dev), None)
     if f is None:
-        f = _FAULTS[dev] = torch.zeros(1, dtype=torch.int32, device=dev)
+        f = _FAULTS[key] = torch.zeros(1, dtype=torch.int32, device=dev)
     return f
 
 
 def solve_faults(dev=None):
-    """Whether a getrs since the last call ran out of a wait bound between its workgroups (its result is then not
-    the solution); clears the record. Reading it synchronises with the stream."""
-    f = _FAULTS.get(torch.device(dev) if dev is not None else device())
-    if f is None:
-        return False
-    bad = bool(f.item())
-    f.zero_()
+    """Whether a getrs since the last call, on any stream, ran out of a wait bound between its workgroups (its result is
+    then not the solution); clears the record. Reading it synchronises with the current stream; what runs on others is
+    reported once it is done."""
+    dev = torch.device(dev) if dev is not None else device()
+    bad = False
+    for f in [f for (d, _), f in list(_FAULTS.items()) if d == dev]:
+        if f.item():
+            f.zero_()
+            bad = True
     return bad
 
 
